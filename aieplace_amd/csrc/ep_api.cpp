@@ -17,6 +17,7 @@
 #include "../../include/eplace_mlp.h"
 #include "ep_sched.h"
 #include "ep_ctx.h"
+#include "ep_fft.h"
 #include "ep_layout.h"
 
 namespace ep {
@@ -1466,8 +1467,11 @@ extern "C" ep_status ep_profile(ep_ctx *c, int32_t reps, ep_kernel_stat *out, in
     // forms execute three products each (1.5x, at the 16-bit rate).
     const double Mxd = c->Mx, Myd = c->My;
     const double gemm_flops = 6.0 * Mxd * Myd * (Mxd + Myd);
-    // reads 6 maps, writes 7; the halves of the six matrices: 1.5 (Mx^2 + My^2) floats
-    const double field_bytes = 4.0 * 13 * nb + 4.0 * 1.5 * (Mxd * Mxd + Myd * Myd);
+    // reads 6 maps, writes 7; the halves of the six matrices: 1.5 (Mx^2 + My^2) floats.
+    // The FFT path reads the map and writes the field; one map and one pair of
+    // maps go between its three kernels.
+    const bool fft = fft_side(c->Mx) && fft_side(c->My);
+    const double field_bytes = fft ? 36.0 * nb : 4.0 * 13 * nb + 4.0 * 1.5 * (Mxd * Mxd + Myd * Myd);
     // Instances that fork their captured evaluation sum the pin partials per cell
     // on the WA branch (k_pin_sum), and the cell gradient reads those sums: both
     // are timed that way here, as the placement runs them.
@@ -1481,7 +1485,7 @@ extern "C" ep_status ep_profile(ep_ctx *c, int32_t reps, ep_kernel_stat *out, in
         // accumulators cleared
         {"overflow", 1, 44.0 * nb, 0},
         {"wa_grad", 1, 4.0 * (N + 1) + 12.0 * P + 8.0 * c->n_all + 8.0 * P, 0},
-        {"field_transforms", 4, field_bytes, gemm_flops},
+        {"field_transforms", fft ? 3 : 4, field_bytes, fft ? 0 : gemm_flops},
     };
     if (forked) {
         // CSR offsets and pin list read, the pins' partials gathered, one sum

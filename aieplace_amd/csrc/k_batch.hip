@@ -388,8 +388,8 @@ __global__ __launch_bounds__(kBlock) void kb_cell_grad(BDev d, int at)
         const int k0 = d.cps[c], k1 = d.cps[c + 1];
         const float2 f = cell_force(p, s, exy, g, M, M);
         const float2 gw = sum_pin_partials(k0, k1, d.cpins, d.pin_grad);
-        const float pre = fmaxf(1.0f, (float)(k1 - k0) + lambda * s.x * s.y);
-        const float gx = (gw.x - lambda * f.x) / pre, gy = (gw.y - lambda * f.y) / pre;
+        const float pre = fmaxf(1.0f, __fmaf_rn(lambda * s.x, s.y, (float)(k1 - k0)));
+        const float gx = __fmaf_rn(-lambda, f.x, gw.x) / pre, gy = __fmaf_rn(-lambda, f.y, gw.y) / pre;
         gout[c] = make_float2(gx, gy);
         if (at == kAtTrial) {
             const double dx = (double)p.x - v0.x, dy = (double)p.y - v0.y;

@@ -1,4 +1,6 @@
-// k_field.hip -- Poisson field solve as dense transform-matrix products on MFMA.
+// k_field.hip -- Poisson field solve as dense transform-matrix products on MFMA,
+// for grids with a side that is not a power of two (the others: k_fft.hip), and
+// the standalone transforms.
 //
 // Reference: the separable DCT field of vck5000/host/src/AIEplace.cpp:752-934
 // (compute_a_uv_DCT / compute_eField_DCT with DCT_naive/IDCT_naive/IDXST_naive,
@@ -37,6 +39,7 @@
 
 #include "ep_batch.h"
 #include "ep_ctx.h"
+#include "ep_fft.h"
 
 namespace ep {
 
@@ -782,7 +785,8 @@ static void set_operand(GemmArgs &a, int z, const HalfMats &hm, int m, int preci
 }
 
 struct FieldMats {
-    HalfMats half[MAT_N];                  // even/odd halves, FP32 and split planes
+    float2 *fft_x, *fft_y;                 // grids that the FFT path takes: its constants (fft_y may equal fft_x)
+    HalfMats half[MAT_N];                  // the others: even/odd halves, FP32 and split planes
     double *f64[MAT_N];                    // full FP64 matrices of the reference (built on first use)
     uint32_t *fmax;                        // FP16X3 running maxima: rho, T1t, Eh, Rt
     double *tA64, *tB64, *exd, *eyd;       // FP64 reference scratch
@@ -790,6 +794,18 @@ struct FieldMats {
 };
 
 constexpr int kErrBlocks = 256;
+
+static ep_status upload_fft_table(int n, float2 *&d)
+{
+    d = nullptr;
+    std::vector<float2> tab;
+    fft_table(n, tab);
+    if (hipMalloc(&d, tab.size() * sizeof(float2)) != hipSuccess)
+        return fail(EP_ENOMEM, "field: hipMalloc of the FFT constants failed");
+    if (hipMemcpy(d, tab.data(), tab.size() * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess)
+        return fail(EP_EDEVICE, "field: upload of the FFT constants failed");
+    return EP_OK;
+}
 
 static bool matrix_desc(const Ctx &c, int m, int &M, bool &sine, bool &tr)
 {
@@ -807,7 +823,14 @@ ep_status field_init(Ctx &c)
     FieldMats *fm = new (std::nothrow) FieldMats();
     if (!fm) return fail(EP_ENOMEM, "field_init: host allocation failed");
     c.split_mats = fm;
-    for (int m = 0; m < MAT_N; ++m) {
+    const bool fft = fft_side(c.Mx) && fft_side(c.My);
+    if (fft) {
+        ep_status st = upload_fft_table(c.Mx, fm->fft_x);
+        if (st != EP_OK) return st;
+        fm->fft_y = fm->fft_x;
+        if (c.My != c.Mx && (st = upload_fft_table(c.My, fm->fft_y)) != EP_OK) return st;
+    }
+    for (int m = 0; m < MAT_N && !fft; ++m) {
         int M;
         bool sine, tr;
         matrix_desc(c, m, M, sine, tr);
@@ -831,7 +854,8 @@ void field_free(Ctx &c)
         free_halves(fm->half[m]);
         if (fm->f64[m]) (void)hipFree(fm->f64[m]);
     }
-    void *p[] = {fm->fmax, fm->tA64, fm->tB64, fm->exd, fm->eyd, fm->err_part};
+    if (fm->fft_y != fm->fft_x && fm->fft_y) (void)hipFree(fm->fft_y);
+    void *p[] = {fm->fft_x, fm->fmax, fm->tA64, fm->tB64, fm->exd, fm->eyd, fm->err_part};
     for (void *q : p)
         if (q) (void)hipFree(q);
     delete fm;
@@ -850,6 +874,12 @@ void launch_field(Ctx &c, int precision, hipStream_t s)
     a.wxs = (float)(M_PI / c.Mx);
     a.wys = (float)(M_PI / c.My * ((double)c.bw / c.bh));
     a.skip = &c.d_scal->halt;  // a finished device-controlled run skips the solve
+    if (fm->fft_x) {
+        FftArgs f{c.map_field, c.map_mean, a.skip, fm->fft_x, fm->fft_y, c.tA, reinterpret_cast<float2 *>(c.tB),
+                  c.exy, c.Mx, c.My, a.scale, a.wxs, a.wys};
+        launch_field_fft(f, s);
+        return;
+    }
     auto setA = [&](int z, int m) { set_operand(a, z, fm->half[m], m, precision); };
     if (f16) {
         launch_map_range(c, s);
@@ -976,8 +1006,25 @@ struct BatchField {
     uint32_t *fmax = nullptr;                // [4 * n_inst]
     int n_inst = 0;
     std::vector<int> M_of;                   // grid side of each instance
+    // instances on grids that the FFT path takes; the products run the others
+    std::vector<float2 *> fft_tabs;          // per distinct M (null: products)
+    FftArgs *d_fft = nullptr;                // [n_inst]
+    FftBatchTiles fft[kFftClasses] = {};
     int tile_var[3] = {1, 1, 1};             // [precision] K-step variant (kSkBatchF32/kSkBatchSplit)
 };
+
+static ep_status upload_fft_tiles(BatchField *bf, const std::vector<int2> (&tiles)[kFftClasses][3])
+{
+    for (int k = 0; k < kFftClasses; ++k)
+        for (int stage = 0; stage < 3; ++stage) {
+            const std::vector<int2> &t = tiles[k][stage];
+            bf->fft[k].n[stage] = (int)t.size();
+            if (!t.empty() &&
+                hipMemcpy(bf->fft[k].d[stage], t.data(), sizeof(int2) * t.size(), hipMemcpyHostToDevice) != hipSuccess)
+                return fail(EP_EDEVICE, "batch field: FFT tile upload failed");
+        }
+    return EP_OK;
+}
 
 ep_status batch_field_init(BatchField *&out, const std::vector<BatchFieldInst> &inst)
 {
@@ -989,11 +1036,18 @@ ep_status batch_field_init(BatchField *&out, const std::vector<BatchFieldInst> &
     for (const BatchFieldInst &d : inst)
         if (std::find(bf->sizes.begin(), bf->sizes.end(), d.M) == bf->sizes.end()) bf->sizes.push_back(d.M);
     bf->sets.resize(bf->sizes.size());
-    for (size_t si = 0; si < bf->sizes.size(); ++si)
+    bf->fft_tabs.resize(bf->sizes.size(), nullptr);
+    for (size_t si = 0; si < bf->sizes.size(); ++si) {
+        if (fft_side(bf->sizes[si])) {
+            ep_status st = upload_fft_table(bf->sizes[si], bf->fft_tabs[si]);
+            if (st != EP_OK) return st;
+            continue;
+        }
         for (int m = 0; m < MAT_N; ++m) {
             ep_status st = upload_halves(bf->sizes[si], m, bf->sets[si].half[m]);
             if (st != EP_OK) return st;
         }
+    }
     const int n = bf->n_inst;
     if (hipMalloc(&bf->fmax, sizeof(uint32_t) * 4 * std::max(1, n)) != hipSuccess ||
         hipMemset(bf->fmax, 0, sizeof(uint32_t) * 4 * std::max(1, n)) != hipSuccess)
@@ -1001,6 +1055,8 @@ ep_status batch_field_init(BatchField *&out, const std::vector<BatchFieldInst> &
     // argument blocks per precision and stage, and the tile lists
     const int precs[3] = {EP_PREC_FP32, EP_PREC_BF16X3, EP_PREC_FP16X3};
     std::vector<int4> tiles[4];
+    std::vector<FftArgs> fargs(n);
+    std::vector<int2> ftiles[kFftClasses][3];
     for (int pi = 0; pi < 3; ++pi) {
         const int prec = precs[pi];
         const bool f16 = prec == EP_PREC_FP16X3;
@@ -1017,6 +1073,11 @@ ep_status batch_field_init(BatchField *&out, const std::vector<BatchFieldInst> &
             a.wys = (float)(M_PI / d.M * ((double)d.bw / d.bh));
             a.M = a.N = a.K = d.M;
             a.skip = d.skip;
+            if (pi == 0 && bf->fft_tabs[si]) {
+                fargs[i] = FftArgs{d.map_field, d.map_mean, d.skip, bf->fft_tabs[si], bf->fft_tabs[si], d.tA,
+                                   reinterpret_cast<float2 *>(d.tB), d.exy, d.M, d.M, a.scale, a.wxs, a.wys};
+                fft_batch_tiles(i, d.M, ftiles);
+            }
             auto setA = [&](GemmArgs &g, int z, int m) { set_operand(g, z, ms.half[m], m, prec); };
             GemmArgs g1 = a;
             setA(g1, 0, MAT_CY); g1.B[0] = d.map_field; g1.C[0] = d.tA;
@@ -1037,7 +1098,7 @@ ep_status batch_field_init(BatchField *&out, const std::vector<BatchFieldInst> &
             st[1].push_back(g2);
             st[2].push_back(g3);
             st[3].push_back(g4);
-            if (pi == 0) {
+            if (pi == 0 && !bf->fft_tabs[si]) {
                 const int mt = ((d.M >> 1) + SBM - 1) / SBM, nt = (d.M + SBN - 1) / SBN;
                 for (int stage = 0; stage < 4; ++stage)
                     for (int z = 0; z < (stage >= 2 ? 2 : 1); ++z)
@@ -1059,15 +1120,28 @@ ep_status batch_field_init(BatchField *&out, const std::vector<BatchFieldInst> &
                       hipMemcpyHostToDevice) != hipSuccess)
             return fail(EP_ENOMEM, "batch field: tile upload failed");
     }
-    return EP_OK;
+    if (hipMalloc(&bf->d_fft, sizeof(FftArgs) * std::max(1, n)) != hipSuccess ||
+        hipMemcpy(bf->d_fft, fargs.data(), sizeof(FftArgs) * n, hipMemcpyHostToDevice) != hipSuccess)
+        return fail(EP_ENOMEM, "batch field: argument upload failed");
+    for (int k = 0; k < kFftClasses; ++k)
+        for (int stage = 0; stage < 3; ++stage)
+            if (!ftiles[k][stage].empty() &&
+                hipMalloc(&bf->fft[k].d[stage], sizeof(int2) * ftiles[k][stage].size()) != hipSuccess)
+                return fail(EP_ENOMEM, "batch field: hipMalloc of the FFT tiles failed");
+    return upload_fft_tiles(bf, ftiles);
 }
 
 ep_status batch_field_set_active(BatchField *bf, const std::vector<char> &active)
 {
     std::vector<int4> tiles[4];
+    std::vector<int2> ftiles[kFftClasses][3];
     for (int i = 0; i < bf->n_inst; ++i) {
         if (!active[i]) continue;
         const int M = bf->M_of[i];
+        if (fft_side(M)) {
+            fft_batch_tiles(i, M, ftiles);
+            continue;
+        }
         const int mt = ((M >> 1) + SBM - 1) / SBM, nt = (M + SBN - 1) / SBN;
         for (int stage = 0; stage < 4; ++stage)
             for (int z = 0; z < (stage >= 2 ? 2 : 1); ++z)
@@ -1081,7 +1155,7 @@ ep_status batch_field_set_active(BatchField *bf, const std::vector<char> &active
                       hipMemcpyHostToDevice) != hipSuccess)
             return fail(EP_EDEVICE, "batch field: tile upload failed");
     }
-    return EP_OK;
+    return upload_fft_tiles(bf, ftiles);
 }
 
 void batch_field_free(BatchField *bf)
@@ -1094,6 +1168,12 @@ void batch_field_free(BatchField *bf)
             if (bf->d_args[pi][st]) (void)hipFree(bf->d_args[pi][st]);
     for (int st = 0; st < 4; ++st)
         if (bf->d_tiles[st]) (void)hipFree(bf->d_tiles[st]);
+    for (float2 *t : bf->fft_tabs)
+        if (t) (void)hipFree(t);
+    for (int k = 0; k < kFftClasses; ++k)
+        for (int st = 0; st < 3; ++st)
+            if (bf->fft[k].d[st]) (void)hipFree(bf->fft[k].d[st]);
+    if (bf->d_fft) (void)hipFree(bf->d_fft);
     if (bf->fmax) (void)hipFree(bf->fmax);
     delete bf;
 }
@@ -1140,7 +1220,8 @@ void launch_stage_b(int precision, int stage, dim3 grid, const GemmArgs *args, c
 void launch_field_batch(BatchField *bf, int precision, hipStream_t s)
 {
     const int pi = prec_index(precision);
-    if (precision == EP_PREC_FP16X3)
+    launch_field_fft_batch(bf->d_fft, bf->fft, s);
+    if (precision == EP_PREC_FP16X3 && bf->n_tiles[0] > 0)
         hipLaunchKernelGGL(k_clear_max_b, dim3((bf->n_inst + 63) / 64), dim3(64), 0, s, bf->fmax, bf->n_inst);
     for (int stage = 0; stage < 4; ++stage) {
         if (bf->n_tiles[stage] == 0) continue;
@@ -1157,6 +1238,7 @@ void launch_field_batch(BatchField *bf, int precision, hipStream_t s)
 
 ep_status batch_field_autotune(BatchField *bf, int reps, hipStream_t s)
 {
+    if (bf->n_tiles[0] == 0) return EP_OK;  // no products to time
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
         if (e0) (void)hipEventDestroy(e0);

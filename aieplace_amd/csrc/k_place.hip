@@ -423,22 +423,24 @@ __global__ __launch_bounds__(kBlock) void k_cell_grad(
         const float2 gw = kGwCell ? (mov ? gwc : make_float2(0.f, 0.f))
                                   : sum_pin_partials(k0, k1, cell_pins, pin_grad);
         const float gwx = gw.x, gwy = gw.y, fx = f.x, fy = f.y;
-        const float pre = fmaxf(1.0f, (float)np + lambda * s.x * s.y);
-        const float gx = (gwx - lambda * fx) / pre, gy = (gwy - lambda * fy) / pre;
+        const float pre = fmaxf(1.0f, __fmaf_rn(lambda * s.x, s.y, (float)np));
+        const float gx = __fmaf_rn(-lambda, fx, gwx) / pre, gy = __fmaf_rn(-lambda, fy, gwy) / pre;
         gout[c] = make_float2(gx, gy);
         if (gw_out) gw_out[c] = make_float2(gwx, gwy);
         if (f_out) f_out[c] = make_float2(fx, fy);
+        // explicit multiply-adds: every instance of the template (and with it the
+        // forked and the single-branch evaluation) adds the same roundings
         if (kVref) {
             const double dx = (double)p.x - v0.x, dy = (double)p.y - v0.y;
-            acc[0] += dx * dx + dy * dy;
+            acc[0] = fma(dx, dx, fma(dy, dy, acc[0]));
         }
         if (kGref) {
             const double dx = (double)gx - g0.x, dy = (double)gy - g0.y;
-            acc[1] += dx * dx + dy * dy;
+            acc[1] = fma(dx, dx, fma(dy, dy, acc[1]));
         }
         acc[2] += fabs((double)gwx) + fabs((double)gwy);
         acc[3] += fabs((double)fx) + fabs((double)fy);
-        acc[4] += (double)gx * gx + (double)gy * gy;
+        acc[4] = fma((double)gx, (double)gx, fma((double)gy, (double)gy, acc[4]));
         if (!isfinite(gx) || !isfinite(gy)) acc[5] += 1.0;
         acc[6] = fmax(acc[6], fmax(fabs((double)gx), fabs((double)gy)));
     };

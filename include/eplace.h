@@ -37,7 +37,9 @@ enum {
     EP_EIO = 7       /* file missing, unreadable or malformed (LEF/DEF)   */
 };
 
-/* Arithmetic of the field-solve transform products. */
+/* Arithmetic of the field-solve transform products.  Grids whose sides are powers
+ * of two (up to 8192) need no products: FP32 FFTs solve them in every form, closer
+ * to the exact field than any of the products. */
 enum {
     EP_PREC_FP32 = 0,   /* FP32 operands, FP32 MFMA (v_mfma_f32_32x32x2_f32)        */
     EP_PREC_BF16X3 = 1, /* operands split hi+lo BF16, 3 MFMA products, FP32 accum */
@@ -200,7 +202,8 @@ typedef struct ep_kernel_stat {
     double avg_us;      /* event time per group launch                           */
     double bytes;       /* algorithmic (unique) HBM bytes per group launch       */
     double flops;       /* algorithmic flops per group launch: the dense transform
-                           products, 6 Mx My (Mx + My) per field solve          */
+                           products, 6 Mx My (Mx + My) per field solve (0 where
+                           FFTs solve it: memory-bound)                         */
 } ep_kernel_stat;
 ep_status ep_profile(ep_ctx *ctx, int32_t reps, ep_kernel_stat *out, int32_t cap, int32_t *n);
 

@@ -1,0 +1,53 @@
+"""Field solve by FFTs (power-of-two grids) against the FP64 oracle."""
+import math
+
+import numpy as np
+import pytest
+
+import aieplace_amd as A
+from aieplace_amd import api
+from aieplace_amd.batch import BatchPlacer
+
+pytestmark = pytest.mark.gpu
+
+
+# every last-stage radix, one and many FFTs per block, the smallest and the
+# largest side, both orientations of a long grid
+@pytest.mark.parametrize("mx,my", [(16, 16), (32, 16), (16, 64), (128, 32), (64, 256), (512, 128), (1024, 16),
+                                   (16, 2048), (4096, 16), (16, 8192), (8192, 32)])
+def test_field_matches_oracle(oracle, mx, my):
+    """Max-norm error within one rounding (2^-24) per butterfly level of the three
+    2-D transforms; the same field in every precision."""
+    print(f"case field fft {mx} x {my}", flush=True)
+    nl = A.generate("stdcell", seed=1, n_movable=2_000)
+    p = A.placer_params(A.CONFIGS["stdcell_200k"], bins_x=mx, bins_y=my)
+    xl, yl, xh, yh = nl.die
+    rng = np.random.default_rng(mx + my)
+    with A.Placer(nl, p) as pl:
+        pl.set_positions(xl + 0.7 * (xh - xl) * rng.random(pl.n_place), yl + 0.7 * (yh - yl) * rng.random(pl.n_place))
+        fmap, _, _, _ = pl.computeOverlaps()
+        fields = [pl.computeElectricFields(k) for k in (api.EP_PREC_FP32, api.EP_PREC_BF16X3, api.EP_PREC_FP16X3)]
+    bw, bh = (xh - xl) / mx, (yh - yl) / my
+    _, ex, ey = oracle.field(fmap.astype(np.float64) / (bw * bh), wy_scale=bw / bh)
+    tol = 2.0 ** -24 * 3 * math.log2(mx * my)
+    for got in fields:
+        err = [np.abs(g - e).max() / np.abs(e).max() for g, e in zip(got, (ex, ey))]
+        print(f"  {err[0]:.2e} {err[1]:.2e} (tolerance {tol:.2e})", flush=True)
+        assert max(err) <= tol
+
+
+def test_batch_mixes_ffts_and_products():
+    """A batch with grids on both paths reproduces its single-instance runs."""
+    bins = [32, 96, 256, 2048]
+    nls = [A.generate("stdcell", seed=k + 1, n_movable=2_000) for k in range(len(bins))]
+    p = A.placer_params(A.CONFIGS["stdcell_200k"], max_iters=6)
+    with BatchPlacer(nls, bins, p) as bp:
+        bp.run()
+        got = [bp.positions(i) for i in range(len(bins))]
+    for nl, b, (x, y) in zip(nls, bins, got):
+        q = A.placer_params(A.CONFIGS["stdcell_200k"], bins_x=b, bins_y=b, max_iters=6, use_graph=1)
+        with A.Placer(nl, q) as pl:
+            pl.run()
+            sx, sy = pl.get_positions()
+        print(f"  bins {b}", flush=True)
+        assert np.array_equal(x, sx) and np.array_equal(y, sy), b
