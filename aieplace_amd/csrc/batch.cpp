@@ -95,6 +95,7 @@ struct ep_batch {
     // Per-instance block counts and WA buckets (blk0 relative to the instance):
     // the block tables cover the instances in `active` only and are rebuilt
     // from these when finished instances are dropped (set_tables).
+    int sort_cpt = kSortBatchMost;  // cells per thread of the sort_blocks kernels
     std::vector<int32_t> nb_cell, nb_sort, nb_bin, nb_wa, nb_dens[3];
     std::vector<std::vector<BBucket>> inst_buckets;
     std::vector<char> active;
@@ -147,6 +148,7 @@ struct ep_batch {
         d.dens_wcap = dens_wcap;
         d.pre_cell = pre_cell;
         d.pre_sort = pre_sort;
+        d.sort_cpt = sort_cpt;
         d.pre_dens = pre_dens[dens_variant];
         d.pre_bin = pre_bin;
         d.pre_wa = pre_wa;
@@ -442,8 +444,6 @@ extern "C" ep_status ep_batch_create(const ep_netlist *const *nls, const int32_t
         fixmap.insert(fixmap.end(), L.fixmap.begin(), L.fixmap.end());
         // block tables
         pre_cell.push_back(pre_cell.back() + (int32_t)((L.n_place + kBlock - 1) / kBlock));
-        pre_sort.push_back(pre_sort.back() + (int32_t)((L.n_place + kBlock * kSortCellsPerThread - 1) /
-                                                       (kBlock * kSortCellsPerThread)));
         for (int v = 0; v < 3; ++v) {
             DensPlan dv{};
             dv.level = I.dens_level;
@@ -455,7 +455,6 @@ extern "C" ep_status ep_batch_create(const ep_netlist *const *nls, const int32_t
         pre_wa.push_back((int32_t)wa_base);
         const size_t ni = pre_cell.size() - 1;
         b->nb_cell.push_back(pre_cell[ni] - pre_cell[ni - 1]);
-        b->nb_sort.push_back(pre_sort[ni] - pre_sort[ni - 1]);
         b->nb_bin.push_back(pre_bin[ni] - pre_bin[ni - 1]);
         b->nb_wa.push_back(pre_wa[ni] - pre_wa[ni - 1]);
         for (int v = 0; v < 3; ++v) b->nb_dens[v].push_back(pre_dens[v][ni] - pre_dens[v][ni - 1]);
@@ -467,6 +466,12 @@ extern "C" ep_status ep_batch_create(const ep_netlist *const *nls, const int32_t
     }
     cps.push_back((int32_t)cpin_base);
     b->total_cells = cell_off;
+    b->sort_cpt = sort_cells_per_thread(cell_off, kSortBatchMost, kSortBatchBlocks);
+    for (const BInst &I : b->inst) {
+        const int64_t per_block = (int64_t)kBlock * b->sort_cpt;
+        b->nb_sort.push_back((int32_t)((I.n_place + per_block - 1) / per_block));
+        pre_sort.push_back(pre_sort.back() + b->nb_sort.back());
+    }
     b->active.assign(n, 1);
     b->init_pos = pos;
     b->n_buckets = (int)bks.size();

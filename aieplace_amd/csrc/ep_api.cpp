@@ -637,7 +637,9 @@ extern "C" ep_status ep_create(const ep_netlist *nl, const ep_params *p, ep_ctx 
     c->part_wa_off = 0;
     c->part_ovf_off = 2 * c->wa_part_blocks;
     c->part_cell_off = c->part_ovf_off + 4 * c->ovf_blocks;
-    c->trial_blocks = (int)(((int64_t)c->n_place + kBlock * kSortCellsPerThread - 1) / (kBlock * kSortCellsPerThread));
+    c->sort_cpt = sort_cells_per_thread(c->n_place, kSortMost, kSortBlocks);
+    const int64_t per_block = (int64_t)kBlock * c->sort_cpt;
+    c->trial_blocks = (int)((c->n_place + per_block - 1) / per_block);
     c->part_trial_off = c->part_cell_off + 7 * c->cell_blocks;
     c->part_total = c->part_trial_off + c->trial_blocks;
 #define EP_TRY(x)                 \

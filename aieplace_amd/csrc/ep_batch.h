@@ -93,7 +93,8 @@ struct BDev {
     int32_t *dens_tab;           // [n_inst * (kSortTiles + 1)] density block tables
     int32_t dens_wcap;           // LDS window capacity per plane (bins), max over instances
     const int32_t *pre_cell;     // 256 cells per block
-    const int32_t *pre_sort;     // kBlock * kSortCellsPerThread cells per block
+    const int32_t *pre_sort;     // kBlock * sort_cpt cells per block
+    int32_t sort_cpt;
     const int32_t *pre_dens;     // density blocks per instance (dens_grid bound)
     const int32_t *pre_bin;      // kBinsPerBlock bins per block
     const int32_t *pre_wa;       // WA blocks of each instance (instance-major buckets)
@@ -107,7 +108,7 @@ enum BCtlMode { kCtlGamma = 0, kCtlLambda = 1, kCtlProbe = 2, kCtlAlpha = 3, kCt
 enum BMoveMode { kMoveTrial = 0, kMoveProbe = 1, kMoveInitU = 2 };
 
 // ---- batched launchers (k_batch.hip)
-// Blocks of kBlock * kSortCellsPerThread cells (the sort's layout); kMoveTrial
+// Blocks of kBlock * sort_cpt cells (the sort's layout); kMoveTrial
 // also counts the trial positions into the sort tiles.
 void bl_move(const BDev &d, int mode, int sort_blocks, hipStream_t s);
 // Density maps of every unfinished instance; `counted`: a kMoveTrial move made

@@ -25,6 +25,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 #include <vector>
 
 #include "ep_common.h"
@@ -41,7 +42,33 @@ constexpr int kCellGridCap = 16384;
 // Spatial counting sort of cells: kSortSide x kSortSide coarse tiles.
 constexpr int kSortSide = 32;
 constexpr int kSortTiles = kSortSide * kSortSide;
-constexpr int kSortCellsPerThread = 16;
+// Cells per thread of the kernels that count or scatter cells by tile (the trial
+// move among them): the most, up to `most`, that still gives `blocks` blocks.
+// Few cells per thread spread a small instance over the CUs; many share the
+// clearing and flushing of a block's 1024 tile counts.  Placements of 100
+// iterations, 1 / 2 / 4 / 8 / 16 cells per thread (ms): 20k cells 7.42 / 7.42 / 7.60 /
+// 7.95 / 8.88, 75k 8.69 / 8.49 / 8.45 / 8.92 / 9.81, 200k 11.3 / 10.7 / 10.5 / 10.8 /
+// 11.6, 500k 18.7 / 16.8 / 16.1 / 16.0 / 16.6, 1M 25.4 / 22.4 / 21.1 / 19.9 / 20.9, 2M
+// 40.8 / 35.3 / 32.7 / 31.6 / 31.6.  A batch's blocks stop at its instances' ends:
+// 16 instances (450k cells in all) 12.6 / 12.6 / 12.7 / 13.0 / 13.9, 64 (3.7M) 53.7 /
+// 50.8 / 50.3 / 50.9 / 51.5.
+constexpr int kSortMost = 8, kSortBlocks = 160;
+constexpr int kSortBatchMost = 4, kSortBatchBlocks = 512;
+inline int sort_cells_per_thread(int64_t n, int most, int blocks)
+{
+    int cpt = most;
+    while (cpt > 1 && n < (int64_t)kBlock * cpt * blocks) cpt >>= 1;
+    return cpt;
+}
+// go(cpt) with the count as a template argument.
+template <class Go>
+inline void with_sort_cpt(int cpt, Go go)
+{
+    if (cpt == 8) go(std::integral_constant<int, 8>());
+    else if (cpt == 4) go(std::integral_constant<int, 4>());
+    else if (cpt == 2) go(std::integral_constant<int, 2>());
+    else go(std::integral_constant<int, 1>());
+}
 // After a rejected model proposal the model sits out 2, 4, ... up to this many
 // iterations (reset by an accepted proposal): phases where it mispredicts cost
 // one extra evaluation per rejection, so they are skipped.
@@ -304,6 +331,7 @@ struct Ctx {
     unsigned *fin_ticket = nullptr;  // finalize blocks done (0 between launches)
     int32_t part_wa_off = 0, part_ovf_off = 0, part_cell_off = 0, part_trial_off = 0, part_total = 0;
     int32_t wa_part_blocks = 0, ovf_blocks = 0, cell_blocks = 0, trial_blocks = 0;
+    int32_t sort_cpt = kSortMost;  // cells per thread of the trial_blocks kernels
     DevScalars *d_scal = nullptr, *h_scal = nullptr;  // device / pinned host
     DevResult *d_res = nullptr, *h_res = nullptr;
 

@@ -59,7 +59,8 @@ __device__ inline const float2 *eval_pos(const BDev &d, int cur, int at)
 // kMoveTrial: u' = clamp(v - alpha g), v' = clamp(u' + coef (u' - u)) into the
 // other parity, counting v' into the instance's sort tiles (the evaluation's
 // sort then skips its counting pass); kMoveProbe: v_-1 = clamp(v - eps g);
-// kMoveInitU: u = v.  Blocks take kBlock * kSortCellsPerThread cells (pre_sort).
+// kMoveInitU: u = v.  Blocks take kBlock * CPT cells (pre_sort).
+template <int CPT>
 __global__ __launch_bounds__(kBlock) void kb_move(BDev d, int mode)
 {
     __shared__ int hist[kSortTiles];
@@ -74,7 +75,7 @@ __global__ __launch_bounds__(kBlock) void kb_move(BDev d, int mode)
     }
     const int a = S->cur;
     const GeomArgs g = inst_geom(I);
-    const int base = (blockIdx.x - d.pre_sort[i]) * kBlock * kSortCellsPerThread;
+    const int base = (blockIdx.x - d.pre_sort[i]) * kBlock * CPT;
     if (mode == kMoveTrial) {
         // All of the thread's cells are loaded before the first is moved, so
         // the loads overlap; a cell past n_place loads the instance's last
@@ -83,10 +84,10 @@ __global__ __launch_bounds__(kBlock) void kb_move(BDev d, int mode)
         const float2 *V = pick<const float2 *>(d.V[0], d.V[1], a);
         const float2 *U = pick<const float2 *>(d.U[0], d.U[1], a);
         const float2 *G = pick<const float2 *>(d.G[0], d.G[1], a);
-        float2 s[kSortCellsPerThread], vv[kSortCellsPerThread], uu[kSortCellsPerThread],
-            gg[kSortCellsPerThread];
+        float2 s[CPT], vv[CPT], uu[CPT],
+            gg[CPT];
 #pragma unroll
-        for (int k = 0; k < kSortCellsPerThread; ++k) {
+        for (int k = 0; k < CPT; ++k) {
             const int c = I.cell_off + min(base + k * kBlock + (int)threadIdx.x, I.n_place - 1);
             s[k] = d.wh[c];
             vv[k] = V[c];
@@ -94,7 +95,7 @@ __global__ __launch_bounds__(kBlock) void kb_move(BDev d, int mode)
             gg[k] = G[c];
         }
 #pragma unroll
-        for (int k = 0; k < kSortCellsPerThread; ++k) {
+        for (int k = 0; k < CPT; ++k) {
             const int lc = base + k * kBlock + threadIdx.x;
             const float2 un =
                 clamp_cell(make_float2(vv[k].x - alpha * gg[k].x, vv[k].y - alpha * gg[k].y), s[k], g);
@@ -109,7 +110,7 @@ __global__ __launch_bounds__(kBlock) void kb_move(BDev d, int mode)
         }
     }
 #pragma unroll
-    for (int k = 0; k < kSortCellsPerThread && mode != kMoveTrial; ++k) {
+    for (int k = 0; k < CPT && mode != kMoveTrial; ++k) {
         const int lc = base + k * kBlock + threadIdx.x;
         if (lc >= I.n_place) continue;
         const int c = I.cell_off + lc;
@@ -134,6 +135,7 @@ __global__ __launch_bounds__(kBlock) void kb_move(BDev d, int mode)
 
 // ------------------------------------------------------------------ maps
 
+template <int CPT>
 __global__ __launch_bounds__(kBlock) void kb_sort_count(BDev d, int at)
 {
     __shared__ int hist[kSortTiles];
@@ -145,9 +147,9 @@ __global__ __launch_bounds__(kBlock) void kb_sort_count(BDev d, int at)
     const GeomArgs g = inst_geom(I);
     for (int t = threadIdx.x; t < kSortTiles; t += kBlock) hist[t] = 0;
     __syncthreads();
-    const int base = (blockIdx.x - d.pre_sort[i]) * kBlock * kSortCellsPerThread;
+    const int base = (blockIdx.x - d.pre_sort[i]) * kBlock * CPT;
 #pragma unroll
-    for (int k = 0; k < kSortCellsPerThread; ++k) {
+    for (int k = 0; k < CPT; ++k) {
         const int idx = base + k * kBlock + threadIdx.x;
         if (idx < I.n_place) {
             const int c = I.cell_off + idx;
@@ -170,6 +172,7 @@ __global__ __launch_bounds__(kSortScanThreads) void kb_sort_scan(BDev d, int K)
                     d.dens_tab + (size_t)i * (kSortTiles + 1), d.inst[i].dens_level, K);
 }
 
+template <int CPT>
 __global__ __launch_bounds__(kBlock) void kb_sort_scatter(BDev d, int at)
 {
     __shared__ int hist[kSortTiles];
@@ -182,20 +185,20 @@ __global__ __launch_bounds__(kBlock) void kb_sort_scatter(BDev d, int at)
     const GeomArgs g = inst_geom(I);
     for (int t = threadIdx.x; t < kSortTiles; t += kBlock) hist[t] = 0;
     __syncthreads();
-    const int base = (blockIdx.x - d.pre_sort[i]) * kBlock * kSortCellsPerThread;
-    int key[kSortCellsPerThread], rank[kSortCellsPerThread];
-    float4 cell[kSortCellsPerThread];
+    const int base = (blockIdx.x - d.pre_sort[i]) * kBlock * CPT;
+    int key[CPT], rank[CPT];
+    float4 cell[CPT];
     // All of the thread's cells are loaded before the first tile count; a
     // cell past n_place loads the instance's last cell (value unused).
-    float2 p[kSortCellsPerThread], s[kSortCellsPerThread];
+    float2 p[CPT], s[CPT];
 #pragma unroll
-    for (int k = 0; k < kSortCellsPerThread; ++k) {
+    for (int k = 0; k < CPT; ++k) {
         const int c = I.cell_off + min(base + k * kBlock + (int)threadIdx.x, I.n_place - 1);
         p[k] = pos[c];
         s[k] = d.wh[c];
     }
 #pragma unroll
-    for (int k = 0; k < kSortCellsPerThread; ++k) {
+    for (int k = 0; k < CPT; ++k) {
         const int idx = base + k * kBlock + threadIdx.x;
         key[k] = -1;
         if (idx < I.n_place) {
@@ -211,7 +214,7 @@ __global__ __launch_bounds__(kBlock) void kb_sort_scatter(BDev d, int at)
     __syncthreads();
     float4 *sorted = d.sorted + I.cell_off;
 #pragma unroll
-    for (int k = 0; k < kSortCellsPerThread; ++k)
+    for (int k = 0; k < CPT; ++k)
         if (key[k] >= 0) {
             const int slot = base_of[key[k]] + rank[k];
             if (slot < I.n_place) sorted[slot] = cell[k];  // counts always sum to n_place
@@ -566,15 +569,22 @@ bool bl_density_cpt_supported(int cpt) { return cpt == 2 || cpt == 4 || cpt == 8
 
 void bl_move(const BDev &d, int mode, int sort_blocks, hipStream_t s)
 {
-    hipLaunchKernelGGL(kb_move, dim3(sort_blocks), dim3(kBlock), 0, s, d, mode);
+    with_sort_cpt(d.sort_cpt, [&](auto cpt) {
+        hipLaunchKernelGGL(kb_move<decltype(cpt)::value>, dim3(sort_blocks), dim3(kBlock), 0, s, d, mode);
+    });
 }
 
 void bl_sort(const BDev &d, int at, bool counted, int bin_blocks, int sort_blocks, int dens_cpt,
              hipStream_t s)
 {
-    if (!counted) hipLaunchKernelGGL(kb_sort_count, dim3(sort_blocks), dim3(kBlock), 0, s, d, at);
+    if (!counted)
+        with_sort_cpt(d.sort_cpt, [&](auto cpt) {
+            hipLaunchKernelGGL(kb_sort_count<decltype(cpt)::value>, dim3(sort_blocks), dim3(kBlock), 0, s, d, at);
+        });
     hipLaunchKernelGGL(kb_sort_scan, dim3(d.n_inst), dim3(kSortScanThreads), 0, s, d, kBlock * dens_cpt);
-    hipLaunchKernelGGL(kb_sort_scatter, dim3(sort_blocks), dim3(kBlock), 0, s, d, at);
+    with_sort_cpt(d.sort_cpt, [&](auto cpt) {
+        hipLaunchKernelGGL(kb_sort_scatter<decltype(cpt)::value>, dim3(sort_blocks), dim3(kBlock), 0, s, d, at);
+    });
 }
 
 void bl_dens(const BDev &d, int bin_blocks, int dens_blocks, int dens_cpt, bool map_range, hipStream_t s)

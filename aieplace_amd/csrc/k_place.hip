@@ -48,6 +48,7 @@ __global__ void k_fill_maps(unsigned long long *__restrict__ acc_field,
 // accumulate in LDS and flush with coalesced atomics.
 
 
+template <int CPT>
 __global__ __launch_bounds__(kBlock) void k_sort_count(Pair<const float2> pos_pair,
                                                        const float2 *__restrict__ wh, int n_place,
                                                        GeomArgs g, int Mx, int My,
@@ -59,9 +60,9 @@ __global__ __launch_bounds__(kBlock) void k_sort_count(Pair<const float2> pos_pa
     __shared__ int hist[kSortTiles];
     for (int t = threadIdx.x; t < kSortTiles; t += kBlock) hist[t] = 0;
     __syncthreads();
-    const int base = blockIdx.x * kBlock * kSortCellsPerThread;
+    const int base = blockIdx.x * kBlock * CPT;
 #pragma unroll
-    for (int k = 0; k < kSortCellsPerThread; ++k) {
+    for (int k = 0; k < CPT; ++k) {
         const int idx = base + k * kBlock + threadIdx.x;
         if (idx < n_place) atomicAdd(&hist[cell_key(pos[idx], wh[idx], g, Mx, My)], 1);
     }
@@ -84,6 +85,7 @@ __global__ __launch_bounds__(kSortScanThreads) void k_sort_scan(int32_t *__restr
 
 // Writes every cell, packed with its size and movable flag (pack_cell), to its
 // slot of the tile-sorted order.
+template <int CPT>
 __global__ __launch_bounds__(kBlock) void k_sort_scatter(Pair<const float2> pos_pair,
                                                          const float2 *__restrict__ wh, int n_place,
                                                          int n_mov, GeomArgs g, int Mx, int My,
@@ -97,20 +99,20 @@ __global__ __launch_bounds__(kBlock) void k_sort_scatter(Pair<const float2> pos_
     __shared__ int base_of[kSortTiles];
     for (int t = threadIdx.x; t < kSortTiles; t += kBlock) hist[t] = 0;
     __syncthreads();
-    const int base = blockIdx.x * kBlock * kSortCellsPerThread;
-    int key[kSortCellsPerThread], rank[kSortCellsPerThread];
-    float4 cell[kSortCellsPerThread];
+    const int base = blockIdx.x * kBlock * CPT;
+    int key[CPT], rank[CPT];
+    float4 cell[CPT];
     // All of the thread's cells are loaded before the first tile count, so
     // the loads overlap; a cell past n_place loads the last cell (unused).
-    float2 p[kSortCellsPerThread], s[kSortCellsPerThread];
+    float2 p[CPT], s[CPT];
 #pragma unroll
-    for (int k = 0; k < kSortCellsPerThread; ++k) {
+    for (int k = 0; k < CPT; ++k) {
         const int idx = min(base + k * kBlock + (int)threadIdx.x, n_place - 1);
         p[k] = pos[idx];
         s[k] = wh[idx];
     }
 #pragma unroll
-    for (int k = 0; k < kSortCellsPerThread; ++k) {
+    for (int k = 0; k < CPT; ++k) {
         const int idx = base + k * kBlock + threadIdx.x;
         key[k] = -1;
         if (idx < n_place) {
@@ -124,7 +126,7 @@ __global__ __launch_bounds__(kBlock) void k_sort_scatter(Pair<const float2> pos_
         if (hist[t]) base_of[t] = atomicAdd(&off[t], hist[t]);
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < kSortCellsPerThread; ++k)
+    for (int k = 0; k < CPT; ++k)
         if (key[k] >= 0) {
             const int slot = base_of[key[k]] + rank[k];
             if (slot < n_place) sorted[slot] = cell[k];  // counts always sum to n_place
@@ -627,7 +629,8 @@ __global__ __launch_bounds__(kFinalizeThreads) void k_finalize(
 // u' = clamp(v - alpha g); v' = clamp(u' + coef (u' - u))   (ePlace Nesterov step)
 // With `count`, the new positions are also counted into the sort's coarse
 // tiles (the first pass of launch_sort, which then skips it).  Blocks take
-// kBlock * kSortCellsPerThread cells, as k_sort_count.
+// kBlock * CPT cells, as k_sort_count.
+template <int CPT>
 __global__ __launch_bounds__(kBlock) void k_trial(Pair<const float2> v_pair,
                                                   Pair<const float2> u_pair,
                                                   Pair<const float2> g_pair,
@@ -652,13 +655,13 @@ __global__ __launch_bounds__(kBlock) void k_trial(Pair<const float2> v_pair,
         __syncthreads();
     }
     const float alpha = sc->alpha, coef = sc->coef;
-    const int base = blockIdx.x * kBlock * kSortCellsPerThread;
+    const int base = blockIdx.x * kBlock * CPT;
     double dv2[1] = {0.0};  // |v' - v|^2, for the step-length estimate
     // One cell per pass: every wave of the grid walks the same slice k at
-    // about the same time.  Loading all of a thread's cells first measured
+    // about the same time.  Loading all of a thread's 16 cells first measured
     // slower at 2M cells (22.4 -> 25.7 us; groups of four cells: 23.5 us).
 #pragma unroll
-    for (int k = 0; k < kSortCellsPerThread; ++k) {
+    for (int k = 0; k < CPT; ++k) {
         const int c = base + k * kBlock + threadIdx.x;
         if (c < n_place) {
             const float2 s = wh[c], vv = v[c], uu = u[c], gg = gr[c];
@@ -928,14 +931,19 @@ void launch_fill_maps(Ctx &c, hipStream_t s)
 
 void launch_sort(Ctx &c, Pair<const float2> pos, bool counted, hipStream_t s)
 {
-    const int blocks = grid_for(c.n_place, kBlock * kSortCellsPerThread, INT_MAX);
-    if (!counted)
-        hipLaunchKernelGGL(k_sort_count, dim3(blocks), dim3(kBlock), 0, s, pos, c.wh, c.n_place,
-                           geom_args(c), c.Mx, c.My, c.sort_count, c.d_scal);
+    with_sort_cpt(c.sort_cpt, [&](auto cpt) {
+        constexpr int CPT = decltype(cpt)::value;
+        if (!counted)
+            hipLaunchKernelGGL(k_sort_count<CPT>, dim3(c.trial_blocks), dim3(kBlock), 0, s, pos, c.wh, c.n_place,
+                               geom_args(c), c.Mx, c.My, c.sort_count, c.d_scal);
+    });
     hipLaunchKernelGGL(k_sort_scan, dim3(1), dim3(kSortScanThreads), 0, s, c.sort_count, c.sort_off,
                        c.dens_tab, c.dens.level, kBlock * c.dens.cpt, c.d_scal);
-    hipLaunchKernelGGL(k_sort_scatter, dim3(blocks), dim3(kBlock), 0, s, pos, c.wh, c.n_place,
-                       c.n_mov, geom_args(c), c.Mx, c.My, c.sort_off, c.sorted, c.d_scal);
+    with_sort_cpt(c.sort_cpt, [&](auto cpt) {
+        constexpr int CPT = decltype(cpt)::value;
+        hipLaunchKernelGGL(k_sort_scatter<CPT>, dim3(c.trial_blocks), dim3(kBlock), 0, s, pos, c.wh, c.n_place,
+                           c.n_mov, geom_args(c), c.Mx, c.My, c.sort_off, c.sorted, c.d_scal);
+    });
 }
 
 void launch_density(Ctx &c, hipStream_t s)
@@ -1028,10 +1036,12 @@ void launch_finalize_decide(Ctx &c, const CtlParams &p, hipStream_t s)
 void launch_trial(Ctx &c, Pair<const float2> v, Pair<const float2> u, Pair<const float2> g,
                   Pair<float2> v_new, Pair<float2> u_new, bool count, hipStream_t s)
 {
-    const int blocks = grid_for(c.n_place, kBlock * kSortCellsPerThread, INT_MAX);
-    hipLaunchKernelGGL(k_trial, dim3(blocks), dim3(kBlock), 0, s, v, u, g, c.wh, c.n_place,
-                       geom_args(c), c.Mx, c.My, c.d_scal, v_new, u_new,
-                       count ? c.sort_count : nullptr, count ? c.part + c.part_trial_off : nullptr);
+    with_sort_cpt(c.sort_cpt, [&](auto cpt) {
+        constexpr int CPT = decltype(cpt)::value;
+        hipLaunchKernelGGL(k_trial<CPT>, dim3(c.trial_blocks), dim3(kBlock), 0, s, v, u, g, c.wh, c.n_place,
+                           geom_args(c), c.Mx, c.My, c.d_scal, v_new, u_new,
+                           count ? c.sort_count : nullptr, count ? c.part + c.part_trial_off : nullptr);
+    });
 }
 
 void launch_step_begin(Ctx &c, const CtlParams &p, hipStream_t s)

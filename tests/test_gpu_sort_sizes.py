@@ -1,0 +1,39 @@
+"""Tile sort and trial move at the sizes where their cells per thread change."""
+import numpy as np
+import pytest
+
+import aieplace_amd as A
+from aieplace_amd import api
+
+pytestmark = pytest.mark.gpu
+
+
+def maps_of(pl):
+    out = [np.zeros(pl.bins, np.float32) for _ in range(2)]
+    api.check(api.lib.ep_get_density(pl._ctx, api.fptr(out[0]), api.fptr(out[1]), None))
+    return out
+
+
+# 1 | 2 | 4 | 8 cells per thread begin at 256 x 160 times as many cells; one block,
+# and the last of a block's cells missing
+@pytest.mark.parametrize("n", [100, 255, 81_919, 81_921, 163_839, 163_840, 327_679, 327_681])
+def test_counted_and_uncounted_sort_agree(n):
+    """The maps of a trial (counted by the move) equal those of the same positions
+    sorted afresh, and hold the movable cells' whole area."""
+    print(f"case sort n={n}", flush=True)
+    nl = A.generate("stdcell", seed=2, n_movable=n)
+    p = A.placer_params(A.CONFIGS["stdcell_200k"], bins_x=128, bins_y=128, use_fillers=0, use_graph=1, max_iters=3)
+    xl, yl, xh, yh = nl.die
+    rng = np.random.default_rng(n)
+    with A.Placer(nl, p) as pl:
+        assert pl.n_place == n
+        pl.set_positions(xl + rng.random(n) * (xh - xl), yl + rng.random(n) * (yh - yl))
+        r = pl.run()
+        assert r["iterations"] >= 1
+        run_field, run_mov = maps_of(pl)
+        field, mov, _, tau = pl.computeOverlaps()
+    assert np.array_equal(run_field, field) and np.array_equal(run_mov, mov)
+    area = float((nl.w[:n].astype(np.float64) * nl.h[:n]).sum())
+    # 2^-24 relative per coordinate of up to 128 bins
+    assert abs(mov.sum(dtype=np.float64) - area) <= 2.0 ** -15 * area
+    assert tau == r["overflow"]
