@@ -537,7 +537,7 @@ extern "C" ep_status ep_batch_create(const ep_netlist *const *nls, const int32_t
     EPB_TRY(dalloc(&b->map_mean, n));
     EPB_TRY(dalloc(&b->map_max, n));
     EPB_TRY(dalloc(&b->sorted, nc));
-    EPB_TRY(dalloc(&b->sort_count, (size_t)n * kSortTiles));
+    EPB_TRY(dalloc(&b->sort_count, (size_t)n * 2 * kSortTiles));
     EPB_TRY(dalloc(&b->sort_off, (size_t)n * kSortTiles));
     EPB_TRY(dalloc(&b->dens_tab, (size_t)n * (kSortTiles + 1)));
     EPB_TRY(dalloc(&b->pre_cell, n + 1));
@@ -572,7 +572,7 @@ extern "C" ep_status ep_batch_create(const ep_netlist *const *nls, const int32_t
     EPB_TRY(upload(b->buckets, bks));
     if (hipMemset(b->pin_grad, 0, sizeof(float2) * std::max<size_t>(1, pin_cell.size())) != hipSuccess ||
         hipMemset(b->exy, 0, sizeof(float2) * nb) != hipSuccess ||
-        hipMemset(b->sort_count, 0, sizeof(int32_t) * n * kSortTiles) != hipSuccess ||
+        hipMemset(b->sort_count, 0, sizeof(int32_t) * n * 2 * kSortTiles) != hipSuccess ||
         hipMemset(b->part_wa, 0, sizeof(double) * 2 * std::max(1, b->wa_blocks)) != hipSuccess ||
         hipMemset(b->part_ovf, 0, sizeof(double) * 4 * b->bin_blocks) != hipSuccess ||
         hipMemset(b->part_cell, 0, sizeof(double) * 7 * b->cell_blocks) != hipSuccess ||

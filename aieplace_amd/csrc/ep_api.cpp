@@ -669,7 +669,7 @@ extern "C" ep_status ep_create(const ep_netlist *nl, const ep_params *p, ep_ctx 
     EP_TRY(dalloc(&c->acc_mov, nb));
     EP_TRY(dalloc(&c->map_fix, nb));
     EP_TRY(dalloc(&c->sorted, std::max(1, c->n_place)));
-    EP_TRY(dalloc(&c->sort_count, kSortTiles));
+    EP_TRY(dalloc(&c->sort_count, 2 * kSortTiles));
     EP_TRY(dalloc(&c->sort_off, kSortTiles));
     EP_TRY(dalloc(&c->dens_tab, kSortTiles + 1));
     EP_TRY(dalloc(&c->exy, nb));
@@ -710,7 +710,7 @@ extern "C" ep_status ep_create(const ep_netlist *nl, const ep_params *p, ep_ctx 
         hipMemset(c->fin_ticket, 0, sizeof(unsigned)) != hipSuccess ||
         hipMemset(c->acc_field, 0, sizeof(unsigned long long) * nb) != hipSuccess ||
         hipMemset(c->acc_mov, 0, sizeof(unsigned long long) * nb) != hipSuccess ||
-        hipMemset(c->sort_count, 0, sizeof(int32_t) * kSortTiles) != hipSuccess) {
+        hipMemset(c->sort_count, 0, sizeof(int32_t) * 2 * kSortTiles) != hipSuccess) {
         destroy_ctx(c);
         return fail(EP_EDEVICE, "ep_create: hipMemset failed");
     }
@@ -1505,7 +1505,10 @@ extern "C" ep_status ep_profile(ep_ctx *c, int32_t reps, ep_kernel_stat *out, in
         EP_HIP(hipEventRecord(e0, c->stream));
         for (int r = 0; r < reps; ++r) {
             const std::string nm = it.name;
-            if (nm == "cell_sort") launch_sort(*c, c->V[a], false, c->stream);
+            if (nm == "cell_sort") {
+                launch_sort_clear(*c, c->stream);
+                launch_sort(*c, c->V[a], false, c->stream);
+            }
             else if (nm == "density_scatter") launch_density(*c, c->stream);
             else if (nm == "overflow") launch_overflow(*c, c->stream);
             else if (nm == "wa_grad") launch_wa(*c, c->V[a], c->stream);
@@ -1519,9 +1522,8 @@ extern "C" ep_status ep_profile(ep_ctx *c, int32_t reps, ep_kernel_stat *out, in
             else launch_finalize(*c, c->stream, true);
         }
         EP_HIP(hipEventRecord(e1, c->stream));
-        // the counting trials left tile counts behind: consume them (the scan
-        // clears the counts) before anything else sorts
-        if (std::string(it.name) == "nesterov_trial") launch_sort(*c, c->V[b], true, c->stream);
+        // the counting trials left tile counts behind
+        if (std::string(it.name) == "nesterov_trial") launch_sort_clear(*c, c->stream);
         EP_HIP(hipEventSynchronize(e1));
         ep_status st = check_launch();
         if (st != EP_OK) return st;
@@ -1543,6 +1545,7 @@ extern "C" ep_status ep_profile(ep_ctx *c, int32_t reps, ep_kernel_stat *out, in
     for (int cpt : {2, 4, 8, 16}) {
         if (cpt == cpt0) continue;
         c->dens.cpt = cpt;
+        launch_sort_clear(*c, c->stream);
         launch_sort(*c, c->V[a], false, c->stream);
         EP_HIP(hipEventRecord(e0, c->stream));
         for (int r = 0; r < reps; ++r) launch_density(*c, c->stream);
@@ -1567,6 +1570,7 @@ extern "C" ep_status ep_profile(ep_ctx *c, int32_t reps, ep_kernel_stat *out, in
     *n = k;
     // leave the maps consistent with the current positions
     launch_fill_maps(*c, c->stream);
+    launch_sort_clear(*c, c->stream);
     launch_sort(*c, c->V[a], false, c->stream);
     launch_density(*c, c->stream);
     launch_overflow(*c, c->stream);

@@ -6,7 +6,8 @@
 //   bins  [2*map_off, 2*map_off + 2*M*M) of the transform scratch tA/tB
 //   nets and pins: contiguous ranges of net_start/pin_cell/pin_off/pin_grad,
 //   with net_start holding global pin indices and pin_cell global cell indices
-//   sort tiles [i*kSortTiles, (i+1)*kSortTiles) of sort_count/sort_off.
+//   sort tiles [i*kSortTiles, (i+1)*kSortTiles) of sort_off, and twice as many
+//   (tile counts, cursors) of sort_count.
 // Blocks of every kernel map to instances through prefix tables (the blocks
 // of instance i are [pre[i], pre[i+1])); blocks of a finished instance return
 // at once, so a replay costs only the unfinished instances' work.

@@ -217,6 +217,8 @@ void launch_fill_maps(Ctx &c, hipStream_t s);
 // Tile-sorts the cells at pos; `counted`: the tile counts were already made by
 // a counting launch_trial at the same positions.
 void launch_sort(Ctx &c, Pair<const float2> pos, bool counted, hipStream_t s);
+// Clears the sort's counts, as launch_overflow does (for sorts without one between).
+void launch_sort_clear(Ctx &c, hipStream_t s);
 // Scatters the cells packed by the last launch_sort (same positions).
 void launch_density(Ctx &c, hipStream_t s);
 void launch_overflow(Ctx &c, hipStream_t s);
@@ -314,7 +316,8 @@ struct Ctx {
     float *map_field = nullptr, *map_mov = nullptr, *map_fix = nullptr;
     unsigned long long *acc_field = nullptr, *acc_mov = nullptr;  // fixed-point scatter targets
     float4 *sorted = nullptr;                        // packed cells in coarse-tile order
-    int32_t *sort_count = nullptr, *sort_off = nullptr;  // kSortTiles each
+    int32_t *sort_count = nullptr;                   // 2 x kSortTiles: tile counts, cursors (zero between evaluations)
+    int32_t *sort_off = nullptr;                     // kSortTiles: end of each tile's run
     int32_t *dens_tab = nullptr;                     // kSortTiles + 1: density block table
     DensPlan dens{};
     float2 *exy = nullptr;                      // field (ex, ey) per bin

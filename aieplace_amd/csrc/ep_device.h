@@ -13,7 +13,6 @@
 namespace ep {
 namespace dev {
 
-constexpr int kSortScanThreads = 1024;
 constexpr int kXcds = 8;  // MI355X: 8 XCDs, each with its own L2
 
 // Workgroups are dispatched to the XCDs round-robin (physical block b runs on
@@ -358,15 +357,12 @@ __device__ inline void wa_net(int s, int e, bool active, int lane, float ginv,
 // against the smoothed one.  Blocks take up to K cells of one super tile and
 // accumulate the window in LDS.
 
-// Exclusive scan of the per-key counts (one block of kSortScanThreads):
-// off[key] = first slot of key, counts cleared, and the density block table
-// dtab[s] = first block of super tile s (level `level`, K cells per block),
-// dtab[NS] = total blocks.
-// Inclusive prefix sum of one int per thread over a kSortScanThreads block:
-// shuffles within each wave, then the wave totals (two block barriers).
+// Inclusive prefix sum of one int per thread over a kBlock block: shuffles
+// within each wave, then the wave totals (one block barrier, and one for the
+// totals of the scan before).
 __device__ inline int block_inclusive_scan(int x)
 {
-    constexpr int kWaves = kSortScanThreads / 64;
+    constexpr int kWaves = kBlock / 64;
     __shared__ int wsum[kWaves];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
@@ -374,65 +370,58 @@ __device__ inline int block_inclusive_scan(int x)
         const int y = __shfl_up(x, d, 64);
         if (lane >= d) x += y;
     }
+    __syncthreads();
     if (lane == 63) wsum[w] = x;
     __syncthreads();
-    if (w == 0) {
-        int t = lane < kWaves ? wsum[lane] : 0;
 #pragma unroll
-        for (int d = 1; d < kWaves; d <<= 1) {
-            const int y = __shfl_up(t, d, 64);
-            if (lane >= d) t += y;
-        }
-        if (lane < kWaves) wsum[lane] = t;
-    }
-    __syncthreads();
-    return w > 0 ? x + wsum[w - 1] : x;
+    for (int k = 0; k < kWaves - 1; ++k)
+        if (k < w) x += wsum[k];
+    return x;
 }
 
-__device__ inline void sort_scan_block(int32_t *__restrict__ count, int32_t *__restrict__ off,
-                                       int32_t *__restrict__ dtab, int level, int K)
+// Tile counts of a thread: four consecutive keys (kBlock threads hold them all).
+constexpr int kTilesPerThread = kSortTiles / kBlock;
+static_assert(kTilesPerThread == 4, "one int4 of tile counts per thread");
+
+// Exclusive scan of the tile counts c (this thread's four): start[key] = first
+// slot of key, start[kSortTiles] = all cells.  Every block of the sort's scatter
+// pass makes it for itself; ends with a barrier.
+__device__ inline void sort_starts(int4 c, int *start)
 {
-    constexpr int per = kSortTiles / kSortScanThreads;
-    __shared__ int so[kSortTiles + 1];
-    const int t = threadIdx.x;
-    int v[per], s = 0;
-#pragma unroll
-    for (int k = 0; k < per; ++k) {
-        v[k] = count[t * per + k];
-        s += v[k];
-    }
+    const int t = threadIdx.x, s = c.x + c.y + c.z + c.w;
     int run = block_inclusive_scan(s) - s;
-#pragma unroll
-    for (int k = 0; k < per; ++k) {
-        off[t * per + k] = run;
-        so[t * per + k] = run;
-        run += v[k];
-        count[t * per + k] = 0;
-    }
-    if (t == kSortScanThreads - 1) so[kSortTiles] = run;
+    start[4 * t] = run;
+    start[4 * t + 1] = run += c.x;
+    start[4 * t + 2] = run += c.y;
+    start[4 * t + 3] = run += c.z;
+    if (t == kBlock - 1) start[kSortTiles] = run + c.w;
     __syncthreads();
-    // blocks per super tile, then the same scan over super tiles
-    const int ns = kSortTiles >> (2 * level);
-    int nb[per], sb = 0;
+}
+
+// What the density scatter needs of a sort, written by one block from its
+// sort_starts: off[key] = end of key's run, and the density block table dtab[s] =
+// first block of super tile s (level `level`, K cells per block), dtab[NS] =
+// total blocks.
+__device__ inline void sort_tables(const int *start, int32_t *__restrict__ off, int32_t *__restrict__ dtab, int level,
+                                   int K)
+{
+    const int t = threadIdx.x, ns = kSortTiles >> (2 * level);
+    int nb[kTilesPerThread], sb = 0;
 #pragma unroll
-    for (int k = 0; k < per; ++k) {
-        const int st = t * per + k;
+    for (int k = 0; k < kTilesPerThread; ++k) {
+        const int st = 4 * t + k;
+        off[st] = start[st + 1];
         nb[k] = 0;
-        if (st < ns) {
-            const int cnt = so[(st + 1) << (2 * level)] - so[st << (2 * level)];
-            nb[k] = (cnt + K - 1) / K;
-        }
+        if (st < ns) nb[k] = (start[(st + 1) << (2 * level)] - start[st << (2 * level)] + K - 1) / K;
         sb += nb[k];
     }
-    __syncthreads();  // the wave totals of the first scan are read before the second reuses them
-    run = block_inclusive_scan(sb) - sb;
+    int run = block_inclusive_scan(sb) - sb;
 #pragma unroll
-    for (int k = 0; k < per; ++k) {
-        const int st = t * per + k;
-        if (st < ns) dtab[st] = run;
+    for (int k = 0; k < kTilesPerThread; ++k) {
+        if (4 * t + k < ns) dtab[4 * t + k] = run;
         run += nb[k];
     }
-    if (t == kSortScanThreads - 1) dtab[ns] = run;
+    if (t == kBlock - 1) dtab[ns] = run;
 }
 
 // Super tile s of density block b (dtab as written by sort_scan_block).
@@ -447,9 +436,8 @@ __device__ inline int dens_super_tile(const int32_t *__restrict__ dtab, int ns, 
     return lo;
 }
 
-// Cells [c0, c1) of the sorted order in block `chunk` of super tile s.  After
-// the sort's scatter pass off[key] holds the END of key's run (clamped to the
-// n sorted cells).
+// Cells [c0, c1) of the sorted order in block `chunk` of super tile s.
+// off[key] is the END of key's run (clamped to the n sorted cells).
 __device__ inline void dens_cell_range(const int32_t *__restrict__ off, int s, int level, int chunk,
                                        int K, int n, int &c0, int &c1)
 {

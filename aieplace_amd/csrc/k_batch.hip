@@ -127,7 +127,7 @@ __global__ __launch_bounds__(kBlock) void kb_move(BDev d, int mode)
     }
     if (count) {
         __syncthreads();
-        int32_t *cnt = d.sort_count + (size_t)i * kSortTiles;
+        int32_t *cnt = d.sort_count + (size_t)i * 2 * kSortTiles;
         for (int t = threadIdx.x; t < kSortTiles; t += kBlock)
             if (hist[t]) atomicAdd(&cnt[t], hist[t]);
     }
@@ -157,34 +157,27 @@ __global__ __launch_bounds__(kBlock) void kb_sort_count(BDev d, int at)
         }
     }
     __syncthreads();
-    int32_t *count = d.sort_count + (size_t)i * kSortTiles;
+    int32_t *count = d.sort_count + (size_t)i * 2 * kSortTiles;
     for (int t = threadIdx.x; t < kSortTiles; t += kBlock)
         if (hist[t]) atomicAdd(&count[t], hist[t]);
 }
 
-// One block per instance: exclusive scan of the tile counts (clears the
-// counts) and the instance's density block table for K cells per block.
-__global__ __launch_bounds__(kSortScanThreads) void kb_sort_scan(BDev d, int K)
-{
-    const int i = blockIdx.x;
-    if (d.st[i].done) return;
-    sort_scan_block(d.sort_count + (size_t)i * kSortTiles, d.sort_off + (size_t)i * kSortTiles,
-                    d.dens_tab + (size_t)i * (kSortTiles + 1), d.inst[i].dens_level, K);
-}
-
+// As k_sort_scatter; the instance's first block leaves its density tables (K cells
+// per density block).
 template <int CPT>
-__global__ __launch_bounds__(kBlock) void kb_sort_scatter(BDev d, int at)
+__global__ __launch_bounds__(kBlock) void kb_sort_scatter(BDev d, int at, int K)
 {
     __shared__ int hist[kSortTiles];
-    __shared__ int base_of[kSortTiles];
+    __shared__ int start[kSortTiles + 1];
     const int i = find_inst(d.pre_sort, d.n_inst, blockIdx.x);
     const BState *S = d.st + i;
     if (S->done) return;
     const BInst &I = d.inst[i];
     const float2 *pos = eval_pos(d, S->cur, at);
     const GeomArgs g = inst_geom(I);
+    int32_t *count = d.sort_count + (size_t)i * 2 * kSortTiles;
+    const int4 cnt = reinterpret_cast<const int4 *>(count)[threadIdx.x];
     for (int t = threadIdx.x; t < kSortTiles; t += kBlock) hist[t] = 0;
-    __syncthreads();
     const int base = (blockIdx.x - d.pre_sort[i]) * kBlock * CPT;
     int key[CPT], rank[CPT];
     float4 cell[CPT];
@@ -197,6 +190,7 @@ __global__ __launch_bounds__(kBlock) void kb_sort_scatter(BDev d, int at)
         p[k] = pos[c];
         s[k] = d.wh[c];
     }
+    sort_starts(cnt, start);
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
         const int idx = base + k * kBlock + threadIdx.x;
@@ -207,16 +201,18 @@ __global__ __launch_bounds__(kBlock) void kb_sort_scatter(BDev d, int at)
             cell[k] = pack_cell(p[k], s[k], idx < I.n_mov);
         }
     }
+    if (base == 0)
+        sort_tables(start, d.sort_off + (size_t)i * kSortTiles, d.dens_tab + (size_t)i * (kSortTiles + 1), I.dens_level,
+                    K);
     __syncthreads();
-    int32_t *off = d.sort_off + (size_t)i * kSortTiles;
     for (int t = threadIdx.x; t < kSortTiles; t += kBlock)
-        if (hist[t]) base_of[t] = atomicAdd(&off[t], hist[t]);
+        if (hist[t]) start[t] += atomicAdd(&count[kSortTiles + t], hist[t]);
     __syncthreads();
     float4 *sorted = d.sorted + I.cell_off;
 #pragma unroll
     for (int k = 0; k < CPT; ++k)
         if (key[k] >= 0) {
-            const int slot = base_of[key[k]] + rank[k];
+            const int slot = start[key[k]] + rank[k];
             if (slot < I.n_place) sorted[slot] = cell[k];  // counts always sum to n_place
         }
 }
@@ -254,6 +250,8 @@ __global__ __launch_bounds__(kBlock) void kb_overflow(BDev d)
     const BInst &I = d.inst[i];
     const int nb = I.M * I.M;
     const int base = (blockIdx.x - d.pre_bin[i]) * kBinsPerBlock;
+    if (base == 0)  // the tile counts and cursors of the next sort
+        for (int t = threadIdx.x; t < 2 * kSortTiles; t += kBlock) d.sort_count[(size_t)i * 2 * kSortTiles + t] = 0;
     constexpr int K = kBinsPerBlock / kBlock;
     double acc[4] = {0.0, 0.0, -1e300, -1e300};
     // All K bins' loads are issued before the first conversion; a bin past
@@ -581,9 +579,9 @@ void bl_sort(const BDev &d, int at, bool counted, int bin_blocks, int sort_block
         with_sort_cpt(d.sort_cpt, [&](auto cpt) {
             hipLaunchKernelGGL(kb_sort_count<decltype(cpt)::value>, dim3(sort_blocks), dim3(kBlock), 0, s, d, at);
         });
-    hipLaunchKernelGGL(kb_sort_scan, dim3(d.n_inst), dim3(kSortScanThreads), 0, s, d, kBlock * dens_cpt);
     with_sort_cpt(d.sort_cpt, [&](auto cpt) {
-        hipLaunchKernelGGL(kb_sort_scatter<decltype(cpt)::value>, dim3(sort_blocks), dim3(kBlock), 0, s, d, at);
+        hipLaunchKernelGGL(kb_sort_scatter<decltype(cpt)::value>, dim3(sort_blocks), dim3(kBlock), 0, s, d, at,
+                           kBlock * dens_cpt);
     });
 }
 

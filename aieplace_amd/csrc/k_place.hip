@@ -71,34 +71,27 @@ __global__ __launch_bounds__(kBlock) void k_sort_count(Pair<const float2> pos_pa
         if (hist[t]) atomicAdd(&count[t], hist[t]);
 }
 
-// Exclusive scan of the tile counts into offsets (clears the counts) and the
-// density block table of the coming scatter.
-__global__ __launch_bounds__(kSortScanThreads) void k_sort_scan(int32_t *__restrict__ count,
-                                                                int32_t *__restrict__ off,
-                                                                int32_t *__restrict__ dtab,
-                                                                int level, int K,
-                                                                const DevScalars *__restrict__ sc)
-{
-    if (sc->halt) return;
-    sort_scan_block(count, off, dtab, level, K);
-}
-
 // Writes every cell, packed with its size and movable flag (pack_cell), to its
-// slot of the tile-sorted order.
+// slot of the tile-sorted order.  `count` holds the tile counts and, behind
+// them, the tiles' cursors (cells placed so far, zero at the start; the overflow
+// pass clears both).  Every block scans the 1024 counts for itself, beside its
+// cell loads: a kernel for the scan took 4.5 us of every evaluation.  Block 0
+// leaves the tables of the coming density scatter.
 template <int CPT>
 __global__ __launch_bounds__(kBlock) void k_sort_scatter(Pair<const float2> pos_pair,
                                                          const float2 *__restrict__ wh, int n_place,
                                                          int n_mov, GeomArgs g, int Mx, int My,
-                                                         int32_t *__restrict__ off,
-                                                         float4 *__restrict__ sorted,
+                                                         int32_t *__restrict__ count,
+                                                         int32_t *__restrict__ off, int32_t *__restrict__ dtab,
+                                                         int level, int K, float4 *__restrict__ sorted,
                                                          const DevScalars *__restrict__ sc)
 {
     if (sc->halt) return;
     const float2 *__restrict__ pos = pos_pair.p[sc->sel];
     __shared__ int hist[kSortTiles];
-    __shared__ int base_of[kSortTiles];
+    __shared__ int start[kSortTiles + 1];
+    const int4 cnt = reinterpret_cast<const int4 *>(count)[threadIdx.x];
     for (int t = threadIdx.x; t < kSortTiles; t += kBlock) hist[t] = 0;
-    __syncthreads();
     const int base = blockIdx.x * kBlock * CPT;
     int key[CPT], rank[CPT];
     float4 cell[CPT];
@@ -111,6 +104,7 @@ __global__ __launch_bounds__(kBlock) void k_sort_scatter(Pair<const float2> pos_
         p[k] = pos[idx];
         s[k] = wh[idx];
     }
+    sort_starts(cnt, start);
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
         const int idx = base + k * kBlock + threadIdx.x;
@@ -121,16 +115,23 @@ __global__ __launch_bounds__(kBlock) void k_sort_scatter(Pair<const float2> pos_
             cell[k] = pack_cell(p[k], s[k], idx < n_mov);
         }
     }
+    if (blockIdx.x == 0) sort_tables(start, off, dtab, level, K);
     __syncthreads();
     for (int t = threadIdx.x; t < kSortTiles; t += kBlock)
-        if (hist[t]) base_of[t] = atomicAdd(&off[t], hist[t]);
+        if (hist[t]) start[t] += atomicAdd(&count[kSortTiles + t], hist[t]);
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < CPT; ++k)
         if (key[k] >= 0) {
-            const int slot = base_of[key[k]] + rank[k];
+            const int slot = start[key[k]] + rank[k];
             if (slot < n_place) sorted[slot] = cell[k];  // counts always sum to n_place
         }
+}
+
+// Clears the tile counts and cursors (repeated sorts without an overflow pass).
+__global__ void k_sort_clear(int32_t *__restrict__ count)
+{
+    for (int t = threadIdx.x; t < 2 * kSortTiles; t += blockDim.x) count[t] = 0;
 }
 
 // ---- density scatter: block b takes up to kBlock * CPT cells of one super
@@ -168,10 +169,12 @@ __global__ __launch_bounds__(kBlock) void k_overflow(unsigned long long *__restr
                                                      float rho_t, float cap, int nb,
                                                      float *__restrict__ map_field,
                                                      float *__restrict__ map_mov,
-                                                     double *__restrict__ part,
+                                                     double *__restrict__ part, int32_t *__restrict__ count,
                                                      const DevScalars *__restrict__ sc)
 {
     if (sc->halt) return;
+    const int t0 = blockIdx.x * kBlock + threadIdx.x;  // the next sort's counts and cursors
+    for (int t = t0; t < 2 * kSortTiles; t += gridDim.x * kBlock) count[t] = 0;
     // The loads of kOvfRun grid-stride bins are issued together, then the
     // bins are converted in the same order as one bin per pass would.  A bin
     // past the map loads the last bin instead (in bounds, value unused).
@@ -929,6 +932,11 @@ void launch_fill_maps(Ctx &c, hipStream_t s)
                        c.acc_field, c.acc_mov, nb, c.d_scal);
 }
 
+void launch_sort_clear(Ctx &c, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_sort_clear, dim3(1), dim3(kBlock), 0, s, c.sort_count);
+}
+
 void launch_sort(Ctx &c, Pair<const float2> pos, bool counted, hipStream_t s)
 {
     with_sort_cpt(c.sort_cpt, [&](auto cpt) {
@@ -936,13 +944,9 @@ void launch_sort(Ctx &c, Pair<const float2> pos, bool counted, hipStream_t s)
         if (!counted)
             hipLaunchKernelGGL(k_sort_count<CPT>, dim3(c.trial_blocks), dim3(kBlock), 0, s, pos, c.wh, c.n_place,
                                geom_args(c), c.Mx, c.My, c.sort_count, c.d_scal);
-    });
-    hipLaunchKernelGGL(k_sort_scan, dim3(1), dim3(kSortScanThreads), 0, s, c.sort_count, c.sort_off,
-                       c.dens_tab, c.dens.level, kBlock * c.dens.cpt, c.d_scal);
-    with_sort_cpt(c.sort_cpt, [&](auto cpt) {
-        constexpr int CPT = decltype(cpt)::value;
         hipLaunchKernelGGL(k_sort_scatter<CPT>, dim3(c.trial_blocks), dim3(kBlock), 0, s, pos, c.wh, c.n_place,
-                           c.n_mov, geom_args(c), c.Mx, c.My, c.sort_off, c.sorted, c.d_scal);
+                           c.n_mov, geom_args(c), c.Mx, c.My, c.sort_count, c.sort_off, c.dens_tab, c.dens.level,
+                           kBlock * c.dens.cpt, c.sorted, c.d_scal);
     });
 }
 
@@ -969,7 +973,7 @@ void launch_overflow(Ctx &c, hipStream_t s)
     const double unit = (double)c.bw * (double)c.bh / kDensFixUnits;
     hipLaunchKernelGGL(k_overflow, dim3(c.ovf_blocks), dim3(kBlock), 0, s, c.acc_field, c.acc_mov,
                        c.map_fix, unit, c.prm.target_density, cap, nb, c.map_field, c.map_mov,
-                       c.part + c.part_ovf_off, c.d_scal);
+                       c.part + c.part_ovf_off, c.sort_count, c.d_scal);
 }
 
 void launch_map_range(Ctx &c, hipStream_t s)
