@@ -36,6 +36,12 @@ constexpr int kBlock = 256;
 // Blocks of the final reduction (k_finalize); the context's fin buffer holds
 // ten partial sums per block.
 constexpr int kFinalizeBlocks = 32;
+// Up to this many partial sums one block reduces them alone: no ticket, fences
+// and second level, which cost 2.7 us; beyond it the loads of one block cost more.
+// One block / 32 blocks, us per evaluation of a run: 576 cells 48.3 / 50.5, 20k 63.9 /
+// 67.2, 200k (9k sums) 92.9 / 95.5, 500k (25k) 145.2 / 145.9, 1M (50k) 185.1 / 183.2, 2M
+// (95k) 294.0 / 289.6.
+constexpr int kFinalizeOneBlock = 32768;
 // Launch caps of the reducing kernels (bounds the partial sums to finalize).
 constexpr int kWaGridCap = 16384;
 constexpr int kCellGridCap = 16384;

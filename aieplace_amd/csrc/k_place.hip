@@ -473,15 +473,15 @@ __global__ __launch_bounds__(kBlock) void k_pin_sum(const int32_t *__restrict__ 
         gw_cell[c] = sum_pin_partials(cell_pin_start[c], cell_pin_start[c + 1], cell_pins, pin_grad);
 }
 
-// Deterministic final reduction of all partial sums: block b of
-// kFinalizeBlocks sums slice b of every partial array in a fixed order and
-// writes its ten values to fin[b]; the last block to finish (atomic ticket)
-// sums fin[0..B) in block order, so the result does not depend on timing.
-constexpr int kFinalizeThreads = 256;
-static_assert(kFinalizeBlocks <= kFinalizeThreads, "one loading thread per block result");
+// Deterministic final reduction of all partial sums, in a fixed order.  kBlocks =
+// 1: one block of 1024 threads sums everything.  Else block b of kBlocks sums
+// slice b of every partial array and writes its ten values to fin[b]; the last
+// block to finish (atomic ticket) sums fin[0..B) in block order, so the result
+// does not depend on timing.
 constexpr int kCtlWords = (int)(sizeof(DevCtl) / 4);
-constexpr int kMlpWordsPerThread = (EP_MLP_NWEIGHTS + kFinalizeThreads - 1) / kFinalizeThreads;
-static_assert(sizeof(DevCtl) % 4 == 0 && kCtlWords <= kFinalizeThreads, "one word of the control state per thread");
+constexpr int finalize_threads(int blocks) { return blocks == 1 ? 1024 : 256; }
+static_assert(kFinalizeBlocks <= 256, "one loading thread per block result");
+static_assert(sizeof(DevCtl) % 4 == 0 && kCtlWords <= 256, "one word of the control state per thread");
 
 struct StepCtlArgs {
     DevCtl *ctl;            // null: no step decision (host-controlled launches)
@@ -491,33 +491,56 @@ struct StepCtlArgs {
     const float *mlp_w;     // learned step: the model proposes the next trial's step
 };
 
-// What the decision leaves for the next trial's model proposal, kept by the
-// deciding thread as it writes the same values to the scalars (so that it
-// need not read them back): the model flag, the halt flag and the features.
-struct NextTrial {
-    int use_model;
-    int halt;
-    float *feat;  // 16 floats, written when the decision starts an iteration
+// Partial sums of the reducing kernels, as offsets into one array.
+struct FinalizeArgs {
+    const double *part;
+    int wa_off, wa_blocks, ovf_off, ovf_blocks, cell_off, cell_blocks, trial_off, trial_blocks;
+    double mov_area;
 };
 
-__device__ inline void step_decide(DevCtl *__restrict__ ctl, const DevCtl &S0, const DevResult &R,
-                                   DevScalars *__restrict__ sc, const CtlParams &p,
-                                   ep_step_info *__restrict__ log, float *__restrict__ rec, NextTrial &nt);
+// What the decision leaves for the rest of its block.
+struct NextTrial {
+    int begin;      // an iteration begins: its features are to be made
+    int use_model;  // the next trial's model flag
+    int halt;       // the run is finished
+};
 
-__global__ __launch_bounds__(kFinalizeThreads) void k_finalize(
-    const double *__restrict__ part, int wa_off, int wa_blocks, int ovf_off, int ovf_blocks,
-    int cell_off, int cell_blocks, int trial_off, int trial_blocks, double mov_area, DevScalars *__restrict__ sc,
-    DevResult *__restrict__ res, double *__restrict__ fin, unsigned *__restrict__ ticket,
-    StepCtlArgs ctl)
+__device__ inline void step_decide(DevCtl &S, const DevResult &R, DevScalars *__restrict__ sc, const CtlParams &p,
+                                   ep_step_info *__restrict__ log, float *__restrict__ rec, NextTrial &nt);
+__device__ inline float ctl_feature(int k, const DevCtl &S, double bw, double isn);
+
+// acc[w] += base[i * stride + w] for i = first, first + step, ... < n, four
+// entries in flight at once, added in that order.
+template <int W, int STRIDE>
+__device__ inline void sum_entries(const double *__restrict__ base, int first, int step, int n, double *acc)
 {
-    if (sc->halt) return;
-    const int B = gridDim.x, b = blockIdx.x;
+    for (int i = first; i < n; i += 4 * step) {
+        double q[4][W];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int w = 0; w < W; ++w) q[u][w] = i + u * step < n ? base[(size_t)(i + u * step) * STRIDE + w] : 0.0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int w = 0; w < W; ++w) acc[w] += q[u][w];
+    }
+}
+
+template <int kBlocks>
+__global__ __launch_bounds__(finalize_threads(kBlocks)) void k_finalize(FinalizeArgs f, DevScalars *__restrict__ sc,
+                                                                        DevResult *__restrict__ res,
+                                                                        double *__restrict__ fin,
+                                                                        unsigned *__restrict__ ticket, StepCtlArgs ctl)
+{
+    constexpr int NT = finalize_threads(kBlocks);
+    const int b = blockIdx.x;
+    // The halt flag is tested after the sums, so that its load overlaps theirs.
     // Device-controlled runs: the control state and the trial's step are
     // loaded now, beside the partial sums, so that the decision at the end of
     // the last block does not wait for them (the previous launch wrote them).
+    const int halt = sc->halt;
     __shared__ DevCtl ctl_s;
-    __shared__ float alpha_s;
-    __shared__ int use_model_s;
     uint32_t ctl_w = 0;
     const bool ctl_load = ctl.ctl && threadIdx.x < kCtlWords;
     if (ctl_load) ctl_w = reinterpret_cast<const uint32_t *>(ctl.ctl)[threadIdx.x];
@@ -525,100 +548,105 @@ __global__ __launch_bounds__(kFinalizeThreads) void k_finalize(
     const int use_model0 = sc->use_model;
     // The step model's weights likewise (learned runs): registers now, LDS
     // after the partial sums, read by the proposal at the end.
+    constexpr int kMlpWords = (EP_MLP_NWEIGHTS + NT - 1) / NT;
     __shared__ float mlp_s[EP_MLP_NWEIGHTS];
-    float mlp_r[kMlpWordsPerThread];
+    float mlp_r[kMlpWords];
     if (ctl.mlp_w)
 #pragma unroll
-        for (int k = 0; k < kMlpWordsPerThread; ++k) {
-            const int i = threadIdx.x + k * kFinalizeThreads;
+        for (int k = 0; k < kMlpWords; ++k) {
+            const int i = threadIdx.x + k * NT;
             mlp_r[k] = i < EP_MLP_NWEIGHTS ? ctl.mlp_w[i] : 0.0f;
         }
-    auto slice = [&](int n, int &lo, int &hi) {
-        lo = (int)((int64_t)n * b / B);
-        hi = (int)((int64_t)n * (b + 1) / B);
-    };
+    auto lo = [&](int n) { return (int)((int64_t)n * b / kBlocks); };
+    auto hi = [&](int n) { return (int)((int64_t)n * (b + 1) / kBlocks); };
+    const int t = threadIdx.x;
     double v[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    int lo, hi;
-    slice(wa_blocks, lo, hi);
-    for (int i = lo + threadIdx.x; i < hi; i += kFinalizeThreads) {
-        v[0] += part[wa_off + 2 * i];
-        v[1] += part[wa_off + 2 * i + 1];
-    }
-    slice(ovf_blocks, lo, hi);
-    for (int i = lo + threadIdx.x; i < hi; i += kFinalizeThreads) v[2] += part[ovf_off + 4 * i];
-    slice(cell_blocks, lo, hi);
-    for (int i = lo + threadIdx.x; i < hi; i += kFinalizeThreads) {
-        const double *q = part + cell_off + 7 * i;
+    for (int i = lo(f.cell_blocks) + t; i < hi(f.cell_blocks); i += NT) {
+        const double *q = f.part + f.cell_off + 7 * (size_t)i;
         v[3] += q[0]; v[4] += q[1]; v[5] += q[2]; v[6] += q[3]; v[7] += q[4]; v[8] += q[5];
         v[9] = fmax(v[9], q[6]);
     }
-    slice(trial_blocks, lo, hi);  // |v' - v|^2 of a trial (k_cell_grad's sum is then 0)
-    for (int i = lo + threadIdx.x; i < hi; i += kFinalizeThreads) v[3] += part[trial_off + i];
+    // |v' - v|^2 of a trial (k_cell_grad's sum is then 0)
+    sum_entries<1, 1>(f.part + f.trial_off, lo(f.trial_blocks) + t, NT, hi(f.trial_blocks), v + 3);
+    sum_entries<1, 4>(f.part + f.ovf_off, lo(f.ovf_blocks) + t, NT, hi(f.ovf_blocks), v + 2);
+    sum_entries<2, 2>(f.part + f.wa_off, lo(f.wa_blocks) + t, NT, hi(f.wa_blocks), v);
     __shared__ double out[10];
-    __shared__ int last;
     if (ctl_load) reinterpret_cast<uint32_t *>(&ctl_s)[threadIdx.x] = ctl_w;
-    if (threadIdx.x == 0) {
-        alpha_s = alpha_used;
-        use_model_s = use_model0;
-    }
     if (ctl.mlp_w)
 #pragma unroll
-        for (int k = 0; k < kMlpWordsPerThread; ++k) {
-            const int i = threadIdx.x + k * kFinalizeThreads;
+        for (int k = 0; k < kMlpWords; ++k) {
+            const int i = threadIdx.x + k * NT;
             if (i < EP_MLP_NWEIGHTS) mlp_s[i] = mlp_r[k];
         }
-    block_reduce<10, 1, kFinalizeThreads>(v, out);  // its barriers also publish ctl_s, alpha_s, mlp_s
-    if (threadIdx.x == 0) {
-        for (int k = 0; k < 10; ++k) fin[b * 10 + k] = out[k];
-        __threadfence();
-        last = atomicAdd(ticket, 1u) == (unsigned)(B - 1);
-    }
-    __syncthreads();
-    if (!last) return;
-    __threadfence();
-    __shared__ double sfin[kFinalizeBlocks][10];  // every block's sums, loaded in parallel
-    if (threadIdx.x < B)
-        for (int k = 0; k < 10; ++k) sfin[threadIdx.x][k] = load_agent(&fin[threadIdx.x * 10 + k]);
-    __syncthreads();
-    // thread k sums column k over the blocks in block order (ten short chains
-    // instead of one long one; the same order, so the same sums)
+    if (halt) return;
+    block_reduce<10, 1, NT>(v, out);  // its barriers also publish ctl_s and mlp_s
     __shared__ double tot[10];
-    if (threadIdx.x < 10) {
-        const int k = threadIdx.x;
-        double t = sfin[0][k];
-        for (int j = 1; j < B; ++j) t = k < 9 ? t + sfin[j][k] : fmax(t, sfin[j][k]);
-        tot[k] = t;
+    if constexpr (kBlocks > 1) {
+        __shared__ int last;
+        if (threadIdx.x == 0) {
+            for (int k = 0; k < 10; ++k) fin[b * 10 + k] = out[k];
+            __threadfence();
+            last = atomicAdd(ticket, 1u) == (unsigned)(kBlocks - 1);
+        }
+        __syncthreads();
+        if (!last) return;
+        __threadfence();
+        __shared__ double sfin[kBlocks][10];  // every block's sums, loaded in parallel
+        if (threadIdx.x < kBlocks)
+            for (int k = 0; k < 10; ++k) sfin[threadIdx.x][k] = load_agent(&fin[threadIdx.x * 10 + k]);
+        __syncthreads();
+        // thread k sums column k over the blocks in block order (ten short chains
+        // instead of one long one; the same order, so the same sums)
+        if (threadIdx.x < 10) {
+            const int k = threadIdx.x;
+            double x = sfin[0][k];
+            for (int j = 1; j < kBlocks; ++j) x = k < 9 ? x + sfin[j][k] : fmax(x, sfin[j][k]);
+            tot[k] = x;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // next launch
     }
-    __syncthreads();
-    __shared__ int propose;
-    __shared__ float feat[16];  // the decision thread's features, for the whole block
+    const double *T = kBlocks > 1 ? tot : out;
+    __shared__ int propose, begin;
+    __shared__ float feat[16];  // the coming iteration's features, for the whole block
     if (threadIdx.x == 0) {
-        double t[10];
-        for (int k = 0; k < 10; ++k) t[k] = tot[k];
-        __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // next launch
         DevResult R;
-        R.hpwl = t[0];
-        R.wa = t[1];
-        R.ovf_num = t[2];
-        R.tau = mov_area > 0 ? t[2] / mov_area : 0.0;
-        R.dv2 = t[3];
-        R.dg2 = t[4];
-        R.sum_gw = t[5];
-        R.sum_f = t[6];
-        R.gnorm2 = t[7];
-        R.nonfinite = (int64_t)t[8];
-        R.gmax = t[9];
-        R.alpha_used = alpha_s;
+        R.hpwl = T[0];
+        R.wa = T[1];
+        R.ovf_num = T[2];
+        R.tau = f.mov_area > 0 ? T[2] / f.mov_area : 0.0;
+        R.dv2 = T[3];
+        R.dg2 = T[4];
+        R.sum_gw = T[5];
+        R.sum_f = T[6];
+        R.gnorm2 = T[7];
+        R.nonfinite = (int64_t)T[8];
+        R.gmax = T[9];
+        R.alpha_used = alpha_used;
         *res = R;
-        if (ctl.ctl) {  // device-controlled run: the decision also fills feat
-            NextTrial nt{use_model_s, 0, feat};
-            step_decide(ctl.ctl, ctl_s, R, sc, ctl.p, ctl.log, ctl.rec, nt);
+        begin = 0;
+        if (ctl.ctl) {
+            NextTrial nt{0, use_model0, 0};
+            step_decide(ctl_s, R, sc, ctl.p, ctl.log, ctl.rec, nt);
+            begin = nt.begin;
             propose = ctl.mlp_w && nt.use_model && !nt.halt;
         } else {
-            propose = ctl.mlp_w && sc->use_model && !sc->halt;
+            propose = ctl.mlp_w && use_model0;
             if (propose)
                 for (int k = 0; k < 16; ++k) feat[k] = sc->feat[k];
         }
+    }
+    if (ctl.ctl) {
+        __syncthreads();
+        if (begin && threadIdx.x < 16) {  // ten logarithms side by side instead of in turn
+            const float x = ctl_feature(threadIdx.x, ctl_s, ctl.p.bw, ctl.p.inv_sqrt_np);
+            feat[threadIdx.x] = x;
+            sc->feat[threadIdx.x] = x;
+        }
+        __syncthreads();
+        if (begin && threadIdx.x < 16) ctl_s.feat[threadIdx.x] = feat[threadIdx.x];
+        __syncthreads();
+        if (ctl_load) reinterpret_cast<uint32_t *>(ctl.ctl)[threadIdx.x] = reinterpret_cast<uint32_t *>(&ctl_s)[threadIdx.x];
     }
     // the model's step for the next trial, while this block is still resident
     if (ctl.mlp_w) {
@@ -728,40 +756,40 @@ __global__ void k_cell_bins(const float2 *__restrict__ pos, const float2 *__rest
 
 __device__ inline float lg10_clamped(double v) { return (float)sched_log10(fmax(v, 1e-30)); }
 
-// Step-model features of the coming iteration (order and definitions:
+// Step-model feature k of the coming iteration (order and definitions:
 // include/eplace_mlp.h); the host's step_features computes the same values.
-__device__ inline void ctl_features(const DevCtl &S, double bw, double isn, float *f)
+__device__ inline float ctl_feature(int k, const DevCtl &S, double bw, double isn)
 {
 #pragma clang fp contract(off)
-    f[0] = lg10_clamped(S.alpha / bw);
-    f[1] = lg10_clamped(S.h_alpha1 / bw);
-    f[2] = lg10_clamped(S.h_alpha2 / bw);
-    f[3] = (float)S.last_tau;
-    f[4] = (float)(S.last_tau - S.h_prev_tau);
-    f[5] = lg10_clamped(S.lambda / S.lambda0);
-    f[6] = lg10_clamped(S.gamma / bw);
-    f[7] = (float)((S.last_hpwl - S.h_prev_hpwl) / fmax(S.last_hpwl, 1e-30));
-    f[8] = lg10_clamped(S.h_gnorm * isn);
-    f[9] = lg10_clamped(S.h_dv * isn / bw);
-    f[10] = lg10_clamped(S.h_dg * isn);
-    f[11] = (float)S.coef;
-    f[12] = (float)S.h_evals;
-    f[13] = lg10_clamped(S.lambda / S.h_sum_ratio);
-    f[14] = lg10_clamped(S.h_ratio);
-    f[15] = (float)(S.iteration / 1000.0);
+    double x = 0.0;  // the logarithm's argument
+    switch (k) {
+    case 0: x = S.alpha / bw; break;
+    case 1: x = S.h_alpha1 / bw; break;
+    case 2: x = S.h_alpha2 / bw; break;
+    case 3: return (float)S.last_tau;
+    case 4: return (float)(S.last_tau - S.h_prev_tau);
+    case 5: x = S.lambda / S.lambda0; break;
+    case 6: x = S.gamma / bw; break;
+    case 7: return (float)((S.last_hpwl - S.h_prev_hpwl) / fmax(S.last_hpwl, 1e-30));
+    case 8: x = S.h_gnorm * isn; break;
+    case 9: x = S.h_dv * isn / bw; break;
+    case 10: x = S.h_dg * isn; break;
+    case 11: return (float)S.coef;
+    case 12: return (float)S.h_evals;
+    case 13: x = S.lambda / S.h_sum_ratio; break;
+    case 14: x = S.h_ratio; break;
+    default: return (float)(S.iteration / 1000.0);
+    }
+    return lg10_clamped(x);
 }
 
-// Nesterov coefficient, features and the scalars of the iteration's first trial
-// (nt, when given, gets the model flag and the features too).
-__device__ inline void ctl_begin(DevCtl &S, DevScalars *sc, const CtlParams &p, NextTrial *nt = nullptr)
+// Nesterov coefficient and the scalars of the iteration's first trial; the
+// features are the caller's (ctl_feature).
+__device__ inline void ctl_begin(DevCtl &S, DevScalars *sc, const CtlParams &p, NextTrial &nt)
 {
 #pragma clang fp contract(off)
     S.ak1 = 0.5 * (1.0 + sqrt(4.0 * S.ak * S.ak + 1.0));
     S.coef = (S.ak - 1.0) / S.ak1;
-    ctl_features(S, p.bw, p.inv_sqrt_np, S.feat);
-    for (int k = 0; k < 16; ++k) sc->feat[k] = S.feat[k];
-    if (nt)
-        for (int k = 0; k < 16; ++k) nt->feat[k] = S.feat[k];
     S.trials = 0;
     S.t = 0;
     S.learned_ok = 0;
@@ -775,17 +803,17 @@ __device__ inline void ctl_begin(DevCtl &S, DevScalars *sc, const CtlParams &p, 
     sc->gamma_inv = (float)(1.0 / S.gamma);
     sc->lambda = (float)S.lambda;
     sc->use_model = propose ? 1 : 0;
-    if (nt) nt->use_model = propose ? 1 : 0;
+    nt.begin = 1;
+    nt.use_model = propose ? 1 : 0;
 }
 
-// The decision after a trial whose reductions are R (one thread); S0 is the
-// control state *ctl as the trial left it, the result goes back to *ctl.
-__device__ inline void step_decide(DevCtl *__restrict__ ctl, const DevCtl &S0, const DevResult &R,
-                                   DevScalars *__restrict__ sc, const CtlParams &p,
+// The decision after a trial whose reductions are R (one thread); C is the
+// control state as the trial left it and takes the result.
+__device__ inline void step_decide(DevCtl &C, const DevResult &R, DevScalars *__restrict__ sc, const CtlParams &p,
                                    ep_step_info *__restrict__ log, float *__restrict__ rec, NextTrial &nt)
 {
 #pragma clang fp contract(off)
-    DevCtl S = S0;
+    DevCtl S = C;  // in registers
     if (S.done) {  // (the halt flag was set with it)
         nt.halt = 1;
         return;
@@ -797,7 +825,7 @@ __device__ inline void step_decide(DevCtl *__restrict__ ctl, const DevCtl &S0, c
         S.done = 1;
         sc->halt = 1;
         nt.halt = 1;
-        *ctl = S;
+        C = S;
         return;
     }
     const double used = R.alpha_used;
@@ -878,10 +906,10 @@ __device__ inline void step_decide(DevCtl *__restrict__ ctl, const DevCtl &S0, c
             sc->halt = 1;
             nt.halt = 1;
         } else {
-            ctl_begin(S, sc, p, &nt);
+            ctl_begin(S, sc, p, nt);
         }
     }
-    *ctl = S;
+    C = S;
 }
 
 // Start of the first iteration of a device-controlled run (and the model's
@@ -889,20 +917,21 @@ __device__ inline void step_decide(DevCtl *__restrict__ ctl, const DevCtl &S0, c
 __global__ void k_step_begin(DevCtl *__restrict__ ctl, DevScalars *__restrict__ sc, CtlParams p,
                              const float *__restrict__ mlp_w)
 {
-    __shared__ int propose;
+    __shared__ DevCtl S;
+    __shared__ NextTrial nt;
     __shared__ float feat[16];
     if (threadIdx.x == 0) {
-        DevCtl S = *ctl;
-        propose = 0;
-        if (!S.done) {
-            ctl_begin(S, sc, p);
-            *ctl = S;
-            propose = mlp_w && sc->use_model && !sc->halt;
-            for (int k = 0; k < 16; ++k) feat[k] = sc->feat[k];
-        }
+        S = *ctl;
+        nt = NextTrial{0, 0, 0};
+        if (!S.done) ctl_begin(S, sc, p, nt);
     }
     __syncthreads();
-    if (mlp_w) mlp_propose_block(mlp_w, feat, sc, propose != 0);
+    if (nt.begin && threadIdx.x < 16) feat[threadIdx.x] = ctl_feature(threadIdx.x, S, p.bw, p.inv_sqrt_np);
+    __syncthreads();
+    if (nt.begin && threadIdx.x < 16) sc->feat[threadIdx.x] = S.feat[threadIdx.x] = feat[threadIdx.x];
+    __syncthreads();
+    if (nt.begin && threadIdx.x == 0) *ctl = S;
+    if (mlp_w) mlp_propose_block(mlp_w, feat, sc, nt.begin && nt.use_model);
 }
 
 GeomArgs geom_args(const Ctx &c)
@@ -1019,22 +1048,29 @@ void launch_cell_grad(Ctx &c, Pair<const float2> pos, Pair<const float2> vref,
     }
 }
 
+namespace {
+void launch_finalize_args(Ctx &c, int trial_blocks, const StepCtlArgs &a, hipStream_t s)
+{
+    const FinalizeArgs f{c.part, c.part_wa_off, c.wa_part_blocks, c.part_ovf_off, c.ovf_blocks, c.part_cell_off,
+                         c.cell_blocks, c.part_trial_off, trial_blocks, c.mov_area};
+    if (c.part_total <= kFinalizeOneBlock)
+        hipLaunchKernelGGL(k_finalize<1>, dim3(1), dim3(finalize_threads(1)), 0, s, f, c.d_scal, c.d_res, c.fin,
+                           c.fin_ticket, a);
+    else
+        hipLaunchKernelGGL(k_finalize<kFinalizeBlocks>, dim3(kFinalizeBlocks), dim3(finalize_threads(kFinalizeBlocks)),
+                           0, s, f, c.d_scal, c.d_res, c.fin, c.fin_ticket, a);
+}
+}  // namespace
+
 void launch_finalize(Ctx &c, hipStream_t s, bool trial)
 {
-    StepCtlArgs none{};
-    hipLaunchKernelGGL(k_finalize, dim3(kFinalizeBlocks), dim3(kFinalizeThreads), 0, s, c.part,
-                       c.part_wa_off, c.wa_part_blocks, c.part_ovf_off, c.ovf_blocks, c.part_cell_off,
-                       c.cell_blocks, c.part_trial_off, trial ? c.trial_blocks : 0, c.mov_area, c.d_scal,
-                       c.d_res, c.fin, c.fin_ticket, none);
+    launch_finalize_args(c, trial ? c.trial_blocks : 0, StepCtlArgs{}, s);
 }
 
 void launch_finalize_decide(Ctx &c, const CtlParams &p, hipStream_t s)
 {
-    const StepCtlArgs a{c.d_ctl, c.d_log, c.d_rec, p, p.learned ? (const float *)c.d_mlp_w : nullptr};
-    hipLaunchKernelGGL(k_finalize, dim3(kFinalizeBlocks), dim3(kFinalizeThreads), 0, s, c.part,
-                       c.part_wa_off, c.wa_part_blocks, c.part_ovf_off, c.ovf_blocks, c.part_cell_off,
-                       c.cell_blocks, c.part_trial_off, c.trial_blocks, c.mov_area, c.d_scal, c.d_res, c.fin,
-                       c.fin_ticket, a);
+    launch_finalize_args(c, c.trial_blocks,
+                         StepCtlArgs{c.d_ctl, c.d_log, c.d_rec, p, p.learned ? (const float *)c.d_mlp_w : nullptr}, s);
 }
 
 void launch_trial(Ctx &c, Pair<const float2> v, Pair<const float2> u, Pair<const float2> g,

@@ -37,3 +37,21 @@ def test_counted_and_uncounted_sort_agree(n):
     # 2^-24 relative per coordinate of up to 128 bins
     assert abs(mov.sum(dtype=np.float64) - area) <= 2.0 ** -15 * area
     assert tau == r["overflow"]
+
+
+@pytest.mark.parametrize("n", [100, 5_000, 500_000, 800_000])
+def test_totals_on_both_sides_of_the_one_block_reduction(n):
+    """HPWL (a sum over every WA block's partial) against the net spans of the FP32
+    pin positions in numpy."""
+    print(f"case totals n={n}", flush=True)
+    nl = A.generate("stdcell", seed=2, n_movable=n)
+    p = A.placer_params(A.CONFIGS["stdcell_200k"], bins_x=512, bins_y=512)
+    with A.Placer(nl, p) as pl:
+        x, y = pl.get_positions()
+        hpwl = pl.hpwl()
+    span = 0.0
+    for pos, fixed, off in ((x, nl.x, nl.pin_dx), (y, nl.y, nl.pin_dy)):
+        at = np.where(nl.pin_cell < n, pos[np.minimum(nl.pin_cell, n - 1)], fixed[nl.pin_cell]) + off
+        s = nl.net_start[:-1]
+        span += (np.maximum.reduceat(at, s) - np.minimum.reduceat(at, s)).sum(dtype=np.float64)
+    assert hpwl == pytest.approx(span, rel=1e-9)
