@@ -25,7 +25,7 @@ namespace {
 
 constexpr int kTrialsPerLaunch = 4;   // Nesterov trials captured per graph replay
 constexpr int kCellAlign = 64;        // instance cell ranges start on this boundary
-constexpr int kDensCpt[3] = {2, 4, 8};
+constexpr int kDensCpt[3] = {1, 2, 4};
 constexpr int kTuneReps = 5;
 
 #define EPB_HIP(call)                                                                        \

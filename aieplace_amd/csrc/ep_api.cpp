@@ -619,7 +619,8 @@ extern "C" ep_status ep_create(const ep_netlist *nl, const ep_params *p, ep_ctx 
     c->buckets = L.buckets;
     c->wa_blocks = L.wa_blocks;
     c->wa_part_blocks = std::min(L.wa_blocks, kWaGridCap);
-    c->dens = make_dens_plan(L.Mx, L.My, L.bw, L.bh, L.max_sw, L.max_sh, 4);
+    c->dens = make_dens_plan(L.Mx, L.My, L.bw, L.bh, L.max_sw, L.max_sh,
+                            sort_cells_per_thread(L.n_place, kDensMost, kDensBlocks));
 
     // ---- device buffers
     hipError_t he = hipStreamCreate(&c->stream);
@@ -1542,7 +1543,7 @@ extern "C" ep_status ep_profile(ep_ctx *c, int32_t reps, ep_kernel_stat *out, in
     // the density scatter at the other tile sizes (cells per thread), each after
     // a sort whose block table matches it: the plan's choice is one of them
     const int cpt0 = c->dens.cpt;
-    for (int cpt : {2, 4, 8, 16}) {
+    for (int cpt : {1, 2, 4}) {
         if (cpt == cpt0) continue;
         c->dens.cpt = cpt;
         launch_sort_clear(*c, c->stream);

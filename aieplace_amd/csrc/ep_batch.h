@@ -127,7 +127,6 @@ void bl_cell_grad(const BDev &d, int at, int cell_blocks, hipStream_t s);
 // The per-instance FP64 reductions of an evaluation, then the control step
 // `mode` (BCtlMode) of every unfinished instance on them.
 void bl_reduce_control(const BDev &d, int mode, hipStream_t s);
-bool bl_density_cpt_supported(int cpt);
 
 // ---- batched field solve (k_field.hip)
 struct BatchFieldInst {

@@ -102,6 +102,13 @@ struct DensPlan {
     int32_t level = 0, ext = 0, wcap = 0, cpt = 4;
 };
 
+// Cells per thread of the scatter (sort_cells_per_thread): the latency of a block's
+// cells, one after the other, against one flush of the window's bins per block.
+// Whole placements at 1 / 2 / 4 / 8 cells per thread, us per evaluation: 20k cells 55.4 /
+// 57.3 / 61.3 / 68.2, 75k 63.0 / 64.2 / 67.6 / 74.9, 200k 84.0 / 83.3 / 87.5 / 93.6, 500k
+// 150 / 141 / 136 / 137, 2M 293 / 275 / 270 / 272.  Blocks of 512 or 1024 threads gain
+// nothing below and lose 5-15% from 500k on.
+constexpr int kDensMost = 4, kDensBlocks = 480;
 constexpr int kDensMaxWin = 6400;  // LDS bins per map of the largest window
 // Fixed-point density units per bin area (the maps accumulate in uint64).
 constexpr double kDensFixUnits = 4294967296.0;  // 2^32
@@ -114,18 +121,22 @@ inline DensPlan make_dens_plan(int Mx, int My, double bw, double bh, double max_
                                int cpt)
 {
     DensPlan p;
-    const int m = Mx < My ? Mx : My;
-    p.level = 6;
-    for (int k = 0; k <= 6; ++k)
-        if (((int64_t)m << k) / kSortSide >= 32) {
-            p.level = k;
-            break;
-        }
     const int ex = (int)(max_w / bw) + 2, ey = (int)(max_h / bh) + 2;
     p.ext = ex > ey ? ex : ey;
-    const int64_t sx = (((int64_t)Mx << p.level) + kSortSide - 1) / kSortSide + 2 + p.ext;
-    const int64_t sy = (((int64_t)My << p.level) + kSortSide - 1) / kSortSide + 2 + p.ext;
-    const int64_t w = sx * sy;
+    auto window = [&](int level) {
+        const int64_t sx = (((int64_t)Mx << level) + kSortSide - 1) / kSortSide + 2 + p.ext;
+        const int64_t sy = (((int64_t)My << level) + kSortSide - 1) / kSortSide + 2 + p.ext;
+        return sx * sy;
+    };
+    // The smallest super tile of 600 bins (32 x 32 on the 512^2 and 1024^2 grids), made
+    // smaller where its window would not fit the LDS: then every overlap is a global
+    // atomic.  Bins per super tile, measured alone with spread cells: 400^2 grid 25 x 25 9.3
+    // us, 50 x 50 13.3; 640 x 320 20 x 40 10.5 us, 40 x 80 18.1; 768^2 24 x 24 20.5 us, 48 x 48
+    // 17.9; 240 x 400 30 x 50 7.5 us, 60 x 100 (no LDS window) 50, and with clustered
+    // cells 10 against 1510.
+    while (p.level < 5 && (((int64_t)Mx * My) << (2 * p.level)) < (int64_t)600 * kSortTiles) ++p.level;
+    while (p.level > 0 && window(p.level) > kDensMaxWin) --p.level;
+    const int64_t w = window(p.level);
     p.wcap = (int)(w < kDensMaxWin ? w : kDensMaxWin);
     p.cpt = cpt;
     return p;

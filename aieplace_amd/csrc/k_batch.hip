@@ -563,8 +563,6 @@ __global__ __launch_bounds__(kBlock) void kb_reduce_control(BDev d, int mode)
 
 // ------------------------------------------------------------------ launchers
 
-bool bl_density_cpt_supported(int cpt) { return cpt == 2 || cpt == 4 || cpt == 8; }
-
 void bl_move(const BDev &d, int mode, int sort_blocks, hipStream_t s)
 {
     with_sort_cpt(d.sort_cpt, [&](auto cpt) {
@@ -588,10 +586,10 @@ void bl_sort(const BDev &d, int at, bool counted, int bin_blocks, int sort_block
 void bl_dens(const BDev &d, int bin_blocks, int dens_blocks, int dens_cpt, bool map_range, hipStream_t s)
 {
     const size_t lds = 2 * sizeof(unsigned long long) * (size_t)d.dens_wcap;
-    if (dens_cpt == 2)
+    if (dens_cpt == 1)
+        hipLaunchKernelGGL(kb_density<1>, dim3(dens_blocks), dim3(kBlock), lds, s, d);
+    else if (dens_cpt == 2)
         hipLaunchKernelGGL(kb_density<2>, dim3(dens_blocks), dim3(kBlock), lds, s, d);
-    else if (dens_cpt == 8)
-        hipLaunchKernelGGL(kb_density<8>, dim3(dens_blocks), dim3(kBlock), lds, s, d);
     else
         hipLaunchKernelGGL(kb_density<4>, dim3(dens_blocks), dim3(kBlock), lds, s, d);
     hipLaunchKernelGGL(kb_overflow, dim3(bin_blocks), dim3(kBlock), 0, s, d);

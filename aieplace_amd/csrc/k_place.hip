@@ -989,9 +989,8 @@ void launch_density(Ctx &c, hipStream_t s)
                            dp.level, dp.ext, dp.wcap, c.n_place, geom_args(c), c.Mx, c.My,
                            c.acc_field, c.acc_mov, c.d_scal);
     };
-    if (dp.cpt == 2) go(k_density<2>);
-    else if (dp.cpt == 8) go(k_density<8>);
-    else if (dp.cpt == 16) go(k_density<16>);
+    if (dp.cpt == 1) go(k_density<1>);
+    else if (dp.cpt == 2) go(k_density<2>);
     else go(k_density<4>);
 }
 

@@ -55,3 +55,32 @@ def test_totals_on_both_sides_of_the_one_block_reduction(n):
         s = nl.net_start[:-1]
         span += (np.maximum.reduceat(at, s) - np.minimum.reduceat(at, s)).sum(dtype=np.float64)
     assert hpwl == pytest.approx(span, rel=1e-9)
+
+
+# one super tile, several, a window cut to fit the LDS, none that fits
+@pytest.mark.parametrize("mx,my,n", [(16, 16, 500), (48, 32, 2_000), (240, 400, 20_000), (640, 320, 90_000),
+                                     (1024, 16, 30_000), (16, 2048, 3_000)])
+def test_density_windows_match_oracle(oracle, mx, my, n):
+    """Clustered and spread cells on grids with different density windows."""
+    from support import oracle_design
+    print(f"case density windows {mx} x {my}, {n} cells", flush=True)
+    nl = A.generate("stdcell", seed=2, n_movable=n)
+    p = A.placer_params(A.CONFIGS["stdcell_200k"], bins_x=mx, bins_y=my)
+    d, x0, y0 = oracle_design(oracle, nl, p)
+    xl, yl, xh, yh = nl.die
+    rng = np.random.default_rng(n)
+    spread = [(xl + rng.random(len(x0)) * (xh - xl)).astype(np.float32),
+              (yl + rng.random(len(x0)) * (yh - yl)).astype(np.float32)]
+    with A.Placer(nl, p) as pl:
+        for x, y in ((x0, y0), spread):
+            pl.set_positions(x, y)
+            x, y = pl.get_positions()
+            field, mov, _, _ = pl.computeOverlaps()
+            omov = d.density(x.astype(np.float64), y.astype(np.float64), "exact", 0, d.n_mov)
+            # every cell's edges round to 2^-24 of the grid side (in bins); a bin sums its cells' errors
+            tol = 2.0 ** -22 * max(mx, my) * (xh - xl) / mx * (yh - yl) / my
+            count = np.abs(omov).max() / ((xh - xl) / mx * (yh - yl) / my) + 4
+            assert np.abs(mov - omov).max() <= tol * count * max(1.0, mx / my, my / mx)
+            ofield = d.density(x.astype(np.float64), y.astype(np.float64), "stretched", 0, d.n_mov + d.n_fill)
+            ofield += float(np.float32(p.target_density)) * d.density_fixed()
+            assert abs(field.sum(dtype=np.float64) / ofield.sum() - 1) <= 1e-4
