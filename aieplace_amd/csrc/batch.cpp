@@ -18,6 +18,7 @@
 #include "../../include/eplace_batch.h"
 #include "ep_batch.h"
 #include "ep_layout.h"
+#include "ep_stage.h"
 
 using namespace ep;
 
@@ -68,8 +69,10 @@ struct ep_batch {
     int n = 0;
     std::vector<BInst> inst;
     std::vector<int32_t> n_fix;
-    std::vector<std::vector<int32_t>> cell_order;  // per instance: stored movable cell -> caller's index
-    std::vector<float2> init_pos;   // all cells, concatenated
+    float2 *init_pos = nullptr;     // all cells, concatenated
+    int32_t *stored = nullptr;      // [total_cells] per instance: caller's movable cell -> stored index
+    Stage stage;                    // pinned slots of the host transfers
+    bool st_current = false;        // h_st is what the device holds
     int64_t total_cells = 0;
 
     BInst *d_inst = nullptr;
@@ -212,10 +215,11 @@ static void destroy_batch(ep_batch *b)
                     b->pin_grad, b->map_field, b->map_mov, b->map_fix, b->acc_field, b->acc_mov, b->exy, b->tA, b->tB,
                     b->map_mean, b->map_max, b->sorted, b->sort_count, b->sort_off, b->dens_tab, b->pre_cell,
                     b->pre_sort, b->pre_bin, b->pre_wa, b->pre_dens[0], b->pre_dens[1],
-                    b->pre_dens[2], b->buckets, b->part_wa, b->part_ovf, b->part_cell};
+                    b->pre_dens[2], b->buckets, b->part_wa, b->part_ovf, b->part_cell, b->init_pos, b->stored};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     batch_field_free(b->bf);
+    stage_free(b->stage);
     if (b->h_st) (void)hipHostFree(b->h_st);
     for (int k = 0; k < 2; ++k) {
         if (b->h_rb[k]) (void)hipHostFree(b->h_rb[k]);
@@ -281,16 +285,11 @@ static ep_status reset_state(ep_batch *b)
         ep_status st = set_tables(b, std::vector<char>(b->n, 1));
         if (st != EP_OK) return st;
     }
-    const size_t nc = (size_t)b->total_cells;
-    for (int k = 0; k < 2; ++k) {
-        EPB_HIP(hipMemcpy(b->V[k], b->init_pos.data(), nc * sizeof(float2), hipMemcpyHostToDevice));
-        EPB_HIP(hipMemcpy(b->U[k], b->init_pos.data(), nc * sizeof(float2), hipMemcpyHostToDevice));
-        EPB_HIP(hipMemset(b->G[k], 0, nc * sizeof(float2)));
-    }
-    std::vector<BState> st(b->n);
-    std::memset(st.data(), 0, st.size() * sizeof(BState));
-    EPB_HIP(hipMemcpy(b->d_st, st.data(), st.size() * sizeof(BState), hipMemcpyHostToDevice));
-    std::memcpy(b->h_st, st.data(), st.size() * sizeof(BState));
+    bl_reset(b->dev(), b->init_pos, b->total_cells, b->stream);
+    EPB_HIP(hipGetLastError());
+    EPB_HIP(hipStreamSynchronize(b->stream));
+    std::memset(b->h_st, 0, sizeof(BState) * b->n);
+    b->st_current = true;
     b->ready = false;
     return EP_OK;
 }
@@ -306,8 +305,10 @@ static ep_status check_errors(ep_batch *b)
 
 static ep_status pull_state(ep_batch *b)
 {
+    if (b->st_current) return EP_OK;
     EPB_HIP(hipMemcpyAsync(b->h_st, b->d_st, sizeof(BState) * b->n, hipMemcpyDeviceToHost, b->stream));
     EPB_HIP(hipStreamSynchronize(b->stream));
+    b->st_current = true;
     return EP_OK;
 }
 
@@ -369,6 +370,7 @@ extern "C" ep_status ep_batch_create(const ep_netlist *const *nls, const int32_t
 
     // ---- concatenated host arrays
     std::vector<float2> wh, pos;
+    std::vector<int32_t> stored;  // per instance: caller's movable cell -> stored index
     std::vector<int32_t> net_start{0}, pin_cell, cps, cpins;
     std::vector<float2> pin_off;
     std::vector<float> fixmap;
@@ -409,7 +411,8 @@ extern "C" ep_status ep_batch_create(const ep_netlist *const *nls, const int32_t
         b->dens_wcap = std::max(b->dens_wcap, dp.wcap);
         b->inst.push_back(I);
         b->n_fix.push_back(L.n_fix);
-        b->cell_order.push_back(L.cell_order);
+        stored.resize(cell_off + L.n_mov);
+        for (int k = 0; k < L.n_mov; ++k) stored[cell_off + caller_cell(L.cell_order, k)] = k;
         means.push_back(field_map_mean(L, p->target_density));
         const int64_t span = (L.n_all + kCellAlign - 1) / kCellAlign * kCellAlign;
         if (cell_off + span > INT32_MAX || map_off + (int64_t)bins[i] * bins[i] > INT32_MAX / 2 ||
@@ -473,7 +476,6 @@ extern "C" ep_status ep_batch_create(const ep_netlist *const *nls, const int32_t
         pre_sort.push_back(pre_sort.back() + b->nb_sort.back());
     }
     b->active.assign(n, 1);
-    b->init_pos = pos;
     b->n_buckets = (int)bks.size();
     b->cell_blocks = pre_cell.back();
     b->sort_blocks = pre_sort.back();
@@ -514,6 +516,9 @@ extern "C" ep_status ep_batch_create(const ep_netlist *const *nls, const int32_t
         EPB_TRY(dalloc(&b->U[k], nc));
         EPB_TRY(dalloc(&b->G[k], nc));
     }
+    EPB_TRY(dalloc(&b->init_pos, nc));
+    stored.resize(nc);
+    EPB_TRY(dalloc(&b->stored, nc));
     EPB_TRY(dalloc(&b->net_start, net_start.size()));
     EPB_TRY(dalloc(&b->pin_cell, pin_cell.size()));
     EPB_TRY(dalloc(&b->pin_off, pin_off.size()));
@@ -558,6 +563,13 @@ extern "C" ep_status ep_batch_create(const ep_netlist *const *nls, const int32_t
     EPB_TRY(upload(b->d_inst, b->inst));
     EPB_TRY(upload(b->map_mean, means));
     EPB_TRY(upload(b->wh, wh));
+    EPB_TRY(upload(b->init_pos, pos));
+    EPB_TRY(upload(b->stored, stored));
+    {
+        int most = 0;
+        for (const BInst &I : b->inst) most = std::max(most, I.n_place);
+        EPB_TRY(stage_init(b->stage, b->stream, sizeof(float2) * (size_t)most));
+    }
     EPB_TRY(upload(b->net_start, net_start));
     EPB_TRY(upload(b->pin_cell, pin_cell));
     EPB_TRY(upload(b->pin_off, pin_off));
@@ -629,6 +641,7 @@ extern "C" ep_status ep_batch_init(ep_batch *b)
     if (b->ready) return EP_OK;
     const BDev d = b->dev();
     hipStream_t s = b->stream;
+    b->st_current = false;
     bl_move(d, kMoveInitU, b->sort_blocks, s);
     bl_maps(d, kAtCur, false, b->bin_blocks, b->sort_blocks, b->dens_blocks[b->dens_variant],
             kDensCpt[b->dens_variant], b->f16(), s);
@@ -712,6 +725,7 @@ extern "C" ep_status ep_batch_run(ep_batch *b, int32_t max_launches, ep_batch_ru
     for (;;) {
         const bool launch = launches < max_launches && !all_done();
         if (launch) {
+            b->st_current = false;
             EPB_HIP(hipGraphLaunch(b->exec, b->stream));
             EPB_HIP(hipMemcpyAsync(b->h_rb[slot], b->d_st, st_bytes, hipMemcpyDeviceToHost, b->stream));
             EPB_HIP(hipEventRecord(b->rb_done[slot], b->stream));
@@ -740,7 +754,10 @@ extern "C" ep_status ep_batch_run(ep_batch *b, int32_t max_launches, ep_batch_ru
         slot ^= 1;
     }
     EPB_HIP(hipStreamSynchronize(b->stream));
-    if (last >= 0) std::memcpy(b->h_st, b->h_rb[last], st_bytes);  // the last replay's state
+    if (last >= 0) {  // the last replay's state
+        std::memcpy(b->h_st, b->h_rb[last], st_bytes);
+        b->st_current = true;
+    }
     if ((st = check_errors(b)) != EP_OK) return st;
     const auto t1 = std::chrono::steady_clock::now();
     if (info) {
@@ -793,14 +810,10 @@ static ep_status pull_pairs(ep_batch *b, int32_t i, bool grad, float *x, float *
     const BInst &I = b->inst[i];
     const int cur = b->h_st[i].cur;
     const float2 *src = (grad ? b->G[cur] : b->V[cur]) + I.cell_off;
-    std::vector<float2> h(I.n_place);
-    EPB_HIP(hipMemcpy(h.data(), src, sizeof(float2) * I.n_place, hipMemcpyDeviceToHost));
-    for (int k = 0; k < I.n_place; ++k) {
-        const int32_t o = caller_cell(b->cell_order[i], k);
-        x[o] = h[k].x;
-        y[o] = h[k].y;
-    }
-    return EP_OK;
+    StageOut out(b->stage);
+    st = out.pairs(src, b->stored + I.cell_off, I.n_mov, I.n_place, x, y);
+    const ep_status fin = out.finish();
+    return st != EP_OK ? st : fin;
 }
 
 extern "C" ep_status ep_batch_positions(ep_batch *b, int32_t i, float *x, float *y)

@@ -270,10 +270,11 @@ static void destroy_ctx(ep_ctx *c)
                     c->map_field, c->map_mov, c->map_fix, c->acc_field, c->acc_mov, c->exy, c->tA, c->tB, c->part,
                     c->sorted, c->sort_count, c->sort_off, c->dens_tab,
                     c->d_scal, c->d_res, c->d_mlp_w, c->d_ctl, c->d_log, c->d_rec, c->fin,
-                    c->fin_ticket, c->gw_cell};
+                    c->fin_ticket, c->gw_cell, c->d_order, c->d_stored};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     field_free(*c);
+    stage_free(c->stage);
     if (c->h_scal) (void)hipHostFree(c->h_scal);
     if (c->h_res) (void)hipHostFree(c->h_res);
     if (c->h_ctl) (void)hipHostFree(c->h_ctl);
@@ -715,6 +716,16 @@ extern "C" ep_status ep_create(const ep_netlist *nl, const ep_params *p, ep_ctx 
         destroy_ctx(c);
         return fail(EP_EDEVICE, "ep_create: hipMemset failed");
     }
+    // a slot holds the cells' coordinates or the field, whichever is larger, or a chunk of it
+    EP_TRY(stage_init(c->stage, c->stream, sizeof(float2) * std::max<size_t>(nb, c->n_place)));
+    if (!L.cell_order.empty()) {
+        std::vector<int32_t> stored(L.cell_order.size());
+        for (size_t k = 0; k < stored.size(); ++k) stored[L.cell_order[k]] = (int32_t)k;
+        EP_TRY(dalloc(&c->d_order, L.cell_order.size()));
+        EP_TRY(dalloc(&c->d_stored, stored.size()));
+        EP_TRY(upload(c->d_order, L.cell_order.data(), L.cell_order.size()));
+        EP_TRY(upload(c->d_stored, stored.data(), stored.size()));
+    }
     EP_TRY(field_init(*c));
     {
         const float mean = field_map_mean(L, p->target_density);
@@ -792,32 +803,41 @@ extern "C" ep_status ep_get_nets(ep_ctx *c, int32_t *net_start, int32_t *pin_cel
 extern "C" ep_status ep_set_positions(ep_ctx *c, const float *x, const float *y)
 {
     if (!c || !x || !y) return fail(EP_EINVAL, "ep_set_positions: null argument");
-    std::vector<float2> p(std::max(1, c->n_place)), wh(std::max(1, c->n_place));
-    EP_HIP(hipMemcpy(wh.data(), c->wh, sizeof(float2) * c->n_place, hipMemcpyDeviceToHost));
-    for (int k = 0; k < c->n_place; ++k) {
-        const int32_t o = caller_cell(c->cell_order, k);
-        if (!std::isfinite(x[o]) || !std::isfinite(y[o]))
-            return fail(EP_ENAN, "ep_set_positions: non-finite position at cell %d", o);
-        p[k] = make_float2(std::min(std::max(x[o], c->xl), c->xh - wh[k].x),
-                           std::min(std::max(y[o], c->yl), c->yh - wh[k].y));
-    }
-    EP_HIP(hipMemcpy(c->V[c->cur], p.data(), sizeof(float2) * c->n_place, hipMemcpyHostToDevice));
-    EP_HIP(hipMemcpy(c->U[c->cur], p.data(), sizeof(float2) * c->n_place, hipMemcpyHostToDevice));
+    // the buffers of the other parity hold a past trial: they take the positions
+    // and become the current ones once these are known to be finite
+    const int b = c->cur ^ 1;
+    float *sx = reinterpret_cast<float *>(c->G[b]), *sy = sx + c->n_place;
+    *c->stage.flag = 0;
+    ep_status st = stage_in(c->stage, sx, x, c->n_place);
+    if (st == EP_OK) st = stage_in(c->stage, sy, y, c->n_place);
+    if (st != EP_OK) return st;
+    launch_place_cells(sx, sy, c->d_order, c->n_mov, c->wh, c->n_place, make_float4(c->xl, c->yl, c->xh, c->yh),
+                       c->V[b], c->U[b], c->stage.flag, c->stream);
+    if ((st = check_launch()) != EP_OK || (st = sync(*c)) != EP_OK) return st;
+    if (*c->stage.flag)
+        for (int k = 0; k < c->n_place; ++k) {
+            const int32_t o = caller_cell(c->cell_order, k);
+            if (!std::isfinite(x[o]) || !std::isfinite(y[o]))
+                return fail(EP_ENAN, "ep_set_positions: non-finite position at cell %d", o);
+        }
+    c->cur = b;
     c->opt_ready = false;
     return EP_OK;
+}
+
+// Per-cell pairs of cells [mov | fill] in the caller's order.
+static ep_status cell_pairs(StageOut &out, const ep_ctx *c, const float2 *d, float *ox, float *oy)
+{
+    return out.pairs(d, c->d_stored, c->n_mov, c->n_place, ox, oy);
 }
 
 extern "C" ep_status ep_get_positions(ep_ctx *c, float *x, float *y)
 {
     if (!c || !x || !y) return fail(EP_EINVAL, "ep_get_positions: null argument");
-    std::vector<float2> p(std::max(1, c->n_place));
-    EP_HIP(hipMemcpy(p.data(), c->V[c->cur], sizeof(float2) * c->n_place, hipMemcpyDeviceToHost));
-    for (int k = 0; k < c->n_place; ++k) {
-        const int32_t o = caller_cell(c->cell_order, k);
-        x[o] = p[k].x;
-        y[o] = p[k].y;
-    }
-    return EP_OK;
+    StageOut out(c->stage);
+    ep_status st = cell_pairs(out, c, c->V[c->cur], x, y);
+    const ep_status fin = out.finish();
+    return st != EP_OK ? st : fin;
 }
 
 static ep_status run_density(ep_ctx *c)
@@ -844,11 +864,13 @@ extern "C" ep_status ep_density(ep_ctx *c, double *overflow)
 extern "C" ep_status ep_get_density(ep_ctx *c, float *field_map, float *mov_map, float *fix_map)
 {
     if (!c) return fail(EP_EINVAL, "ep_get_density: null context");
-    const size_t nb = (size_t)c->Mx * c->My;
-    if (field_map) EP_HIP(hipMemcpy(field_map, c->map_field, nb * sizeof(float), hipMemcpyDeviceToHost));
-    if (mov_map) EP_HIP(hipMemcpy(mov_map, c->map_mov, nb * sizeof(float), hipMemcpyDeviceToHost));
-    if (fix_map) EP_HIP(hipMemcpy(fix_map, c->map_fix, nb * sizeof(float), hipMemcpyDeviceToHost));
-    return EP_OK;
+    const int64_t nb = (int64_t)c->Mx * c->My;
+    StageOut out(c->stage);
+    ep_status st = out.flat(c->map_field, nb, field_map);
+    if (st == EP_OK) st = out.flat(c->map_mov, nb, mov_map);
+    if (st == EP_OK) st = out.flat(c->map_fix, nb, fix_map);
+    const ep_status fin = out.finish();
+    return st != EP_OK ? st : fin;
 }
 
 extern "C" ep_status ep_field(ep_ctx *c, int32_t precision)
@@ -875,29 +897,10 @@ extern "C" ep_status ep_field_error(ep_ctx *c, int32_t precision, double *err_ex
 extern "C" ep_status ep_get_field(ep_ctx *c, float *ex, float *ey)
 {
     if (!c) return fail(EP_EINVAL, "ep_get_field: null context");
-    const size_t nb = (size_t)c->Mx * c->My;
-    if (!ex && !ey) return EP_OK;
-    std::vector<float2> e(nb);
-    EP_HIP(hipMemcpy(e.data(), c->exy, nb * sizeof(float2), hipMemcpyDeviceToHost));
-    for (size_t b = 0; b < nb; ++b) {
-        if (ex) ex[b] = e[b].x;
-        if (ey) ey[b] = e[b].y;
-    }
-    return EP_OK;
-}
-
-// Per-cell pairs of cells [mov | fill] back to the caller, in the caller's order.
-static ep_status copy_pairs(const ep_ctx *c, const float2 *d, int n, float *ox, float *oy)
-{
-    if (!ox && !oy) return EP_OK;
-    std::vector<float2> h(std::max(1, n));
-    EP_HIP(hipMemcpy(h.data(), d, sizeof(float2) * n, hipMemcpyDeviceToHost));
-    for (int k = 0; k < n; ++k) {
-        const int32_t o = caller_cell(c->cell_order, k);
-        if (ox) ox[o] = h[k].x;
-        if (oy) oy[o] = h[k].y;
-    }
-    return EP_OK;
+    StageOut out(c->stage);
+    ep_status st = out.pairs(c->exy, nullptr, 0, (int64_t)c->Mx * c->My, ex, ey);
+    const ep_status fin = out.finish();
+    return st != EP_OK ? st : fin;
 }
 
 extern "C" ep_status ep_wa_grad(ep_ctx *c, float gamma, double *wa, double *hpwl)
@@ -920,18 +923,18 @@ extern "C" ep_status ep_wa_grad(ep_ctx *c, float gamma, double *wa, double *hpwl
 extern "C" ep_status ep_get_wa_grad(ep_ctx *c, float *gx, float *gy)
 {
     if (!c) return fail(EP_EINVAL, "ep_get_wa_grad: null context");
-    float2 *gw = nullptr;
-    ep_status st = dalloc(&gw, std::max(1, c->n_place));
-    if (st != EP_OK) return st;
     c->h_scal->lambda = 0.0f;
     push_scalars(*c, c->stream);
-    float2 *scratch = c->G[c->cur ^ 1];
+    // the other parity's buffers hold a past trial
+    float2 *scratch = c->G[c->cur ^ 1], *gw = c->U[c->cur ^ 1];
     launch_cell_grad(*c, c->V[c->cur], nullptr, nullptr, scratch, gw, nullptr, c->stream);
-    st = check_launch();
-    if (st == EP_OK) st = sync(*c);
-    if (st == EP_OK) st = copy_pairs(c, gw, c->n_place, gx, gy);
-    (void)hipFree(gw);
-    return st;
+    ep_status st = check_launch();
+    if (st != EP_OK) return st;
+    StageOut out(c->stage);
+    st = cell_pairs(out, c, gw, gx, gy);
+    const ep_status fin = out.finish();
+    if (st != EP_OK || fin != EP_OK) return st != EP_OK ? st : fin;
+    return sync(*c);
 }
 
 extern "C" ep_status ep_gradient(ep_ctx *c, float gamma, float lambda, float *gx, float *gy,
@@ -940,28 +943,24 @@ extern "C" ep_status ep_gradient(ep_ctx *c, float gamma, float lambda, float *gx
 {
     if (!c) return fail(EP_EINVAL, "ep_gradient: null context");
     if (!(gamma > 0.f)) return fail(EP_EINVAL, "ep_gradient: gamma must be > 0");
-    float2 *gw = nullptr, *f = nullptr;
-    ep_status st = dalloc(&gw, std::max(1, c->n_place));
-    if (st == EP_OK) st = dalloc(&f, std::max(1, c->n_place));
-    if (st != EP_OK) {
-        if (gw) (void)hipFree(gw);
-        return st;
-    }
+    c->opt_ready = false;  // G[cur] gets caller-chosen gamma/lambda
     c->h_scal->gamma_inv = 1.0f / gamma;
     c->h_scal->lambda = lambda;
     push_scalars(*c, c->stream);
+    // the other parity's buffers (a past trial) take the components
+    float2 *gw = c->U[c->cur ^ 1], *f = c->V[c->cur ^ 1];
     enqueue_eval(*c, c->V[c->cur], nullptr, nullptr, c->G[c->cur], gw, f, c->stream);
-    st = check_launch();
-    if (st == EP_OK) st = sync(*c);
-    if (st == EP_OK) st = copy_pairs(c, c->G[c->cur], c->n_place, gx, gy);
-    if (st == EP_OK) st = copy_pairs(c, gw, c->n_place, gwx, gwy);
-    if (st == EP_OK) st = copy_pairs(c, f, c->n_place, fx, fy);
-    (void)hipFree(gw);
-    (void)hipFree(f);
+    ep_status st = check_launch();
     if (st != EP_OK) return st;
+    StageOut out(c->stage);
+    st = cell_pairs(out, c, c->G[c->cur], gx, gy);
+    if (st == EP_OK) st = cell_pairs(out, c, gw, gwx, gwy);
+    if (st == EP_OK) st = cell_pairs(out, c, f, fx, fy);
+    const ep_status fin = out.finish();
+    if (st != EP_OK || fin != EP_OK) return st != EP_OK ? st : fin;
+    if ((st = sync(*c)) != EP_OK) return st;
     if (hpwl) *hpwl = c->h_res->hpwl;
     if (overflow) *overflow = c->h_res->tau;
-    c->opt_ready = false;  // G[cur] was overwritten with caller-chosen gamma/lambda
     return EP_OK;
 }
 

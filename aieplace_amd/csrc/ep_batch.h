@@ -112,6 +112,8 @@ enum BMoveMode { kMoveTrial = 0, kMoveProbe = 1, kMoveInitU = 2 };
 // Blocks of kBlock * sort_cpt cells (the sort's layout); kMoveTrial
 // also counts the trial positions into the sort tiles.
 void bl_move(const BDev &d, int mode, int sort_blocks, hipStream_t s);
+// Every instance at the positions `pos` (all cells), gradients and states cleared.
+void bl_reset(const BDev &d, const float2 *pos, int64_t cells, hipStream_t s);
 // Density maps of every unfinished instance; `counted`: a kMoveTrial move made
 // the sort counts at the evaluated positions.
 // bl_maps = bl_sort (tile sort) then bl_dens (scatter; overflow, which also

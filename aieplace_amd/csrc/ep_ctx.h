@@ -29,6 +29,7 @@
 #include <vector>
 
 #include "ep_common.h"
+#include "ep_stage.h"
 
 namespace ep {
 
@@ -324,6 +325,8 @@ struct Ctx {
     int32_t wa_blocks = 0;
     std::vector<int32_t> net_perm;  // stored net k -> original net index
     std::vector<int32_t> cell_order;  // stored movable cell k -> caller's index (empty: same order)
+    int32_t *d_order = nullptr, *d_stored = nullptr;  // the same on the device, and its inverse (null: same order)
+    Stage stage;                      // pinned slots of the host transfers
 
     // optimiser state
     float2 *V[2] = {nullptr, nullptr}, *U[2] = {nullptr, nullptr}, *G[2] = {nullptr, nullptr};

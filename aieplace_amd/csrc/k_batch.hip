@@ -8,6 +8,7 @@
 // indexed by the global block id and reduced per instance in a fixed order.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cfloat>
 #include <climits>
 
@@ -130,6 +131,21 @@ __global__ __launch_bounds__(kBlock) void kb_move(BDev d, int mode)
         int32_t *cnt = d.sort_count + (size_t)i * 2 * kSortTiles;
         for (int t = threadIdx.x; t < kSortTiles; t += kBlock)
             if (hist[t]) atomicAdd(&cnt[t], hist[t]);
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void kb_reset(BDev d, const float2 *__restrict__ pos, int64_t cells)
+{
+    const int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    const int64_t words = (int64_t)(sizeof(BState) / 4) * d.n_inst;
+    if (c < words) reinterpret_cast<uint32_t *>(d.st)[c] = 0u;
+    if (c >= cells) return;
+    const float2 p = pos[c], z = make_float2(0.f, 0.f);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        d.V[k][c] = p;
+        d.U[k][c] = p;
+        d.G[k][c] = z;
     }
 }
 
@@ -562,6 +578,12 @@ __global__ __launch_bounds__(kBlock) void kb_reduce_control(BDev d, int mode)
 }  // namespace
 
 // ------------------------------------------------------------------ launchers
+
+void bl_reset(const BDev &d, const float2 *pos, int64_t cells, hipStream_t s)
+{
+    const int64_t n = std::max<int64_t>(cells, (int64_t)(sizeof(BState) / 4) * d.n_inst);
+    hipLaunchKernelGGL(kb_reset, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, d, pos, cells);
+}
 
 void bl_move(const BDev &d, int mode, int sort_blocks, hipStream_t s)
 {

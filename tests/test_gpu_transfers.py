@@ -1,0 +1,81 @@
+"""Host transfers through the pinned slots: sizes around a slot's (131072 cells),
+both cell orders, refused positions."""
+import numpy as np
+import pytest
+
+import aieplace_amd as A
+from aieplace_amd import api
+from aieplace_amd.batch import BatchPlacer
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("order", [0, 1])
+@pytest.mark.parametrize("n", [100, 1_000, 131_071, 131_072, 131_073, 300_000])
+def test_positions_round_trip(n, order):
+    print(f"case round trip n={n} order={order}", flush=True)
+    nl = A.generate("stdcell", seed=3, n_movable=n)
+    p = A.placer_params(A.CONFIGS["stdcell_200k"], bins_x=64, bins_y=64, use_fillers=0, cell_order=order)
+    xl, yl, xh, yh = nl.die
+    rng = np.random.default_rng(n)
+    with A.Placer(nl, p) as pl:
+        assert pl.n_place == n
+        x = (xl + rng.random(n) * (xh - xl - nl.w[:n])).astype(np.float32)
+        y = (yl + rng.random(n) * (yh - yl - nl.h[:n])).astype(np.float32)
+        x = np.minimum(np.maximum(x, np.float32(xl)), np.float32(xh) - nl.w[:n])
+        y = np.minimum(np.maximum(y, np.float32(yl)), np.float32(yh) - nl.h[:n])
+        pl.set_positions(x, y)
+        gx, gy = pl.get_positions()
+        assert np.array_equal(gx, x) and np.array_equal(gy, y)
+        # clamped into the die
+        pl.set_positions(np.full(n, xl - 5.0), np.full(n, yh + 5.0))
+        gx, gy = pl.get_positions()
+        assert np.array_equal(gx, np.full(n, xl, np.float32)) and np.array_equal(gy, np.float32(yh) - nl.h[:n])
+        # a refused call leaves the positions alone
+        for bad in (np.nan, np.inf):
+            z = x.copy()
+            z[n // 2] = bad
+            with pytest.raises(api.EplaceError, match=f"non-finite position at cell {n // 2}$") as e:
+                pl.set_positions(z, y)
+            assert e.value.code == api.EP_ENAN
+        hx, hy = pl.get_positions()
+        assert np.array_equal(hx, gx) and np.array_equal(hy, gy)
+
+
+@pytest.mark.parametrize("mx,my", [(16, 16), (512, 256), (528, 512), (1024, 1024)])
+def test_maps_and_field_come_whole(mx, my):
+    """Each output alone equals the same output taken with the others."""
+    print(f"case maps {mx} x {my}", flush=True)
+    nl = A.generate("stdcell", seed=3, n_movable=5_000)
+    p = A.placer_params(A.CONFIGS["stdcell_200k"], bins_x=mx, bins_y=my)
+    with A.Placer(nl, p) as pl:
+        maps = pl.computeOverlaps()[:3]
+        fields = pl.computeElectricFields()
+        for k in range(3):
+            one = np.full((mx, my), -1.0, np.float32)
+            api.check(api.lib.ep_get_density(pl._ctx, *[api.fptr(one) if j == k else None for j in range(3)]))
+            assert np.array_equal(one, maps[k])
+        for k in range(2):
+            one = np.full((mx, my), -1.0, np.float32)
+            api.check(api.lib.ep_get_field(pl._ctx, *[api.fptr(one) if j == k else None for j in range(2)]))
+            assert np.array_equal(one, fields[k])
+
+
+@pytest.mark.parametrize("order", [0, 1])
+def test_batch_positions_after_reset(order):
+    print(f"case batch reset order={order}", flush=True)
+    nls = [A.generate("stdcell", seed=k + 1, n_movable=n) for k, n in enumerate((300, 140_000))]
+    p = A.placer_params(A.CONFIGS["stdcell_200k"], max_iters=3, cell_order=order, use_fillers=0)
+    with BatchPlacer(nls, [64, 256], p) as bp:
+        start = [bp.positions(i) for i in range(2)]
+        bp.run()
+        moved = [bp.positions(i) for i in range(2)]
+        bp.reset()
+        again = [bp.positions(i) for i in range(2)]
+    for nl, s, m, a in zip(nls, start, moved, again):
+        n = nl.n_mov
+        xl, yl, xh, yh = (np.float32(v) for v in nl.die)
+        want = (np.minimum(np.maximum(nl.x[:n], xl), xh - nl.w[:n]), np.minimum(np.maximum(nl.y[:n], yl), yh - nl.h[:n]))
+        for k in range(2):
+            assert np.array_equal(s[k], want[k]) and np.array_equal(a[k], want[k])
+            assert not np.array_equal(m[k], want[k])
