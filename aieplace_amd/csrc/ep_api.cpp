@@ -1713,8 +1713,17 @@ extern "C" ep_status ep_transform(int32_t row_kind, int32_t col_kind, int32_t nx
     ep_status pst = check_precision(precision, "ep_transform");
     if (pst != EP_OK) return pst;
     const size_t nb = (size_t)nx * ny;
-    for (size_t k = 0; k < nb; ++k)
-        if (!std::isfinite(in[k])) return fail(EP_ENAN, "ep_transform: non-finite input at %zu", k);
+    for (size_t k = 0; k < nb; k += 4096) {
+        const size_t end = std::min(nb, k + 4096);
+        uint32_t bad = 0;  // no branch per value: vectorised
+        for (size_t j = k; j < end; ++j) {
+            uint32_t u;
+            std::memcpy(&u, &in[j], 4);
+            bad |= (u & 0x7F800000u) == 0x7F800000u;
+        }
+        for (size_t j = k; bad && j < end; ++j)
+            if (!std::isfinite(in[j])) return fail(EP_ENAN, "ep_transform: non-finite input at %zu", j);
+    }
     int nd = 0;
     if (hipGetDeviceCount(&nd) != hipSuccess || nd < 1) return fail(EP_EDEVICE, "ep_transform: no HIP device");
     return run_transform(row_kind, col_kind, nx, ny, in, out, precision);

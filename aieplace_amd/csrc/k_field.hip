@@ -33,7 +33,6 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
-#include <cstring>
 #include <new>
 #include <vector>
 
@@ -326,8 +325,8 @@ __device__ inline f32x16 mfma16(const uint16_t *pa, const uint16_t *pb, f32x16 a
 // Splits two values into 16-bit hi and lo parts, x0 in the low half of each
 // word.  Both conversions are the packed hardware ones (one instruction for two
 // values, rounding to nearest even); for finite values the BF16 bits equal
-// rounding the FP32 pattern, (u + 0x7FFF + bit 16 of u) >> 16, as the host's
-// bf16_rne_host does for the constant matrices.
+// rounding the FP32 pattern, (u + 0x7FFF + bit 16 of u) >> 16, as k_halves
+// does for the constant matrices.
 template <bool F16>
 __device__ inline void split2(float x0, float x1, uint32_t &h, uint32_t &l)
 {
@@ -666,55 +665,6 @@ std::vector<double> trig(int M, bool sine, bool transpose)
     return t;
 }
 
-uint16_t bf16_rne_host(float x)
-{
-    uint32_t u;
-    std::memcpy(&u, &x, 4);
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
-}
-
-float bf16_to_f_host(uint16_t h)
-{
-    uint32_t u = (uint32_t)h << 16;
-    float f;
-    std::memcpy(&f, &u, 4);
-    return f;
-}
-
-uint16_t f16_host(float x)
-{
-    const _Float16 h = (_Float16)x;
-    uint16_t u;
-    std::memcpy(&u, &h, 2);
-    return u;
-}
-
-float f16_to_f_host(uint16_t u)
-{
-    _Float16 h;
-    std::memcpy(&h, &u, 2);
-    return (float)h;
-}
-
-// Even and odd halves, (M/2) x (M/2) row-major, of one transform matrix:
-//   forward (T[f][x]):  E[r][x] = T[2r][x],  O[r][x] = T[2r+1][x]     (x < M/2)
-//   inverse (T'[x][f]): E[x][r] = T'[x][2r], O[x][r] = T'[x][2r+1]    (x < M/2)
-// with T[f][x] = cos|sin(pi f (x + 1/2) / M) and T' its transpose.
-void halves(int M, bool sine, bool inverse, std::vector<double> &E, std::vector<double> &O)
-{
-    const int h = M / 2;
-    E.assign((size_t)h * h, 0.0);
-    O.assign((size_t)h * h, 0.0);
-    for (int r = 0; r < h; ++r)
-        for (int x = 0; x < h; ++x) {
-            const double ae = M_PI * (2.0 * r) * (x + 0.5) / M, ao = M_PI * (2.0 * r + 1.0) * (x + 0.5) / M;
-            const size_t o = inverse ? (size_t)x * h + r : (size_t)r * h + x;
-            E[o] = sine ? std::sin(ae) : std::cos(ae);
-            O[o] = sine ? std::sin(ao) : std::cos(ao);
-        }
-}
-
 }  // namespace
 
 // Matrix slots (all copies share the index).
@@ -725,49 +675,88 @@ constexpr bool kSlotSine[MAT_N] = {false, false, false, true, true, false};
 constexpr bool kSlotInv[MAT_N] = {false, false, true, true, true, true};
 constexpr float kSlotSign[MAT_N] = {1.f, 1.f, 1.f, -1.f, -1.f, 1.f};
 
-// Device copies of one slot's halves ([0] even, [1] odd) in every precision.
+// Device copies of one slot's halves ([0] even, [1] odd) in every precision, in
+// one allocation.
 struct HalfMats {
+    void *mem = nullptr;
     float *f32[2] = {};
     uint16_t *bh[2] = {}, *bl[2] = {};   // BF16 hi/lo
     uint16_t *fh[2] = {}, *fl[2] = {};   // FP16 hi/lo
 };
 
-static ep_status upload_halves(int M, int slot, HalfMats &hm)
+// Sets the pointers of an M x M transform's halves in `mem` (may be null);
+// returns its bytes.  (M/2)^2 elements and 256-byte planes.
+static size_t place_halves(int M, void *mem, HalfMats &hm)
 {
-    std::vector<double> d[2];
-    halves(M, kSlotSine[slot], kSlotInv[slot], d[0], d[1]);
+    const size_t n = (size_t)(M / 2) * (M / 2);
+    size_t at = 0;
+    auto plane = [&](size_t bytes) {
+        char *p = mem ? static_cast<char *>(mem) + at : nullptr;
+        at += (n * bytes + 255) / 256 * 256;
+        return p;
+    };
     for (int k = 0; k < 2; ++k) {
-        const size_t n = d[k].size();
-        std::vector<float> f(n);
-        std::vector<uint16_t> h(n), l(n), h16(n), l16(n);
-        for (size_t e = 0; e < n; ++e) {
-            f[e] = (float)d[k][e];
-            h[e] = bf16_rne_host(f[e]);
-            l[e] = bf16_rne_host(f[e] - bf16_to_f_host(h[e]));
-            h16[e] = f16_host(f[e]);
-            l16[e] = f16_host(f[e] - f16_to_f_host(h16[e]));
-        }
-        if (hipMalloc(&hm.f32[k], n * 4) != hipSuccess || hipMalloc(&hm.bh[k], n * 2) != hipSuccess ||
-            hipMalloc(&hm.bl[k], n * 2) != hipSuccess || hipMalloc(&hm.fh[k], n * 2) != hipSuccess ||
-            hipMalloc(&hm.fl[k], n * 2) != hipSuccess)
-            return fail(EP_ENOMEM, "field: hipMalloc of transform matrices failed");
-        if (hipMemcpy(hm.f32[k], f.data(), n * 4, hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(hm.bh[k], h.data(), n * 2, hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(hm.bl[k], l.data(), n * 2, hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(hm.fh[k], h16.data(), n * 2, hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(hm.fl[k], l16.data(), n * 2, hipMemcpyHostToDevice) != hipSuccess)
-            return fail(EP_EDEVICE, "field: upload of transform matrices failed");
+        hm.f32[k] = reinterpret_cast<float *>(plane(4));
+        hm.bh[k] = reinterpret_cast<uint16_t *>(plane(2));
+        hm.bl[k] = reinterpret_cast<uint16_t *>(plane(2));
+        hm.fh[k] = reinterpret_cast<uint16_t *>(plane(2));
+        hm.fl[k] = reinterpret_cast<uint16_t *>(plane(2));
     }
+    return at;
+}
+
+// Even and odd halves, (M/2) x (M/2) row-major, of one transform matrix:
+//   forward (T[f][x]):  E[r][x] = T[2r][x],  O[r][x] = T[2r+1][x]     (x < M/2)
+//   inverse (T'[x][f]): E[x][r] = T'[x][2r], O[x][r] = T'[x][2r+1]    (x < M/2)
+// with T[f][x] = cos|sin(pi f (x + 1/2) / M) and T' its transpose.  The angle is
+// pi m / 2M with the integer m = f (2x + 1), reduced exactly mod 4M; FP64, then
+// rounded to FP32 and split.  Bound by FP64 arithmetic, 2-3 us up to 1024 x 1024.
+// Made on the host, the matrices were most of a standalone transform: 512 x 512 6.5
+// ms, 0.24 with them made here, one allocation per call and no staging of plain rows.
+__global__ __launch_bounds__(256) void k_halves(HalfMats hm, int M, int sine, int inverse)
+{
+    const int h = M / 2, odd = blockIdx.y;
+    const uint32_t e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= (uint32_t)h * h) return;
+    const uint32_t row = e / h, col = e - row * h;
+    const uint32_t f = 2 * (inverse ? col : row) + odd, x = inverse ? row : col;
+    const double t = (double)(f * (2 * x + 1) % (4u * M)) / (2.0 * M);
+    const float v = (float)(sine ? sinpi(t) : cospi(t));
+    hm.f32[odd][e] = v;
+    auto bf16 = [](float a, float &back) {  // rounded to nearest even
+        const uint32_t u = __float_as_uint(a), r = (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
+        back = __uint_as_float(r << 16);
+        return (uint16_t)r;
+    };
+    float back;
+    hm.bh[odd][e] = bf16(v, back);
+    hm.bl[odd][e] = bf16(v - back, back);
+    const _Float16 fh = (_Float16)v, fl = (_Float16)(v - (float)fh);
+    hm.fh[odd][e] = __builtin_bit_cast(uint16_t, fh);
+    hm.fl[odd][e] = __builtin_bit_cast(uint16_t, fl);
+}
+
+static void launch_halves(const HalfMats &hm, int M, int slot, hipStream_t s)
+{
+    const unsigned n = (unsigned)(M / 2) * (M / 2);
+    hipLaunchKernelGGL(k_halves, dim3((n + 255) / 256, 2), dim3(256), 0, s, hm, M, kSlotSine[slot] ? 1 : 0,
+                       kSlotInv[slot] ? 1 : 0);
+}
+
+static ep_status make_halves(int M, int slot, HalfMats &hm)
+{
+    const size_t bytes = place_halves(M, nullptr, hm);
+    if (hipMalloc(&hm.mem, bytes) != hipSuccess)
+        return fail(EP_ENOMEM, "field: hipMalloc of transform matrices failed");
+    place_halves(M, hm.mem, hm);
+    launch_halves(hm, M, slot, nullptr);
+    if (hipGetLastError() != hipSuccess) return fail(EP_EDEVICE, "field: transform matrices: launch failed");
     return EP_OK;
 }
 
 static void free_halves(HalfMats &hm)
 {
-    for (int k = 0; k < 2; ++k) {
-        void *p[] = {hm.f32[k], hm.bh[k], hm.bl[k], hm.fh[k], hm.fl[k]};
-        for (void *q : p)
-            if (q) (void)hipFree(q);
-    }
+    if (hm.mem) (void)hipFree(hm.mem);
     hm = HalfMats();
 }
 
@@ -834,7 +823,7 @@ ep_status field_init(Ctx &c)
         int M;
         bool sine, tr;
         matrix_desc(c, m, M, sine, tr);
-        ep_status st = upload_halves(M, m, fm->half[m]);
+        ep_status st = make_halves(M, m, fm->half[m]);
         if (st != EP_OK) return st;
     }
     // [0,4): split-FP16 operand maxima; [4]: field map mean (float)
@@ -1044,7 +1033,7 @@ ep_status batch_field_init(BatchField *&out, const std::vector<BatchFieldInst> &
             continue;
         }
         for (int m = 0; m < MAT_N; ++m) {
-            ep_status st = upload_halves(bf->sizes[si], m, bf->sets[si].half[m]);
+            ep_status st = make_halves(bf->sizes[si], m, bf->sets[si].half[m]);
             if (st != EP_OK) return st;
         }
     }
@@ -1295,7 +1284,8 @@ constexpr int kTrBlock = 256;
 // X[r][k] = rowsign(r) * h(k) * src[r][k'] over R rows of length n, where
 // k' = n - k for reversed rows (k > 0), h(0) = 1/2 when `halve`, and rowsign(r)
 // = (-1)^r when `altsign` (the previous pass was an IDXST).  `tr`: the source is
-// the n x R map whose columns are the rows (src[k'][r]).  Tracks max |X| in maxbits.
+// the n x R map whose columns are the rows (src[k'][r]).  Tracks max |X| in maxbits
+// (null: not needed; the blocks' atomics take most of the pass).
 __global__ __launch_bounds__(kTrBlock) void k_tr_prep(const float *__restrict__ src, float *__restrict__ X,
                                                       int R, int n, int tr, int reverse, int halve, int altsign,
                                                       uint32_t *__restrict__ maxbits)
@@ -1311,7 +1301,7 @@ __global__ __launch_bounds__(kTrBlock) void k_tr_prep(const float *__restrict__ 
         X[e] = v;
         m = fmaxf(m, fabsf(v));
     }
-    track_max(maxbits, m);
+    if (maxbits) track_max(maxbits, m);
 }
 
 // Product output C[f][r] (n x R) -> Y: sign (-1)^f when `altsign`; Y[r][f] when
@@ -1336,7 +1326,7 @@ __global__ void k_tr_zero(uint32_t *p, int n)
 int tr_grid(int64_t n)
 {
     const int64_t g = (n + kTrBlock - 1) / kTrBlock;
-    return (int)std::min<int64_t>(std::max<int64_t>(g, 1), 4096);
+    return (int)std::min<int64_t>(std::max<int64_t>(g, 1), 1024);
 }
 
 }  // namespace
@@ -1344,82 +1334,72 @@ int tr_grid(int64_t n)
 ep_status run_transform(int row_kind, int col_kind, int nx, int ny, const float *in, float *out, int precision)
 {
     const size_t nb = (size_t)nx * ny;
-    float *d_in = nullptr, *d_x = nullptr, *d_c = nullptr, *d_out = nullptr;
-    uint32_t *d_max = nullptr;
-    HalfMats mats[2];
-    ep_status st = EP_OK;
-    hipStream_t s = nullptr;
-    auto cleanup = [&]() {
-        void *p[] = {d_in, d_x, d_c, d_out, d_max};
-        for (void *q : p)
-            if (q) (void)hipFree(q);
-        free_halves(mats[0]);
-        free_halves(mats[1]);
-    };
-    if (hipMalloc(&d_in, nb * 4) != hipSuccess || hipMalloc(&d_x, nb * 4) != hipSuccess ||
-        hipMalloc(&d_c, nb * 4) != hipSuccess || hipMalloc(&d_out, nb * 4) != hipSuccess ||
-        hipMalloc(&d_max, 4 * sizeof(uint32_t)) != hipSuccess) {
-        cleanup();
+    const hipStream_t s = nullptr;
+    // one allocation: operand maxima, three maps, and the matrix of the pass that runs
+    // (the passes follow each other on the stream)
+    HalfMats hm;
+    const int longest = std::max(col_kind == EP_TR_NONE ? 0 : nx, row_kind == EP_TR_NONE ? 0 : ny);
+    const size_t map_bytes = (nb * 4 + 255) / 256 * 256, mat_bytes = place_halves(longest, nullptr, hm);
+    char *mem = nullptr;
+    if (hipMalloc(&mem, 256 + 3 * map_bytes + mat_bytes) != hipSuccess)
         return fail(EP_ENOMEM, "ep_transform: hipMalloc failed");
-    }
+    uint32_t *d_max = reinterpret_cast<uint32_t *>(mem);
+    float *d_in = reinterpret_cast<float *>(mem + 256);
+    float *d_x = reinterpret_cast<float *>(mem + 256 + map_bytes);
+    float *d_c = reinterpret_cast<float *>(mem + 256 + 2 * map_bytes);
+    void *mats = mem + 256 + 3 * map_bytes;
     if (hipMemcpy(d_in, in, nb * 4, hipMemcpyHostToDevice) != hipSuccess) {
-        cleanup();
+        (void)hipFree(mem);
         return fail(EP_EDEVICE, "ep_transform: upload failed");
     }
-    hipLaunchKernelGGL(k_tr_zero, dim3(1), dim3(64), 0, s, d_max, 4);
-    // One pass: rows of X (R x n, staged from src) through the product into C (n x R).
-    auto pass = [&](int kind, int n, int R, const float *src, int tr, int altsign, HalfMats &hm,
-                    uint32_t *bmax, uint32_t *cmax) -> ep_status {
+    const bool f16 = precision == EP_PREC_FP16X3;  // its products scale by the operand's maximum
+    if (f16) hipLaunchKernelGGL(k_tr_zero, dim3(1), dim3(64), 0, s, d_max, 4);
+    // One pass: the rows of src (R x n; `tr`: its columns) through the product into C
+    // (n x R).  A DCT of plain rows reads src itself, the others a staged copy.
+    auto pass = [&](int kind, int n, int R, const float *src, float *X, float *C, int tr, int altsign, int k) {
         const int slot = kind == EP_TR_DCT ? MAT_CX : MAT_CXT;  // forward / inverse cosine
-        ep_status e = upload_halves(n, slot, hm);
-        if (e != EP_OK) return e;
-        hipLaunchKernelGGL(k_tr_prep, dim3(tr_grid((int64_t)R * n)), dim3(kTrBlock), 0, s, src, d_x, R, n, tr,
-                           kind == EP_TR_IDXST ? 1 : 0, kind == EP_TR_DCT ? 0 : 1, altsign, bmax);
+        place_halves(n, mats, hm);
+        launch_halves(hm, n, slot, s);
+        const bool plain = kind == EP_TR_DCT && !tr && !altsign && !f16;
+        if (!plain)
+            hipLaunchKernelGGL(k_tr_prep, dim3(tr_grid((int64_t)R * n)), dim3(kTrBlock), 0, s, src, X, R, n, tr,
+                               kind == EP_TR_IDXST ? 1 : 0, kind == EP_TR_DCT ? 0 : 1, altsign,
+                               f16 ? d_max + k : nullptr);
         GemmArgs a{};
         set_operand(a, 0, hm, slot, precision);
         a.M = n;
         a.N = R;
         a.K = n;
-        a.B[0] = d_x;
-        a.C[0] = d_c;
-        a.bmax = bmax;
-        a.cmax = cmax;
+        a.B[0] = plain ? src : X;
+        a.C[0] = C;
+        a.bmax = d_max + k;
         gemm(a, 1, kind != EP_TR_DCT, 0, precision, s);
-        return EP_OK;
+    };
+    // `C` (n x R) -> the result: transposed, or with an IDXST's alternating signs
+    const float *result = nullptr;
+    auto post = [&](int kind, int n, int R, const float *C, float *Y, int tr) {
+        const int altsign = kind == EP_TR_IDXST ? 1 : 0;
+        result = altsign || tr ? Y : C;
+        if (altsign || tr)
+            hipLaunchKernelGGL(k_tr_post, dim3(tr_grid((int64_t)nb)), dim3(kTrBlock), 0, s, C, Y, R, n, altsign, tr);
     };
     if (row_kind != EP_TR_NONE && col_kind != EP_TR_NONE) {
         // rows of in (nx rows of length ny) -> C1[v][i]; then the rows of C1
         // (ny rows of length nx) -> C2[u][v] = out
-        if ((st = pass(row_kind, ny, nx, d_in, 0, 0, mats[0], d_max + 0, d_max + 1)) != EP_OK) {
-            cleanup();
-            return st;
-        }
-        if ((st = pass(col_kind, nx, ny, d_c, 0, row_kind == EP_TR_IDXST, mats[1], d_max + 2, d_max + 3)) !=
-            EP_OK) {
-            cleanup();
-            return st;
-        }
-        hipLaunchKernelGGL(k_tr_post, dim3(tr_grid((int64_t)nb)), dim3(kTrBlock), 0, s, d_c, d_out, ny, nx,
-                           col_kind == EP_TR_IDXST ? 1 : 0, 0);
+        pass(row_kind, ny, nx, d_in, d_x, d_c, 0, 0, 0);
+        pass(col_kind, nx, ny, d_c, d_x, d_in, 0, row_kind == EP_TR_IDXST, 1);
+        post(col_kind, nx, ny, d_in, d_c, 0);
     } else if (row_kind != EP_TR_NONE) {
-        if ((st = pass(row_kind, ny, nx, d_in, 0, 0, mats[0], d_max + 0, d_max + 1)) != EP_OK) {
-            cleanup();
-            return st;
-        }
-        hipLaunchKernelGGL(k_tr_post, dim3(tr_grid((int64_t)nb)), dim3(kTrBlock), 0, s, d_c, d_out, nx, ny,
-                           row_kind == EP_TR_IDXST ? 1 : 0, 1);
+        pass(row_kind, ny, nx, d_in, d_x, d_c, 0, 0, 0);
+        post(row_kind, ny, nx, d_c, d_x, 1);
     } else {
         // columns of in: staged transposed (ny rows of length nx) -> C[u][j] = out
-        if ((st = pass(col_kind, nx, ny, d_in, 1, 0, mats[0], d_max + 0, d_max + 1)) != EP_OK) {
-            cleanup();
-            return st;
-        }
-        hipLaunchKernelGGL(k_tr_post, dim3(tr_grid((int64_t)nb)), dim3(kTrBlock), 0, s, d_c, d_out, ny, nx,
-                           col_kind == EP_TR_IDXST ? 1 : 0, 0);
+        pass(col_kind, nx, ny, d_in, d_x, d_c, 1, 0, 0);
+        post(col_kind, nx, ny, d_c, d_x, 0);
     }
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpy(out, d_out, nb * 4, hipMemcpyDeviceToHost);
-    cleanup();
+    if (e == hipSuccess) e = hipMemcpy(out, result, nb * 4, hipMemcpyDeviceToHost);
+    (void)hipFree(mem);
     if (e != hipSuccess) return fail(EP_EDEVICE, "ep_transform: %s", hipGetErrorString(e));
     return EP_OK;
 }
