@@ -677,7 +677,7 @@ static ep_status build_graph(ep_batch *b)
     hipError_t e = hipSuccess;
     for (int t = 0; t < kTrialsPerLaunch && e == hipSuccess; ++t) {
         bl_move(d, kMoveTrial, b->sort_blocks, b->stream);
-        if (b->active_cells() >= fork_min_cells(b->prm))
+        if (b->active_cells() >= fork_min_cells(b->prm, kForkMinCellsBatch))
             e = b->eval_forked(d, kAtTrial, true, b->stream, kCtlIterate);
         else b->eval(d, kAtTrial, true, b->stream, kCtlIterate);
     }

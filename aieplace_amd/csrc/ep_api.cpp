@@ -94,10 +94,10 @@ void push_scalars(Ctx &c, hipStream_t s)
 void enqueue_eval(Ctx &c, const float2 *pos, const float2 *vref, const float2 *gref, float2 *gout,
                   float2 *gw_out, float2 *f_out, hipStream_t s, bool counted = false)
 {
-    launch_sort(c, pos, counted, s);
-    launch_density(c, s);
+    if (!counted) launch_sort_count(c, pos, s);
+    launch_sort_wa(c, pos, s);
+    launch_density_pins(c, s);
     launch_overflow(c, s);
-    launch_wa(c, pos, s);
     launch_field(c, c.prm.precision, s);
     launch_cell_grad(c, pos, counted ? nullptr : vref, gref, gout, gw_out, f_out, s);
     launch_finalize(c, s, counted);
@@ -842,7 +842,8 @@ extern "C" ep_status ep_get_positions(ep_ctx *c, float *x, float *y)
 
 static ep_status run_density(ep_ctx *c)
 {
-    launch_sort(*c, c->V[c->cur], false, c->stream);
+    launch_sort_count(*c, c->V[c->cur], c->stream);
+    launch_sort(*c, c->V[c->cur], c->stream);
     launch_density(*c, c->stream);
     launch_overflow(*c, c->stream);
     launch_finalize(*c, c->stream);
@@ -927,6 +928,7 @@ extern "C" ep_status ep_get_wa_grad(ep_ctx *c, float *gx, float *gy)
     push_scalars(*c, c->stream);
     // the other parity's buffers hold a past trial
     float2 *scratch = c->G[c->cur ^ 1], *gw = c->U[c->cur ^ 1];
+    launch_pin_sum(*c, c->stream);
     launch_cell_grad(*c, c->V[c->cur], nullptr, nullptr, scratch, gw, nullptr, c->stream);
     ep_status st = check_launch();
     if (st != EP_OK) return st;
@@ -1277,14 +1279,13 @@ static ep_status build_ctl_graph(ep_ctx *c, const CtlParams &p)
         // the model's proposal for this trial was made by the previous decision
         // (k_finalize) or by k_step_begin
         launch_trial(x, vc, uc, gc, vn, un, true, s);
-        if (x.n_place >= fork_min_cells(x.prm)) {
+        if (x.n_place >= fork_min_cells(x.prm, kForkMinCells)) {
             // fork right after the trial: the tile sort, the density scatter and
-            // the transform products on the second stream (the critical chain;
-            // the products take issue priority), the WA gradient and the
-            // per-cell pin sums beside them
+            // the transforms on the second stream (the critical chain), the WA
+            // gradient and the per-cell pin sums beside them
             EP_CAP(hipEventRecord(x.fork, s), s);
             EP_CAP(hipStreamWaitEvent(x.side, x.fork, 0), s);
-            launch_sort(x, vt, true, x.side);
+            launch_sort(x, vt, x.side);
             launch_density(x, x.side);
             launch_overflow(x, x.side);
             launch_field(x, x.prm.precision, x.side);
@@ -1292,12 +1293,11 @@ static ep_status build_ctl_graph(ep_ctx *c, const CtlParams &p)
             launch_wa(x, vt, s);
             launch_pin_sum(x, s);
             EP_CAP(hipStreamWaitEvent(s, x.join, 0), s);
-            launch_cell_grad(x, vt, none, gc, gn, nullptr, nullptr, s, x.gw_cell);
+            launch_cell_grad(x, vt, none, gc, gn, nullptr, nullptr, s);
         } else {
-            launch_sort(x, vt, true, s);
-            launch_density(x, s);
+            launch_sort_wa(x, vt, s);
+            launch_density_pins(x, s);
             launch_overflow(x, s);
-            launch_wa(x, vt, s);
             launch_field(x, x.prm.precision, s);
             launch_cell_grad(x, vt, none, gc, gn, nullptr, nullptr, s);
         }
@@ -1451,7 +1451,8 @@ extern "C" ep_status ep_profile(ep_ctx *c, int32_t reps, ep_kernel_stat *out, in
     c->h_scal->coef = 0.0f;
     push_scalars(*c, c->stream);
     // field input must be a real map: build it once at the current positions
-    launch_sort(*c, c->V[a], false, c->stream);
+    launch_sort_count(*c, c->V[a], c->stream);
+    launch_sort(*c, c->V[a], c->stream);
     launch_density(*c, c->stream);
     launch_overflow(*c, c->stream);
     hipEvent_t e0, e1;
@@ -1474,10 +1475,8 @@ extern "C" ep_status ep_profile(ep_ctx *c, int32_t reps, ep_kernel_stat *out, in
     // maps go between its three kernels.
     const bool fft = fft_side(c->Mx) && fft_side(c->My);
     const double field_bytes = fft ? 36.0 * nb : 4.0 * 13 * nb + 4.0 * 1.5 * (Mxd * Mxd + Myd * Myd);
-    // Instances that fork their captured evaluation sum the pin partials per cell
-    // on the WA branch (k_pin_sum), and the cell gradient reads those sums: both
-    // are timed that way here, as the placement runs them.
-    const bool forked = c->n_place >= fork_min_cells(c->prm);
+    // Each kernel is timed by itself, also where the placement runs two in one launch
+    // or on two branches.
     std::vector<Item> items = {
         // positions and sizes read twice, packed cells written once
         {"cell_sort", 3, 2 * 16.0 * np + 16.0 * np + 8.0 * kSortTiles, 0},
@@ -1488,18 +1487,14 @@ extern "C" ep_status ep_profile(ep_ctx *c, int32_t reps, ep_kernel_stat *out, in
         {"overflow", 1, 44.0 * nb, 0},
         {"wa_grad", 1, 4.0 * (N + 1) + 12.0 * P + 8.0 * c->n_all + 8.0 * P, 0},
         {"field_transforms", fft ? 3 : 4, field_bytes, fft ? 0 : gemm_flops},
-    };
-    if (forked) {
         // CSR offsets and pin list read, the pins' partials gathered, one sum
         // per movable cell written
-        items.push_back({"pin_sum", 1, 4.0 * (c->n_mov + 1) + 12.0 * pm + 8.0 * c->n_mov, 0});
-        items.push_back({"cell_grad", 1, 36.0 * np + 8.0 * c->n_mov + 8.0 * nb, 0});
-    } else {
-        items.push_back({"cell_grad", 1, 36.0 * np + 12.0 * pm + 4.0 * c->n_mov + 8.0 * nb, 0});
-    }
-    // v, u, g, size read; v, u written (the tile counts stay in LDS)
-    items.push_back({"nesterov_trial", 1, 40.0 * np, 0});
-    items.push_back({"finalize", 1, 8.0 * c->part_total, 0});
+        {"pin_sum", 1, 4.0 * (c->n_mov + 1) + 12.0 * pm + 8.0 * c->n_mov, 0},
+        {"cell_grad", 1, 36.0 * np + 8.0 * c->n_mov + 8.0 * nb, 0},
+        // v, u, g, size read; v, u written (the tile counts stay in LDS)
+        {"nesterov_trial", 1, 40.0 * np, 0},
+        {"finalize", 1, 8.0 * c->part_total, 0},
+    };
     int k = 0;
     for (const Item &it : items) {
         EP_HIP(hipEventRecord(e0, c->stream));
@@ -1507,7 +1502,8 @@ extern "C" ep_status ep_profile(ep_ctx *c, int32_t reps, ep_kernel_stat *out, in
             const std::string nm = it.name;
             if (nm == "cell_sort") {
                 launch_sort_clear(*c, c->stream);
-                launch_sort(*c, c->V[a], false, c->stream);
+                launch_sort_count(*c, c->V[a], c->stream);
+                launch_sort(*c, c->V[a], c->stream);
             }
             else if (nm == "density_scatter") launch_density(*c, c->stream);
             else if (nm == "overflow") launch_overflow(*c, c->stream);
@@ -1516,8 +1512,7 @@ extern "C" ep_status ep_profile(ep_ctx *c, int32_t reps, ep_kernel_stat *out, in
             else if (nm == "pin_sum") launch_pin_sum(*c, c->stream);
             else if (nm == "cell_grad")
                 launch_cell_grad(*c, same<const float2>(c->V[a]), same<const float2>(nullptr),
-                                 same<const float2>(c->G[a]), same<float2>(c->G[b]), nullptr, nullptr, c->stream,
-                                 forked ? c->gw_cell : nullptr);
+                                 same<const float2>(c->G[a]), same<float2>(c->G[b]), nullptr, nullptr, c->stream);
             else if (nm == "nesterov_trial") launch_trial(*c, c->V[a], c->U[a], c->G[a], c->V[b], c->U[b], true, c->stream);
             else launch_finalize(*c, c->stream, true);
         }
@@ -1546,7 +1541,8 @@ extern "C" ep_status ep_profile(ep_ctx *c, int32_t reps, ep_kernel_stat *out, in
         if (cpt == cpt0) continue;
         c->dens.cpt = cpt;
         launch_sort_clear(*c, c->stream);
-        launch_sort(*c, c->V[a], false, c->stream);
+        launch_sort_count(*c, c->V[a], c->stream);
+        launch_sort(*c, c->V[a], c->stream);
         EP_HIP(hipEventRecord(e0, c->stream));
         for (int r = 0; r < reps; ++r) launch_density(*c, c->stream);
         EP_HIP(hipEventRecord(e1, c->stream));
@@ -1571,7 +1567,8 @@ extern "C" ep_status ep_profile(ep_ctx *c, int32_t reps, ep_kernel_stat *out, in
     // leave the maps consistent with the current positions
     launch_fill_maps(*c, c->stream);
     launch_sort_clear(*c, c->stream);
-    launch_sort(*c, c->V[a], false, c->stream);
+    launch_sort_count(*c, c->V[a], c->stream);
+    launch_sort(*c, c->V[a], c->stream);
     launch_density(*c, c->stream);
     launch_overflow(*c, c->stream);
     return sync(*c);

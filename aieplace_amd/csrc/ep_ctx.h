@@ -59,7 +59,9 @@ constexpr int kSortTiles = kSortSide * kSortSide;
 // 40.8 / 35.3 / 32.7 / 31.6 / 31.6.  A batch's blocks stop at its instances' ends:
 // 16 instances (450k cells in all) 12.6 / 12.6 / 12.7 / 13.0 / 13.9, 64 (3.7M) 53.7 /
 // 50.8 / 50.3 / 50.9 / 51.5.
-constexpr int kSortMost = 8, kSortBlocks = 160;
+// Beside net tiles (k_sort_wa) 4 is the most: the registers of 8 cells (73) would
+// leave the gathers 6 waves a SIMD instead of 8.
+constexpr int kSortMost = 8, kSortBlocks = 160, kSortWaMost = 4;
 constexpr int kSortBatchMost = 4, kSortBatchBlocks = 512;
 inline int sort_cells_per_thread(int64_t n, int most, int blocks)
 {
@@ -80,13 +82,19 @@ inline void with_sort_cpt(int cpt, Go go)
 // iterations (reset by an accepted proposal): phases where it mispredicts cost
 // one extra evaluation per rejection, so they are skipped.
 constexpr int kModelBackoffMax = 32;
-// Captured evaluations fork the WA gradient onto a second branch only from this
-// many placeable cells on (ep_params.fork_min_cells = 0): the fork and join cost
-// ~15 us per trial, more than the overlap saves on small instances.
-constexpr int64_t kForkMinCells = 400000;
-inline int64_t fork_min_cells(const ep_params &p)
+// Captured evaluations fork the WA gradient and the pin sums onto a second branch
+// only from this many placeable cells on (ep_params.fork_min_cells = 0).  Below, each
+// shares a launch with the sort and the density scatter (k_sort_wa, k_density_pins):
+// the fork and join cost ~15 us per trial, and a small instance's kernels leave CUs
+// idle.  A large one's kernels fill the chip; its branches overlap the gathers with the
+// transforms too.  us per evaluation, two branches / shared launches (before those: one
+// branch of single kernels): 383k placeable cells 90.7 / 84.6 (93.4), 643k 134.3 / 133.5
+// (145), 1.28M 173 / 179 (193), 2.56M 271 / 295 (302).
+constexpr int64_t kForkMinCells = 800000;
+constexpr int64_t kForkMinCellsBatch = 400000;  // of a batch's running instances
+inline int64_t fork_min_cells(const ep_params &p, int64_t most)
 {
-    return p.fork_min_cells > 0 ? (int64_t)p.fork_min_cells : kForkMinCells;
+    return p.fork_min_cells > 0 ? (int64_t)p.fork_min_cells : most;
 }
 // Step-model records kept per context between ep_take_step_records calls.
 constexpr size_t kMaxStepRecords = (size_t)1 << 21;
@@ -232,26 +240,29 @@ struct Ctx;
 // Clears the scatter accumulators (set-up and re-synchronisation; every
 // evaluation's overflow pass leaves them clear).
 void launch_fill_maps(Ctx &c, hipStream_t s);
-// Tile-sorts the cells at pos; `counted`: the tile counts were already made by
-// a counting launch_trial at the same positions.
-void launch_sort(Ctx &c, Pair<const float2> pos, bool counted, hipStream_t s);
-// Clears the sort's counts, as launch_overflow does (for sorts without one between).
+// Counts the cells at pos into the sort's tiles (a counting launch_trial does the
+// same), clears the counts as launch_overflow does (for sorts without one between).
+void launch_sort_count(Ctx &c, Pair<const float2> pos, hipStream_t s);
 void launch_sort_clear(Ctx &c, hipStream_t s);
-// Scatters the cells packed by the last launch_sort (same positions).
+// Tile-sorts the counted cells at pos; the WA gradient's pin partials at pos; both
+// in one launch.
+void launch_sort(Ctx &c, Pair<const float2> pos, hipStream_t s);
+void launch_wa(Ctx &c, Pair<const float2> pos, hipStream_t s);
+void launch_sort_wa(Ctx &c, Pair<const float2> pos, hipStream_t s);
+// Scatters the cells packed by the last sort (same positions); gw_cell[c] = sum of
+// movable cell c's pin partials (after the WA gradient); both in one launch.
 void launch_density(Ctx &c, hipStream_t s);
+void launch_pin_sum(Ctx &c, hipStream_t s);
+void launch_density_pins(Ctx &c, hipStream_t s);
 void launch_overflow(Ctx &c, hipStream_t s);
 // Split-FP16 products: max |field map - mean| of the last overflow pass into
 // field_max[0] (the operand scale of the first product).
 void launch_map_range(Ctx &c, hipStream_t s);
-void launch_wa(Ctx &c, Pair<const float2> pos, hipStream_t s);
 void launch_field(Ctx &c, int precision, hipStream_t s);
-// gw_cell (nullable): per-cell pin-partial sums made by launch_pin_sum; without
-// it the kernel gathers them itself.
+// Reads the cells' pin-partial sums (gw_cell).
 void launch_cell_grad(Ctx &c, Pair<const float2> pos, Pair<const float2> vref,
                       Pair<const float2> gref, Pair<float2> gout, float2 *gw_out, float2 *f_out,
-                      hipStream_t s, const float2 *gw_cell = nullptr);
-// gw_cell[c] = sum of movable cell c's pin partials (after launch_wa).
-void launch_pin_sum(Ctx &c, hipStream_t s);
+                      hipStream_t s);
 // trial: the evaluated point came from a counting launch_trial, whose partial
 // sums hold |v' - v|^2 (k_cell_grad then gets no vref)
 void launch_finalize(Ctx &c, hipStream_t s, bool trial = false);
@@ -264,10 +275,9 @@ void launch_trial(Ctx &c, Pair<const float2> v, Pair<const float2> u, Pair<const
 void launch_step_begin(Ctx &c, const CtlParams &p, hipStream_t s);
 void launch_finalize_decide(Ctx &c, const CtlParams &p, hipStream_t s);
 // Fixed-buffer forms of the launchers above.
-inline void launch_sort(Ctx &c, const float2 *pos, bool counted, hipStream_t s)
-{
-    launch_sort(c, same(pos), counted, s);
-}
+inline void launch_sort_count(Ctx &c, const float2 *pos, hipStream_t s) { launch_sort_count(c, same(pos), s); }
+inline void launch_sort(Ctx &c, const float2 *pos, hipStream_t s) { launch_sort(c, same(pos), s); }
+inline void launch_sort_wa(Ctx &c, const float2 *pos, hipStream_t s) { launch_sort_wa(c, same(pos), s); }
 inline void launch_wa(Ctx &c, const float2 *pos, hipStream_t s) { launch_wa(c, same(pos), s); }
 inline void launch_cell_grad(Ctx &c, const float2 *pos, const float2 *vref, const float2 *gref,
                              float2 *gout, float2 *gw_out, float2 *f_out, hipStream_t s)

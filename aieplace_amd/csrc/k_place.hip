@@ -10,6 +10,7 @@
 // overflow Bin.h:123-126; HPWL Net.cpp:136-155; cell update AIEplace.cpp:993-1046.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cfloat>
 #include <climits>
 #include <mutex>
@@ -77,22 +78,29 @@ __global__ __launch_bounds__(kBlock) void k_sort_count(Pair<const float2> pos_pa
 // pass clears both).  Every block scans the 1024 counts for itself, beside its
 // cell loads: a kernel for the scan took 4.5 us of every evaluation.  Block 0
 // leaves the tables of the coming density scatter.
+struct SortArgs {
+    const float2 *wh;
+    int n_place, n_mov;
+    GeomArgs g;
+    int Mx, My;
+    int32_t *count, *off, *dtab;
+    int level, K;  // super-tile level and cells per block of the density scatter
+    float4 *sorted;
+    int blocks, grid;  // grid: a multiple of the XCDs, 0 for no sort
+};
+
 template <int CPT>
-__global__ __launch_bounds__(kBlock) void k_sort_scatter(Pair<const float2> pos_pair,
-                                                         const float2 *__restrict__ wh, int n_place,
-                                                         int n_mov, GeomArgs g, int Mx, int My,
-                                                         int32_t *__restrict__ count,
-                                                         int32_t *__restrict__ off, int32_t *__restrict__ dtab,
-                                                         int level, int K, float4 *__restrict__ sorted,
-                                                         const DevScalars *__restrict__ sc)
+__device__ inline void sort_scatter(const SortArgs &a, const float2 *__restrict__ pos, int blk)
 {
-    if (sc->halt) return;
-    const float2 *__restrict__ pos = pos_pair.p[sc->sel];
+    const float2 *__restrict__ wh = a.wh;
+    int32_t *__restrict__ count = a.count;
+    float4 *__restrict__ sorted = a.sorted;
+    const int n_place = a.n_place;
     __shared__ int hist[kSortTiles];
     __shared__ int start[kSortTiles + 1];
     const int4 cnt = reinterpret_cast<const int4 *>(count)[threadIdx.x];
     for (int t = threadIdx.x; t < kSortTiles; t += kBlock) hist[t] = 0;
-    const int base = blockIdx.x * kBlock * CPT;
+    const int base = blk * kBlock * CPT;
     int key[CPT], rank[CPT];
     float4 cell[CPT];
     // All of the thread's cells are loaded before the first tile count, so
@@ -110,12 +118,12 @@ __global__ __launch_bounds__(kBlock) void k_sort_scatter(Pair<const float2> pos_
         const int idx = base + k * kBlock + threadIdx.x;
         key[k] = -1;
         if (idx < n_place) {
-            key[k] = cell_key(p[k], s[k], g, Mx, My);
+            key[k] = cell_key(p[k], s[k], a.g, a.Mx, a.My);
             rank[k] = atomicAdd(&hist[key[k]], 1);
-            cell[k] = pack_cell(p[k], s[k], idx < n_mov);
+            cell[k] = pack_cell(p[k], s[k], idx < a.n_mov);
         }
     }
-    if (blockIdx.x == 0) sort_tables(start, off, dtab, level, K);
+    if (blk == 0) sort_tables(start, a.off, a.dtab, a.level, a.K);
     __syncthreads();
     for (int t = threadIdx.x; t < kSortTiles; t += kBlock)
         if (hist[t]) start[t] += atomicAdd(&count[kSortTiles + t], hist[t]);
@@ -135,26 +143,28 @@ __global__ void k_sort_clear(int32_t *__restrict__ count)
 }
 
 // ---- density scatter: block b takes up to kBlock * CPT cells of one super
-// tile (dtab from k_sort_scan) and accumulates them in an LDS window.
+// tile (dtab from the sort) and accumulates them in an LDS window.
+struct DensArgs {
+    const float4 *sorted;
+    const int32_t *off, *dtab;
+    int level, ext, wcap, n_place;
+    GeomArgs g;
+    int Mx, My;
+    unsigned long long *acc_field, *acc_mov;
+    int blocks, grid;  // grid: a multiple of the XCDs, 0 for no scatter
+};
+
 template <int CPT>
-__global__ __launch_bounds__(kBlock) void k_density(const float4 *__restrict__ sorted,
-                                                    const int32_t *__restrict__ off,
-                                                    const int32_t *__restrict__ dtab, int level,
-                                                    int ext, int wcap, int n_place, GeomArgs g,
-                                                    int Mx, int My,
-                                                    unsigned long long *__restrict__ acc_field,
-                                                    unsigned long long *__restrict__ acc_mov,
-                                                    const DevScalars *__restrict__ sc)
+__device__ inline void density_block(const DensArgs &a, int blk)
 {
-    if (sc->halt) return;
-    const int ns = kSortTiles >> (2 * level);
-    const int b = xcd_run_block(blockIdx.x, gridDim.x, kXcdRun);  // neighbouring super tiles share an L2
-    if (b >= dtab[ns]) return;
-    const int s = dens_super_tile(dtab, ns, b);
+    const int ns = kSortTiles >> (2 * a.level);
+    const int b = xcd_run_block(blk, a.blocks, kXcdRun);  // neighbouring super tiles share an L2
+    if (b >= a.dtab[ns]) return;
+    const int s = dens_super_tile(a.dtab, ns, b);
     int c0, c1, x0, y0, nx, ny;
-    dens_cell_range(off, s, level, b - dtab[s], kBlock * CPT, n_place, c0, c1);
-    super_window(s, level, Mx, My, ext, x0, y0, nx, ny);
-    density_window<CPT>(sorted, c0, c1, g, Mx, My, x0, y0, nx, ny, acc_field, acc_mov, wcap);
+    dens_cell_range(a.off, s, a.level, b - a.dtab[s], kBlock * CPT, a.n_place, c0, c1);
+    super_window(s, a.level, a.Mx, a.My, a.ext, x0, y0, nx, ny);
+    density_window<CPT>(a.sorted, c0, c1, a.g, a.Mx, a.My, x0, y0, nx, ny, a.acc_field, a.acc_mov, a.wcap);
 }
 
 // Converts the fixed-point accumulators into the FP32 maps (field map =
@@ -262,37 +272,107 @@ __device__ inline void wa_bucket(const Bucket &bk, int blk, const int32_t *__res
     wa_net<G>(s, e, active, lane, ginv, pin_cell, pin_off, pos, pin_grad, hp, wa);
 }
 
-__global__ __launch_bounds__(kBlock) void k_wa(BucketTable bt, const int32_t *__restrict__ net_start,
-                                               const int32_t *__restrict__ pin_cell,
-                                               const float2 *__restrict__ pin_off,
-                                               Pair<const float2> pos_pair,
-                                               float2 *__restrict__ pin_grad,
-                                               const DevScalars *__restrict__ sc,
-                                               int total_blocks, double *__restrict__ part)
+struct WaArgs {
+    BucketTable bt;
+    const int32_t *net_start, *pin_cell;
+    const float2 *pin_off;
+    float2 *pin_grad;
+    int total_blocks, grid;  // net tiles, and blocks that take them
+    double *part;
+};
+
+__device__ inline void wa_block(const WaArgs &a, const float2 *__restrict__ pos, float ginv, int blk)
 {
-    if (sc->halt) return;
-    const float2 *__restrict__ pos = pos_pair.p[sc->sel];
-    const float ginv = sc->gamma_inv;
+    const int32_t *__restrict__ net_start = a.net_start;
+    const int32_t *__restrict__ pin_cell = a.pin_cell;
+    const float2 *__restrict__ pin_off = a.pin_off;
+    float2 *__restrict__ pin_grad = a.pin_grad;
     double hp = 0.0, wa = 0.0;
     // one net tile per block (virtual blocks if the launch is capped); runs of
     // neighbouring tiles share an XCD's L2
-    for (int vb = xcd_run_block(blockIdx.x, gridDim.x, kXcdRun); vb < total_blocks;
-         vb += gridDim.x) {
+    for (int vb = xcd_run_block(blk, a.grid, kXcdRun); vb < a.total_blocks; vb += a.grid) {
         int b = 0;
-        while (b + 1 < bt.n && vb >= bt.b[b + 1].blk0) ++b;
-        const Bucket bk = bt.b[b];
-        const int blk = vb - bk.blk0;
+        while (b + 1 < a.bt.n && vb >= a.bt.b[b + 1].blk0) ++b;
+        const Bucket bk = a.bt.b[b];
+        const int t = vb - bk.blk0;
         switch (bk.lanes) {
-        case 2: wa_bucket<2>(bk, blk, net_start, pin_cell, pin_off, pos, pin_grad, ginv, hp, wa); break;
-        case 4: wa_bucket<4>(bk, blk, net_start, pin_cell, pin_off, pos, pin_grad, ginv, hp, wa); break;
-        case 8: wa_bucket<8>(bk, blk, net_start, pin_cell, pin_off, pos, pin_grad, ginv, hp, wa); break;
-        case 16: wa_bucket<16>(bk, blk, net_start, pin_cell, pin_off, pos, pin_grad, ginv, hp, wa); break;
-        case 32: wa_bucket<32>(bk, blk, net_start, pin_cell, pin_off, pos, pin_grad, ginv, hp, wa); break;
-        default: wa_bucket<64>(bk, blk, net_start, pin_cell, pin_off, pos, pin_grad, ginv, hp, wa); break;
+        case 2: wa_bucket<2>(bk, t, net_start, pin_cell, pin_off, pos, pin_grad, ginv, hp, wa); break;
+        case 4: wa_bucket<4>(bk, t, net_start, pin_cell, pin_off, pos, pin_grad, ginv, hp, wa); break;
+        case 8: wa_bucket<8>(bk, t, net_start, pin_cell, pin_off, pos, pin_grad, ginv, hp, wa); break;
+        case 16: wa_bucket<16>(bk, t, net_start, pin_cell, pin_off, pos, pin_grad, ginv, hp, wa); break;
+        case 32: wa_bucket<32>(bk, t, net_start, pin_cell, pin_off, pos, pin_grad, ginv, hp, wa); break;
+        default: wa_bucket<64>(bk, t, net_start, pin_cell, pin_off, pos, pin_grad, ginv, hp, wa); break;
         }
     }
     double v[2] = {hp, wa};
-    block_reduce<2, 0>(v, part + 2 * blockIdx.x);
+    block_reduce<2, 0>(v, a.part + 2 * blk);
+}
+
+__global__ __launch_bounds__(kBlock) void k_wa(Pair<const float2> pos_pair, WaArgs w, const DevScalars *__restrict__ sc)
+{
+    if (sc->halt) return;
+    wa_block(w, pos_pair.p[sc->sel], sc->gamma_inv, blockIdx.x);
+}
+
+template <int CPT>
+__global__ __launch_bounds__(kBlock) void k_sort_scatter(Pair<const float2> pos_pair, SortArgs a,
+                                                         const DevScalars *__restrict__ sc)
+{
+    if (sc->halt) return;
+    sort_scatter<CPT>(a, pos_pair.p[sc->sel], blockIdx.x);
+}
+
+// The tile sort's scatter pass and the WA gradient, which need only the positions,
+// in one launch: the first blocks sort, the others take net tiles.  Neither fills
+// the chip alone below about a million cells.  Eight waves a SIMD as the net tiles
+// have alone: the gathers' latency is what bounds them.  With the pin sums beside the
+// density scatter, us per evaluation before and after: 576 cells 44.9 / 40.8, 20k
+// 57.8 / 50.7, 200k 88.6 / 82.4.
+template <int CPT>
+__global__ __launch_bounds__(kBlock, 8) void k_sort_wa(Pair<const float2> pos_pair, SortArgs a, WaArgs w,
+                                                       const DevScalars *__restrict__ sc)
+{
+    if (sc->halt) return;
+    const float2 *__restrict__ pos = pos_pair.p[sc->sel];
+    if ((int)blockIdx.x >= a.grid) wa_block(w, pos, sc->gamma_inv, blockIdx.x - a.grid);
+    else if ((int)blockIdx.x < a.blocks) sort_scatter<CPT>(a, pos, blockIdx.x);
+}
+
+struct PinArgs {
+    const int32_t *start, *pins;  // cell -> pin CSR
+    const float2 *pin_grad;
+    int n_mov, grid;
+    float2 *gw_cell;
+};
+
+// Per movable cell the sum of its pin partials (the cell gradient reads it).
+__device__ inline void pin_block(const PinArgs &a, int blk)
+{
+    for (int c = xcd_block(blk, a.grid) * kBlock + threadIdx.x; c < a.n_mov; c += a.grid * kBlock)
+        a.gw_cell[c] = sum_pin_partials(a.start[c], a.start[c + 1], a.pins, a.pin_grad);
+}
+
+__global__ __launch_bounds__(kBlock) void k_pin_sum(PinArgs p, const DevScalars *__restrict__ sc)
+{
+    if (sc->halt) return;
+    pin_block(p, blockIdx.x);
+}
+
+template <int CPT>
+__global__ __launch_bounds__(kBlock) void k_density(DensArgs d, const DevScalars *__restrict__ sc)
+{
+    if (sc->halt) return;
+    density_block<CPT>(d, blockIdx.x);
+}
+
+// The density scatter and the pin sums in one launch: the first blocks scatter,
+// the others sum.
+template <int CPT>
+__global__ __launch_bounds__(kBlock) void k_density_pins(DensArgs d, PinArgs p, const DevScalars *__restrict__ sc)
+{
+    if (sc->halt) return;
+    if ((int)blockIdx.x >= d.grid) pin_block(p, blockIdx.x - d.grid);
+    else if ((int)blockIdx.x < d.blocks) density_block<CPT>(d, blockIdx.x);
 }
 
 // ------------------------------------------------------------------ reference packet format
@@ -391,14 +471,13 @@ __global__ void k_wa_packet_fast64(const float *__restrict__ data, int net_size,
 
 // g = (gW - lambda * F) / max(1, pins + lambda * area); F = r * sum ov * E over
 // the smoothed rectangle.  Also the FP64 partial norms for the step length.
-// kVref / kGref / kGwCell: whether vref_pair, gref_pair and gw_cell are set.
-// As compile-time flags they leave the loads of a cell in one basic block,
-// so they are in flight together.
-template <bool kVref, bool kGref, bool kGwCell>
+// kVref / kGref: whether vref_pair and gref_pair are set.  As compile-time flags
+// they leave the loads of a cell in one basic block, so they are in flight
+// together.
+template <bool kVref, bool kGref>
 __global__ __launch_bounds__(kBlock) void k_cell_grad(
     Pair<const float2> pos_pair, const float2 *__restrict__ wh, int n_place, int n_mov,
     GeomArgs g, int Mx, int My, const int32_t *__restrict__ cell_pin_start,
-    const int32_t *__restrict__ cell_pins, const float2 *__restrict__ pin_grad,
     const float2 *__restrict__ exy, Pair<const float2> vref_pair,
     Pair<const float2> gref_pair, Pair<float2> gout_pair, float2 *__restrict__ gw_out,
     float2 *__restrict__ f_out, const DevScalars *__restrict__ sc, double *__restrict__ part,
@@ -421,12 +500,10 @@ __global__ __launch_bounds__(kBlock) void k_cell_grad(
         // n_mov + 1 entries, so a fixed cell or filler reads k0 == k1 (no pins).
         const bool mov = c < n_mov;
         const int k0 = cell_pin_start[min(c, n_mov)], k1 = cell_pin_start[min(c + 1, n_mov)];
-        float2 gwc = make_float2(0.f, 0.f);
-        if (kGwCell) gwc = gw_cell[max(0, min(c, n_mov - 1))];  // holds max(1, n_mov) entries
+        const float2 gwc = gw_cell[max(0, min(c, n_mov - 1))];  // holds max(1, n_mov) entries
         const int np = k1 - k0;
         const float2 f = cell_force(p, s, exy, g, Mx, My);
-        const float2 gw = kGwCell ? (mov ? gwc : make_float2(0.f, 0.f))
-                                  : sum_pin_partials(k0, k1, cell_pins, pin_grad);
+        const float2 gw = mov ? gwc : make_float2(0.f, 0.f);
         const float gwx = gw.x, gwy = gw.y, fx = f.x, fy = f.y;
         const float pre = fmaxf(1.0f, __fmaf_rn(lambda * s.x, s.y, (float)np));
         const float gx = __fmaf_rn(-lambda, fx, gwx) / pre, gy = __fmaf_rn(-lambda, fy, gwy) / pre;
@@ -456,21 +533,6 @@ __global__ __launch_bounds__(kBlock) void k_cell_grad(
         if (c + stride < n_place) one(c + stride);
     }
     block_reduce<7, 1>(acc, part + 7 * blockIdx.x);
-}
-
-// Per movable cell, the sum of its pin partials (what k_cell_grad gathers
-// itself when it gets no gw_cell): lets the gather run beside the transform
-// products, off the path to the field.
-__global__ __launch_bounds__(kBlock) void k_pin_sum(const int32_t *__restrict__ cell_pin_start,
-                                                   const int32_t *__restrict__ cell_pins,
-                                                   const float2 *__restrict__ pin_grad, int n_mov,
-                                                   float2 *__restrict__ gw_cell,
-                                                   const DevScalars *__restrict__ sc)
-{
-    if (sc->halt) return;
-    for (int c = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x; c < n_mov;
-         c += gridDim.x * kBlock)
-        gw_cell[c] = sum_pin_partials(cell_pin_start[c], cell_pin_start[c + 1], cell_pins, pin_grad);
 }
 
 // Deterministic final reduction of all partial sums, in a fixed order.  kBlocks =
@@ -966,32 +1028,101 @@ void launch_sort_clear(Ctx &c, hipStream_t s)
     hipLaunchKernelGGL(k_sort_clear, dim3(1), dim3(kBlock), 0, s, c.sort_count);
 }
 
-void launch_sort(Ctx &c, Pair<const float2> pos, bool counted, hipStream_t s)
+namespace {
+
+int pad_xcds(int blocks) { return (blocks + kXcds - 1) / kXcds * kXcds; }
+
+// `beside`: the blocks share a launch with others, which begin at a multiple of the XCDs
+SortArgs sort_args(const Ctx &c, int cpt, bool beside)
+{
+    const int blocks = (int)(((int64_t)c.n_place + kBlock * cpt - 1) / (kBlock * cpt));
+    return {c.wh, c.n_place, c.n_mov, geom_args(c), c.Mx, c.My, c.sort_count, c.sort_off, c.dens_tab, c.dens.level,
+            kBlock * c.dens.cpt, c.sorted, blocks, beside ? pad_xcds(blocks) : blocks};
+}
+
+WaArgs wa_args(const Ctx &c)
+{
+    return {c.buckets, c.net_start, c.pin_cell, c.pin_off, c.pin_grad, c.wa_blocks,
+            c.wa_blocks ? c.wa_part_blocks : 0, c.part + c.part_wa_off};
+}
+
+DensArgs dens_args(const Ctx &c, bool beside)
+{
+    const int blocks = dens_grid(c.dens, c.n_place);
+    return {c.sorted, c.sort_off, c.dens_tab, c.dens.level, c.dens.ext, c.dens.wcap, c.n_place, geom_args(c),
+            c.Mx, c.My, c.acc_field, c.acc_mov, blocks, beside ? pad_xcds(blocks) : blocks};
+}
+
+PinArgs pin_args(const Ctx &c)
+{
+    const int grid = c.n_mov ? grid_for(c.n_mov, kBlock, kCellGridCap) : 0;
+    return {c.cell_pin_start, c.cell_pins, c.pin_grad, c.n_mov, grid, c.gw_cell};
+}
+
+}  // namespace
+
+void launch_sort_count(Ctx &c, Pair<const float2> pos, hipStream_t s)
 {
     with_sort_cpt(c.sort_cpt, [&](auto cpt) {
-        constexpr int CPT = decltype(cpt)::value;
-        if (!counted)
-            hipLaunchKernelGGL(k_sort_count<CPT>, dim3(c.trial_blocks), dim3(kBlock), 0, s, pos, c.wh, c.n_place,
-                               geom_args(c), c.Mx, c.My, c.sort_count, c.d_scal);
-        hipLaunchKernelGGL(k_sort_scatter<CPT>, dim3(c.trial_blocks), dim3(kBlock), 0, s, pos, c.wh, c.n_place,
-                           c.n_mov, geom_args(c), c.Mx, c.My, c.sort_count, c.sort_off, c.dens_tab, c.dens.level,
-                           kBlock * c.dens.cpt, c.sorted, c.d_scal);
+        hipLaunchKernelGGL(k_sort_count<decltype(cpt)::value>, dim3(c.trial_blocks), dim3(kBlock), 0, s, pos, c.wh,
+                           c.n_place, geom_args(c), c.Mx, c.My, c.sort_count, c.d_scal);
     });
+}
+
+void launch_sort(Ctx &c, Pair<const float2> pos, hipStream_t s)
+{
+    const SortArgs a = sort_args(c, c.sort_cpt, false);
+    with_sort_cpt(c.sort_cpt, [&](auto t) {
+        hipLaunchKernelGGL(k_sort_scatter<decltype(t)::value>, dim3(a.grid), dim3(kBlock), 0, s, pos, a, c.d_scal);
+    });
+}
+
+void launch_wa(Ctx &c, Pair<const float2> pos, hipStream_t s)
+{
+    const WaArgs w = wa_args(c);
+    if (w.grid) hipLaunchKernelGGL(k_wa, dim3(w.grid), dim3(kBlock), 0, s, pos, w, c.d_scal);
+}
+
+void launch_sort_wa(Ctx &c, Pair<const float2> pos, hipStream_t s)
+{
+    const int cpt = std::min(c.sort_cpt, kSortWaMost);
+    const SortArgs a = sort_args(c, cpt, true);
+    const WaArgs w = wa_args(c);
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(a.grid + w.grid), dim3(kBlock), 0, s, pos, a, w, c.d_scal);
+    };
+    if (cpt == 1) go(k_sort_wa<1>);
+    else if (cpt == 2) go(k_sort_wa<2>);
+    else go(k_sort_wa<kSortWaMost>);
 }
 
 void launch_density(Ctx &c, hipStream_t s)
 {
-    const DensPlan &dp = c.dens;
-    const int blocks = dens_grid(dp, c.n_place);
-    const size_t lds = dens_lds_bytes(dp);
+    const DensArgs d = dens_args(c, false);
     auto go = [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3(blocks), dim3(kBlock), lds, s, c.sorted, c.sort_off, c.dens_tab,
-                           dp.level, dp.ext, dp.wcap, c.n_place, geom_args(c), c.Mx, c.My,
-                           c.acc_field, c.acc_mov, c.d_scal);
+        hipLaunchKernelGGL(kern, dim3(d.grid), dim3(kBlock), dens_lds_bytes(c.dens), s, d, c.d_scal);
     };
-    if (dp.cpt == 1) go(k_density<1>);
-    else if (dp.cpt == 2) go(k_density<2>);
+    if (c.dens.cpt == 1) go(k_density<1>);
+    else if (c.dens.cpt == 2) go(k_density<2>);
     else go(k_density<4>);
+}
+
+void launch_pin_sum(Ctx &c, hipStream_t s)
+{
+    const PinArgs p = pin_args(c);
+    if (p.grid) hipLaunchKernelGGL(k_pin_sum, dim3(p.grid), dim3(kBlock), 0, s, p, c.d_scal);
+}
+
+void launch_density_pins(Ctx &c, hipStream_t s)
+{
+    const DensArgs d = dens_args(c, true);
+    const PinArgs p = pin_args(c);
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(d.grid + p.grid), dim3(kBlock), dens_lds_bytes(c.dens), s, d, p, c.d_scal);
+    };
+    if (c.dens.cpt == 1) go(k_density_pins<1>);
+    else if (c.dens.cpt == 2) go(k_density_pins<2>);
+    else go(k_density_pins<4>);
 }
 
 void launch_overflow(Ctx &c, hipStream_t s)
@@ -1010,40 +1141,21 @@ void launch_map_range(Ctx &c, hipStream_t s)
                        c.map_mean, c.field_max, c.d_scal);
 }
 
-void launch_wa(Ctx &c, Pair<const float2> pos, hipStream_t s)
-{
-    if (c.wa_blocks == 0) return;
-    hipLaunchKernelGGL(k_wa, dim3(c.wa_part_blocks), dim3(kBlock), 0, s, c.buckets, c.net_start,
-                       c.pin_cell, c.pin_off, pos, c.pin_grad, c.d_scal, c.wa_blocks,
-                       c.part + c.part_wa_off);
-}
-
-void launch_pin_sum(Ctx &c, hipStream_t s)
-{
-    if (c.n_mov == 0) return;
-    hipLaunchKernelGGL(k_pin_sum, dim3(grid_for(c.n_mov, kBlock, kCellGridCap)), dim3(kBlock), 0, s,
-                       c.cell_pin_start, c.cell_pins, c.pin_grad, c.n_mov, c.gw_cell, c.d_scal);
-}
-
 void launch_cell_grad(Ctx &c, Pair<const float2> pos, Pair<const float2> vref,
                       Pair<const float2> gref, Pair<float2> gout, float2 *gw_out, float2 *f_out,
-                      hipStream_t s, const float2 *gw_cell)
+                      hipStream_t s)
 {
     // Every caller sets both entries of a pair or neither.
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3(c.cell_blocks), dim3(kBlock), 0, s, pos, c.wh, c.n_place, c.n_mov,
-                           geom_args(c), c.Mx, c.My, c.cell_pin_start, c.cell_pins, c.pin_grad, c.exy,
-                           vref, gref, gout, gw_out, f_out, c.d_scal, c.part + c.part_cell_off, gw_cell);
+                           geom_args(c), c.Mx, c.My, c.cell_pin_start, c.exy, vref, gref, gout, gw_out, f_out, c.d_scal,
+                           c.part + c.part_cell_off, c.gw_cell);
     };
-    switch ((vref.p[0] ? 1 : 0) | (gref.p[0] ? 2 : 0) | (gw_cell ? 4 : 0)) {
-    case 0: go(k_cell_grad<false, false, false>); break;
-    case 1: go(k_cell_grad<true, false, false>); break;
-    case 2: go(k_cell_grad<false, true, false>); break;
-    case 3: go(k_cell_grad<true, true, false>); break;
-    case 4: go(k_cell_grad<false, false, true>); break;
-    case 5: go(k_cell_grad<true, false, true>); break;
-    case 6: go(k_cell_grad<false, true, true>); break;
-    default: go(k_cell_grad<true, true, true>); break;
+    switch ((vref.p[0] ? 1 : 0) | (gref.p[0] ? 2 : 0)) {
+    case 0: go(k_cell_grad<false, false>); break;
+    case 1: go(k_cell_grad<true, false>); break;
+    case 2: go(k_cell_grad<false, true>); break;
+    default: go(k_cell_grad<true, true>); break;
     }
 }
 

@@ -43,7 +43,9 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 PROFILES = os.path.join(ROOT, "profiles")
 PREC_NAME = {0: "fp32", 1: "bf16x3", 2: "fp16x3"}
 # kernel families of one gradient evaluation (name prefix -> ep_profile item)
+# (two items in one launch belong to neither; ep_profile times each alone)
 FAMILIES = [
+    ("k_sort_wa", None), ("k_density_pins", None), ("k_fft_", "field_transforms"),
     ("k_sort_", "cell_sort"), ("k_density", "density_scatter"), ("k_overflow", "overflow"),
     ("k_map_stats", "overflow"), ("k_wa", "wa_grad"), ("k_sym_", "field_transforms"),
     ("k_clear_max", "field_transforms"), ("k_pin_sum", "pin_sum"), ("k_cell_grad", "cell_grad"),
@@ -160,10 +162,11 @@ def stats(args) -> str:
              "Command (from the repository root):", "", "```", _cmd_text(full),
              "```", "",
              f"One full placement (graph replays) followed by {args.reps} ep_profile repetitions of each "
-             "kernel at the final placement.  In the placement the WA gradient and the per-cell pin sums "
+             "kernel at the final placement.  In a large placement the WA gradient and the per-cell pin sums "
              "(k_wa, k_pin_sum) run on a second captured branch beside the density scatter and the "
-             "transform products, so those kernels' durations include the sharing of the CUs and the "
-             "shares add up to more than the wall time; ep_profile (below) times each item alone.", ""]
+             "transforms, so those kernels' durations include the sharing of the CUs and the "
+             "shares add up to more than the wall time; a smaller one runs them in one launch with the "
+             "sort and the scatter (k_sort_wa, k_density_pins).  ep_profile (below) times each item alone.", ""]
     if res:
         r = res["run"]
         lines += [f"Run: {r['iterations']} iterations, {r['evals']} gradient evaluations, "

@@ -88,7 +88,8 @@ typedef struct ep_params {
                                  the backtracking condition (fallback to the search) */
     int32_t fork_min_cells;   /* captured evaluations run the WA gradient on a second
                                  branch from this many placeable cells on (results are
-                                 identical either way); 0 = the default, 400000     */
+                                 identical either way); 0 = the default, 800000
+                                 (a batch: 400000 cells of running instances)       */
     int32_t cell_order;       /* 1 (default): movable cells stored in breadth-first order
                                  over the netlist, so that cells of one net sit at nearby
                                  indices (gather locality for netlists in any order);
@@ -192,10 +193,11 @@ ep_status ep_set_precision(ep_ctx *ctx, int32_t precision);
  * Times each kernel group of one gradient evaluation at the current state with
  * HIP events on the context's stream, `reps` launches each, and reports the
  * algorithmic HBM bytes and flops of one launch.  Groups: cell_sort,
- * density_scatter, overflow, wa_grad, field_transforms, [pin_sum,] cell_grad,
- * nesterov_trial, finalize, then the scatter at other cells per thread; contexts
- * that fork their captured evaluation (fork_min_cells) report pin_sum and a
- * cell_grad that reads its sums, as the graph runs them. */
+ * density_scatter, overflow, wa_grad, field_transforms, pin_sum, cell_grad,
+ * nesterov_trial, finalize, then the scatter at other cells per thread.  Each is
+ * timed by itself; an evaluation runs cell_sort's scatter pass and wa_grad, and
+ * density_scatter and pin_sum, in one launch each, or on two branches
+ * (fork_min_cells). */
 typedef struct ep_kernel_stat {
     char name[32];
     int32_t launches;   /* launches of this group per gradient evaluation        */
