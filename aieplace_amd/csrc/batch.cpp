@@ -80,7 +80,7 @@ struct ep_batch {
     BRes *d_res = nullptr;
     float2 *wh = nullptr, *V[2] = {}, *U[2] = {}, *G[2] = {};
     int32_t *net_start = nullptr, *pin_cell = nullptr, *cps = nullptr, *cpins = nullptr;
-    float2 *pin_off = nullptr, *pin_grad = nullptr;
+    float2 *pin_off = nullptr, *pin_grad = nullptr, *gw = nullptr;
     float *map_field = nullptr, *map_mov = nullptr, *map_fix = nullptr;
     float2 *exy = nullptr;
     float *tA = nullptr, *tB = nullptr, *map_mean = nullptr;
@@ -134,6 +134,7 @@ struct ep_batch {
         d.pin_cell = pin_cell;
         d.pin_off = pin_off;
         d.pin_grad = pin_grad;
+        d.gw = gw;
         d.cps = cps;
         d.cpins = cpins;
         d.map_field = map_field;
@@ -171,23 +172,34 @@ struct ep_batch {
         return n_cells;
     }
 
+    // Density maps of every unfinished instance at its current positions.
+    void maps_at_cur()
+    {
+        const BDev d = dev();
+        const int v = dens_variant;
+        bl_sort_count(d, kAtCur, sort_blocks, stream);
+        bl_sort(d, kAtCur, sort_blocks, kDensCpt[v], stream);
+        bl_density(d, dens_blocks[v], kDensCpt[v], stream);
+        bl_overflow(d, bin_blocks, f16(), stream);
+    }
+
     // One gradient evaluation as a captured fork: the tile sort, the density
-    // scatter and the transform products on the side stream beside the WA
-    // gradient (the captured stream of the longer branch decides how soon it
-    // starts), as in the single-instance graph.
-    hipError_t eval_forked(const BDev &d, int at, bool counted, hipStream_t s, int ctl_mode)
+    // scatter and the transforms on the side stream beside the WA gradient (the
+    // captured stream of the longer branch decides how soon it starts).
+    hipError_t eval_forked(const BDev &d, int at, hipStream_t s, int ctl_mode)
     {
         const int v = dens_variant;
         hipError_t e = hipEventRecord(fork, s);
         if (e == hipSuccess) e = hipStreamWaitEvent(side, fork, 0);
         if (e != hipSuccess) return e;
-        bl_sort(d, at, counted, bin_blocks, sort_blocks, kDensCpt[v], side);
-        bl_dens(d, bin_blocks, dens_blocks[v], kDensCpt[v], f16(), side);
+        bl_sort(d, at, sort_blocks, kDensCpt[v], side);
+        bl_density(d, dens_blocks[v], kDensCpt[v], side);
+        bl_overflow(d, bin_blocks, f16(), side);
         launch_field_batch(bf, prm.precision, side);
         if ((e = hipEventRecord(join, side)) != hipSuccess) return e;
         bl_wa(d, at, wa_blocks, s);
         if ((e = hipStreamWaitEvent(s, join, 0)) != hipSuccess) return e;
-        bl_cell_grad(d, at, cell_blocks, s);
+        bl_cell_grad(d, at, false, cell_blocks, s);
         bl_reduce_control(d, ctl_mode, s);
         return hipSuccess;
     }
@@ -197,11 +209,13 @@ struct ep_batch {
     // the control step `ctl_mode` on them.
     void eval(const BDev &d, int at, bool counted, hipStream_t s, int ctl_mode)
     {
-        bl_maps(d, at, counted, bin_blocks, sort_blocks, dens_blocks[dens_variant],
-                kDensCpt[dens_variant], f16(), s);
-        bl_wa(d, at, wa_blocks, s);
+        const int v = dens_variant;
+        if (!counted) bl_sort_count(d, at, sort_blocks, s);
+        bl_sort_wa(d, at, sort_blocks, kDensCpt[v], wa_blocks, s);
+        bl_density_pins(d, dens_blocks[v], kDensCpt[v], cell_blocks, s);
+        bl_overflow(d, bin_blocks, f16(), s);
         launch_field_batch(bf, prm.precision, s);
-        bl_cell_grad(d, at, cell_blocks, s);
+        bl_cell_grad(d, at, true, cell_blocks, s);
         bl_reduce_control(d, ctl_mode, s);
     }
 };
@@ -212,7 +226,7 @@ static void destroy_batch(ep_batch *b)
     if (b->exec) (void)hipGraphExecDestroy(b->exec);
     void *ptrs[] = {b->d_inst, b->d_st, b->d_res, b->wh, b->V[0], b->V[1], b->U[0], b->U[1],
                     b->G[0], b->G[1], b->net_start, b->pin_cell, b->cps, b->cpins, b->pin_off,
-                    b->pin_grad, b->map_field, b->map_mov, b->map_fix, b->acc_field, b->acc_mov, b->exy, b->tA, b->tB,
+                    b->pin_grad, b->gw, b->map_field, b->map_mov, b->map_fix, b->acc_field, b->acc_mov, b->exy, b->tA, b->tB,
                     b->map_mean, b->map_max, b->sorted, b->sort_count, b->sort_off, b->dens_tab, b->pre_cell,
                     b->pre_sort, b->pre_bin, b->pre_wa, b->pre_dens[0], b->pre_dens[1],
                     b->pre_dens[2], b->buckets, b->part_wa, b->part_ovf, b->part_cell, b->init_pos, b->stored};
@@ -323,13 +337,9 @@ static ep_status autotune(ep_batch *b)
     int best_v = 1;
     for (int v = 0; v < 3; ++v) {
         b->dens_variant = v;
-        const BDev d = b->dev();
-        bl_maps(d, kAtCur, false, b->bin_blocks, b->sort_blocks, b->dens_blocks[v], kDensCpt[v], b->f16(),
-                b->stream);
+        b->maps_at_cur();
         (void)hipEventRecord(e0, b->stream);
-        for (int r = 0; r < kTuneReps; ++r)
-            bl_maps(d, kAtCur, false, b->bin_blocks, b->sort_blocks, b->dens_blocks[v], kDensCpt[v], b->f16(),
-                    b->stream);
+        for (int r = 0; r < kTuneReps; ++r) b->maps_at_cur();
         (void)hipEventRecord(e1, b->stream);
         hipError_t e = hipEventSynchronize(e1);
         if (e != hipSuccess) {
@@ -523,6 +533,7 @@ extern "C" ep_status ep_batch_create(const ep_netlist *const *nls, const int32_t
     EPB_TRY(dalloc(&b->pin_cell, pin_cell.size()));
     EPB_TRY(dalloc(&b->pin_off, pin_off.size()));
     EPB_TRY(dalloc(&b->pin_grad, pin_cell.size()));
+    EPB_TRY(dalloc(&b->gw, nc));
     EPB_TRY(dalloc(&b->cps, cps.size()));
     EPB_TRY(dalloc(&b->cpins, cpins.size()));
     EPB_TRY(dalloc(&b->map_field, nb));
@@ -643,16 +654,15 @@ extern "C" ep_status ep_batch_init(ep_batch *b)
     hipStream_t s = b->stream;
     b->st_current = false;
     bl_move(d, kMoveInitU, b->sort_blocks, s);
-    bl_maps(d, kAtCur, false, b->bin_blocks, b->sort_blocks, b->dens_blocks[b->dens_variant],
-            kDensCpt[b->dens_variant], b->f16(), s);
+    b->maps_at_cur();
     bl_reduce_control(d, kCtlGamma, s);
     // gradient pieces at v_0 with lambda = 0: |gW|_1 and |F|_1
     bl_wa(d, kAtCur, b->wa_blocks, s);
     launch_field_batch(b->bf, b->prm.precision, s);
-    bl_cell_grad(d, kAtCur, b->cell_blocks, s);
+    bl_cell_grad(d, kAtCur, false, b->cell_blocks, s);
     bl_reduce_control(d, kCtlLambda, s);
     // preconditioned gradient with lambda_0, then the probe displacement
-    bl_cell_grad(d, kAtCur, b->cell_blocks, s);
+    bl_cell_grad(d, kAtCur, false, b->cell_blocks, s);
     bl_reduce_control(d, kCtlProbe, s);
     bl_move(d, kMoveProbe, b->sort_blocks, s);
     b->eval(d, kAtTrial, false, s, kCtlAlpha);
@@ -677,8 +687,8 @@ static ep_status build_graph(ep_batch *b)
     hipError_t e = hipSuccess;
     for (int t = 0; t < kTrialsPerLaunch && e == hipSuccess; ++t) {
         bl_move(d, kMoveTrial, b->sort_blocks, b->stream);
-        if (b->active_cells() >= fork_min_cells(b->prm, kForkMinCellsBatch))
-            e = b->eval_forked(d, kAtTrial, true, b->stream, kCtlIterate);
+        if (b->active_cells() >= fork_min_cells(b->prm))
+            e = b->eval_forked(d, kAtTrial, b->stream, kCtlIterate);
         else b->eval(d, kAtTrial, true, b->stream, kCtlIterate);
     }
     if (e == hipSuccess) e = hipGetLastError();

@@ -1279,7 +1279,7 @@ static ep_status build_ctl_graph(ep_ctx *c, const CtlParams &p)
         // the model's proposal for this trial was made by the previous decision
         // (k_finalize) or by k_step_begin
         launch_trial(x, vc, uc, gc, vn, un, true, s);
-        if (x.n_place >= fork_min_cells(x.prm, kForkMinCells)) {
+        if (x.n_place >= fork_min_cells(x.prm)) {
             // fork right after the trial: the tile sort, the density scatter and
             // the transforms on the second stream (the critical chain), the WA
             // gradient and the per-cell pin sums beside them

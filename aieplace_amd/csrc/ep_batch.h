@@ -84,6 +84,7 @@ struct BDev {
     const float2 *pin_off;
     float2 *pin_grad;
     const int32_t *cps, *cpins;  // global cell -> pin CSR (empty for non-movable cells)
+    float2 *gw;                  // per movable cell the sum of its pin partials
     float *map_field, *map_mov, *map_fix;
     float2 *exy;                 // field (ex, ey) per bin
     unsigned long long *acc_field, *acc_mov;  // fixed-point scatter targets (2^32 per bin area)
@@ -114,18 +115,21 @@ enum BMoveMode { kMoveTrial = 0, kMoveProbe = 1, kMoveInitU = 2 };
 void bl_move(const BDev &d, int mode, int sort_blocks, hipStream_t s);
 // Every instance at the positions `pos` (all cells), gradients and states cleared.
 void bl_reset(const BDev &d, const float2 *pos, int64_t cells, hipStream_t s);
-// Density maps of every unfinished instance; `counted`: a kMoveTrial move made
-// the sort counts at the evaluated positions.
-// bl_maps = bl_sort (tile sort) then bl_dens (scatter; overflow, which also
-// clears the accumulators; with `map_range`, the field-map range that the
-// split-FP16 products scale by).  The accumulators start cleared at creation.
-void bl_sort(const BDev &d, int at, bool counted, int bin_blocks, int sort_blocks, int dens_cpt,
-             hipStream_t s);
-void bl_dens(const BDev &d, int bin_blocks, int dens_blocks, int dens_cpt, bool map_range, hipStream_t s);
-void bl_maps(const BDev &d, int at, bool counted, int bin_blocks, int sort_blocks, int dens_blocks,
-             int dens_cpt, bool map_range, hipStream_t s);
+// Density maps of every unfinished instance: the sort's counts (made by a kMoveTrial
+// move or bl_sort_count), the tile sort, the scatter, and the overflow pass, which also
+// clears the accumulators (they start cleared at creation) and, with `map_range`, finds
+// the field-map range that the split-FP16 products scale by.  bl_sort_wa and
+// bl_density_pins run two of them in one launch.
+void bl_sort_count(const BDev &d, int at, int sort_blocks, hipStream_t s);
+void bl_sort(const BDev &d, int at, int sort_blocks, int dens_cpt, hipStream_t s);
 void bl_wa(const BDev &d, int at, int wa_blocks, hipStream_t s);
-void bl_cell_grad(const BDev &d, int at, int cell_blocks, hipStream_t s);
+void bl_sort_wa(const BDev &d, int at, int sort_blocks, int dens_cpt, int wa_blocks, hipStream_t s);
+void bl_density(const BDev &d, int dens_blocks, int dens_cpt, hipStream_t s);
+void bl_density_pins(const BDev &d, int dens_blocks, int dens_cpt, int cell_blocks, hipStream_t s);
+void bl_overflow(const BDev &d, int bin_blocks, bool map_range, hipStream_t s);
+// Per-cell gradients from the pin sums of bl_density_pins, or (`sums` unset) from the
+// pin partials.
+void bl_cell_grad(const BDev &d, int at, bool sums, int cell_blocks, hipStream_t s);
 // The per-instance FP64 reductions of an evaluation, then the control step
 // `mode` (BCtlMode) of every unfinished instance on them.
 void bl_reduce_control(const BDev &d, int mode, hipStream_t s);

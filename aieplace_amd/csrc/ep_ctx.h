@@ -89,12 +89,13 @@ constexpr int kModelBackoffMax = 32;
 // idle.  A large one's kernels fill the chip; its branches overlap the gathers with the
 // transforms too.  us per evaluation, two branches / shared launches (before those: one
 // branch of single kernels): 383k placeable cells 90.7 / 84.6 (93.4), 643k 134.3 / 133.5
-// (145), 1.28M 173 / 179 (193), 2.56M 271 / 295 (302).
+// (145), 1.28M 173 / 179 (193), 2.56M 271 / 295 (302).  A batch's running instances
+// count together; 100 iterations in ms: 16 instances (358k movable cells) 12.0 / 11.5
+// (12.3), 24 (513k) 13.9 / 13.9 (15.0), 32 (1.6M) 28.7 / 31.9 (32.7).
 constexpr int64_t kForkMinCells = 800000;
-constexpr int64_t kForkMinCellsBatch = 400000;  // of a batch's running instances
-inline int64_t fork_min_cells(const ep_params &p, int64_t most)
+inline int64_t fork_min_cells(const ep_params &p)
 {
-    return p.fork_min_cells > 0 ? (int64_t)p.fork_min_cells : most;
+    return p.fork_min_cells > 0 ? (int64_t)p.fork_min_cells : kForkMinCells;
 }
 // Step-model records kept per context between ep_take_step_records calls.
 constexpr size_t kMaxStepRecords = (size_t)1 << 21;

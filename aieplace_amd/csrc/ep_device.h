@@ -14,6 +14,7 @@ namespace ep {
 namespace dev {
 
 constexpr int kXcds = 8;  // MI355X: 8 XCDs, each with its own L2
+inline int pad_xcds(int blocks) { return (blocks + kXcds - 1) / kXcds * kXcds; }
 
 // Workgroups are dispatched to the XCDs round-robin (physical block b runs on
 // XCD b % 8).  Returns the logical block of physical block b in a grid of n so

@@ -178,14 +178,14 @@ __global__ __launch_bounds__(kBlock) void kb_sort_count(BDev d, int at)
         if (hist[t]) atomicAdd(&count[t], hist[t]);
 }
 
-// As k_sort_scatter; the instance's first block leaves its density tables (K cells
-// per density block).
+// As sort_scatter of a single instance; the instance's first block leaves its density
+// tables (K cells per density block).
 template <int CPT>
-__global__ __launch_bounds__(kBlock) void kb_sort_scatter(BDev d, int at, int K)
+__device__ inline void sort_scatter(const BDev &d, int at, int K, int blk)
 {
     __shared__ int hist[kSortTiles];
     __shared__ int start[kSortTiles + 1];
-    const int i = find_inst(d.pre_sort, d.n_inst, blockIdx.x);
+    const int i = find_inst(d.pre_sort, d.n_inst, blk);
     const BState *S = d.st + i;
     if (S->done) return;
     const BInst &I = d.inst[i];
@@ -194,7 +194,7 @@ __global__ __launch_bounds__(kBlock) void kb_sort_scatter(BDev d, int at, int K)
     int32_t *count = d.sort_count + (size_t)i * 2 * kSortTiles;
     const int4 cnt = reinterpret_cast<const int4 *>(count)[threadIdx.x];
     for (int t = threadIdx.x; t < kSortTiles; t += kBlock) hist[t] = 0;
-    const int base = (blockIdx.x - d.pre_sort[i]) * kBlock * CPT;
+    const int base = (blk - d.pre_sort[i]) * kBlock * CPT;
     int key[CPT], rank[CPT];
     float4 cell[CPT];
     // All of the thread's cells are loaded before the first tile count; a
@@ -233,12 +233,13 @@ __global__ __launch_bounds__(kBlock) void kb_sort_scatter(BDev d, int at, int K)
         }
 }
 
-// Density scatter (as k_density): the instance's blocks take up to kBlock * CPT
-// packed cells of one super tile each and accumulate them in an LDS window.
+// Density scatter (as density_block of a single instance): the instance's blocks take
+// up to kBlock * CPT packed cells of one super tile each and accumulate them in an LDS
+// window.
 template <int CPT>
-__global__ __launch_bounds__(kBlock) void kb_density(BDev d)
+__device__ inline void density_block(const BDev &d, int blk, int blocks)
 {
-    const int lb = xcd_run_block(blockIdx.x, gridDim.x, kXcdRun);
+    const int lb = xcd_run_block(blk, blocks, kXcdRun);
     const int i = find_inst(d.pre_dens, d.n_inst, lb);
     const BState *S = d.st + i;
     if (S->done) return;
@@ -345,9 +346,9 @@ __device__ inline void wa_tile(const BDev &d, const BBucket &bk, int blk, const 
     wa_net<G>(s, e, active, lane, ginv, d.pin_cell, d.pin_off, pos, d.pin_grad, hp, wa);
 }
 
-__global__ __launch_bounds__(kBlock) void kb_wa(BDev d, int at)
+__device__ inline void wa_block(const BDev &d, int at, int tile, int blocks)
 {
-    const int lb = xcd_run_block(blockIdx.x, gridDim.x, kXcdRun);
+    const int lb = xcd_run_block(tile, blocks, kXcdRun);
     int lo = 0, hi = d.n_buckets;
     while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
@@ -373,11 +374,64 @@ __global__ __launch_bounds__(kBlock) void kb_wa(BDev d, int at)
     block_reduce<2, 0>(v, d.part_wa + 2 * (size_t)lb);
 }
 
+// Per movable cell the sum of its pin partials (the cell gradient reads it).
+__device__ inline void pin_block(const BDev &d, int blk, int blocks)
+{
+    const int lb = xcd_block(blk, blocks);
+    const int i = find_inst(d.pre_cell, d.n_inst, lb);
+    if (d.st[i].done) return;
+    const BInst &I = d.inst[i];
+    const int lc = (lb - d.pre_cell[i]) * kBlock + threadIdx.x;
+    if (lc >= I.n_mov) return;
+    const int c = I.cell_off + lc;
+    d.gw[c] = sum_pin_partials(d.cps[c], d.cps[c + 1], d.cpins, d.pin_grad);
+}
+
+// ------------------------------------------------------------------ maps and WA gradient
+// Each by itself (the density plan's timing, evaluations of two branches), and two by
+// two as in a single instance (k_sort_wa, k_density_pins): 100 iterations of 4
+// instances (54k movable cells) 6.8 -> 6.3 ms, of 16 (358k) 12.3 -> 11.5.
+
+template <int CPT>
+__global__ __launch_bounds__(kBlock) void kb_sort_scatter(BDev d, int at, int K)
+{
+    sort_scatter<CPT>(d, at, K, blockIdx.x);
+}
+
+__global__ __launch_bounds__(kBlock) void kb_wa(BDev d, int at) { wa_block(d, at, blockIdx.x, gridDim.x); }
+
+template <int CPT>
+__global__ __launch_bounds__(kBlock, 8) void kb_sort_wa(BDev d, int at, int K, int sort_blocks, int sort_grid)
+{
+    const int blk = blockIdx.x;
+    if (blk >= sort_grid) wa_block(d, at, blk - sort_grid, gridDim.x - sort_grid);
+    else if (blk < sort_blocks) sort_scatter<CPT>(d, at, K, blk);
+}
+
+template <int CPT>
+__global__ __launch_bounds__(kBlock) void kb_density(BDev d)
+{
+    density_block<CPT>(d, blockIdx.x, gridDim.x);
+}
+
+template <int CPT>
+__global__ __launch_bounds__(kBlock) void kb_density_pins(BDev d, int dens_blocks, int dens_grid)
+{
+    const int blk = blockIdx.x;
+    if (blk >= dens_grid) pin_block(d, blk - dens_grid, gridDim.x - dens_grid);
+    else if (blk < dens_blocks) density_block<CPT>(d, blk, dens_blocks);
+}
+
 // ------------------------------------------------------------------ per-cell gather
 
+// kSums: reads the pin sums that kb_density_pins left; else gathers the pin partials
+// itself, as evaluations of two branches do (a pin sum pass beside the transforms
+// pays at 1.6M movable cells, 28.5 for 28.7 ms per 100 iterations, and costs at 3.3M,
+// 54.3 for 51.9).
 // One cell per thread (as k_cell_grad): g = (gW - lambda F) / max(1, pins + lambda area).
 // at == kAtTrial: position V[cur^1], references V[cur]/G[cur], output G[cur^1];
 // at == kAtCur:   position V[cur], no references, output G[cur].
+template <bool kSums>
 __global__ __launch_bounds__(kBlock) void kb_cell_grad(BDev d, int at)
 {
     const int lb = xcd_block(blockIdx.x, gridDim.x);
@@ -404,7 +458,9 @@ __global__ __launch_bounds__(kBlock) void kb_cell_grad(BDev d, int at)
         }
         const int k0 = d.cps[c], k1 = d.cps[c + 1];
         const float2 f = cell_force(p, s, exy, g, M, M);
-        const float2 gw = sum_pin_partials(k0, k1, d.cpins, d.pin_grad);
+        float2 gw;
+        if constexpr (kSums) gw = lc < I.n_mov ? d.gw[c] : make_float2(0.f, 0.f);
+        else gw = sum_pin_partials(k0, k1, d.cpins, d.pin_grad);
         const float pre = fmaxf(1.0f, __fmaf_rn(lambda * s.x, s.y, (float)(k1 - k0)));
         const float gx = __fmaf_rn(-lambda, f.x, gw.x) / pre, gy = __fmaf_rn(-lambda, f.y, gw.y) / pre;
         gout[c] = make_float2(gx, gy);
@@ -592,37 +648,19 @@ void bl_move(const BDev &d, int mode, int sort_blocks, hipStream_t s)
     });
 }
 
-void bl_sort(const BDev &d, int at, bool counted, int bin_blocks, int sort_blocks, int dens_cpt,
-             hipStream_t s)
+void bl_sort_count(const BDev &d, int at, int sort_blocks, hipStream_t s)
 {
-    if (!counted)
-        with_sort_cpt(d.sort_cpt, [&](auto cpt) {
-            hipLaunchKernelGGL(kb_sort_count<decltype(cpt)::value>, dim3(sort_blocks), dim3(kBlock), 0, s, d, at);
-        });
+    with_sort_cpt(d.sort_cpt, [&](auto cpt) {
+        hipLaunchKernelGGL(kb_sort_count<decltype(cpt)::value>, dim3(sort_blocks), dim3(kBlock), 0, s, d, at);
+    });
+}
+
+void bl_sort(const BDev &d, int at, int sort_blocks, int dens_cpt, hipStream_t s)
+{
     with_sort_cpt(d.sort_cpt, [&](auto cpt) {
         hipLaunchKernelGGL(kb_sort_scatter<decltype(cpt)::value>, dim3(sort_blocks), dim3(kBlock), 0, s, d, at,
                            kBlock * dens_cpt);
     });
-}
-
-void bl_dens(const BDev &d, int bin_blocks, int dens_blocks, int dens_cpt, bool map_range, hipStream_t s)
-{
-    const size_t lds = 2 * sizeof(unsigned long long) * (size_t)d.dens_wcap;
-    if (dens_cpt == 1)
-        hipLaunchKernelGGL(kb_density<1>, dim3(dens_blocks), dim3(kBlock), lds, s, d);
-    else if (dens_cpt == 2)
-        hipLaunchKernelGGL(kb_density<2>, dim3(dens_blocks), dim3(kBlock), lds, s, d);
-    else
-        hipLaunchKernelGGL(kb_density<4>, dim3(dens_blocks), dim3(kBlock), lds, s, d);
-    hipLaunchKernelGGL(kb_overflow, dim3(bin_blocks), dim3(kBlock), 0, s, d);
-    if (map_range) hipLaunchKernelGGL(kb_map_stats, dim3(d.n_inst), dim3(kBlock), 0, s, d);
-}
-
-void bl_maps(const BDev &d, int at, bool counted, int bin_blocks, int sort_blocks, int dens_blocks,
-             int dens_cpt, bool map_range, hipStream_t s)
-{
-    bl_sort(d, at, counted, bin_blocks, sort_blocks, dens_cpt, s);
-    bl_dens(d, bin_blocks, dens_blocks, dens_cpt, map_range, s);
 }
 
 void bl_wa(const BDev &d, int at, int wa_blocks, hipStream_t s)
@@ -630,9 +668,54 @@ void bl_wa(const BDev &d, int at, int wa_blocks, hipStream_t s)
     if (wa_blocks > 0) hipLaunchKernelGGL(kb_wa, dim3(wa_blocks), dim3(kBlock), 0, s, d, at);
 }
 
-void bl_cell_grad(const BDev &d, int at, int cell_blocks, hipStream_t s)
+void bl_sort_wa(const BDev &d, int at, int sort_blocks, int dens_cpt, int wa_blocks, hipStream_t s)
 {
-    hipLaunchKernelGGL(kb_cell_grad, dim3(cell_blocks), dim3(kBlock), 0, s, d, at);
+    const int grid = pad_xcds(sort_blocks);
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(grid + wa_blocks), dim3(kBlock), 0, s, d, at, kBlock * dens_cpt, sort_blocks,
+                           grid);
+    };
+    static_assert(kSortBatchMost <= kSortWaMost, "cells per thread of a sort beside net tiles");
+    if (d.sort_cpt == 1) go(kb_sort_wa<1>);
+    else if (d.sort_cpt == 2) go(kb_sort_wa<2>);
+    else go(kb_sort_wa<4>);
+}
+
+namespace {
+size_t dens_lds(const BDev &d) { return 2 * sizeof(unsigned long long) * (size_t)d.dens_wcap; }
+}  // namespace
+
+void bl_density(const BDev &d, int dens_blocks, int dens_cpt, hipStream_t s)
+{
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(dens_blocks), dim3(kBlock), dens_lds(d), s, d);
+    };
+    if (dens_cpt == 1) go(kb_density<1>);
+    else if (dens_cpt == 2) go(kb_density<2>);
+    else go(kb_density<4>);
+}
+
+void bl_density_pins(const BDev &d, int dens_blocks, int dens_cpt, int cell_blocks, hipStream_t s)
+{
+    const int grid = pad_xcds(dens_blocks);
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(grid + cell_blocks), dim3(kBlock), dens_lds(d), s, d, dens_blocks, grid);
+    };
+    if (dens_cpt == 1) go(kb_density_pins<1>);
+    else if (dens_cpt == 2) go(kb_density_pins<2>);
+    else go(kb_density_pins<4>);
+}
+
+void bl_overflow(const BDev &d, int bin_blocks, bool map_range, hipStream_t s)
+{
+    hipLaunchKernelGGL(kb_overflow, dim3(bin_blocks), dim3(kBlock), 0, s, d);
+    if (map_range) hipLaunchKernelGGL(kb_map_stats, dim3(d.n_inst), dim3(kBlock), 0, s, d);
+}
+
+void bl_cell_grad(const BDev &d, int at, bool sums, int cell_blocks, hipStream_t s)
+{
+    if (sums) hipLaunchKernelGGL(kb_cell_grad<true>, dim3(cell_blocks), dim3(kBlock), 0, s, d, at);
+    else hipLaunchKernelGGL(kb_cell_grad<false>, dim3(cell_blocks), dim3(kBlock), 0, s, d, at);
 }
 
 void bl_reduce_control(const BDev &d, int mode, hipStream_t s)

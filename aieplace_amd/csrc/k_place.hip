@@ -1030,8 +1030,6 @@ void launch_sort_clear(Ctx &c, hipStream_t s)
 
 namespace {
 
-int pad_xcds(int blocks) { return (blocks + kXcds - 1) / kXcds * kXcds; }
-
 // `beside`: the blocks share a launch with others, which begin at a multiple of the XCDs
 SortArgs sort_args(const Ctx &c, int cpt, bool beside)
 {

@@ -270,7 +270,7 @@ def batch_stats(args) -> str:
              "```", "",
              "Two full batched runs (the first captures the graphs and autotunes the tiles; the second is the "
              "measured one), so every count is about twice one run's.  The WA gradient runs on a second captured "
-             "branch while the running instances hold >= 400k cells, so the shares add up to more than the "
+             "branch while the running instances hold >= 800k cells, so the shares add up to more than the "
              "wall time.", ""]
     if res:
         r = res["run"]

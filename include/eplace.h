@@ -88,8 +88,7 @@ typedef struct ep_params {
                                  the backtracking condition (fallback to the search) */
     int32_t fork_min_cells;   /* captured evaluations run the WA gradient on a second
                                  branch from this many placeable cells on (results are
-                                 identical either way); 0 = the default, 800000
-                                 (a batch: 400000 cells of running instances)       */
+                                 identical either way); 0 = the default, 800000     */
     int32_t cell_order;       /* 1 (default): movable cells stored in breadth-first order
                                  over the netlist, so that cells of one net sit at nearby
                                  indices (gather locality for netlists in any order);

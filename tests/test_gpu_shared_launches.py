@@ -44,3 +44,21 @@ def test_no_nets():
     assert g["fx"].any() and g["fy"].any()
     # every movable cell has area 1 and no pins: the preconditioner is 1
     assert np.array_equal(g["gx"], -g["fx"]) and np.array_equal(g["gy"], -g["fy"])
+
+
+# instances whose blocks end mid-grid: sort, net tile, density and cell grids that
+# are no multiple of the XCDs
+@pytest.mark.parametrize("counts", [(40,), (255, 1_025, 3_000), (9_000, 40, 20_001, 5_000, 700)])
+def test_batch_shared_launches_equal_forked(counts):
+    """As above for a batch's instances."""
+    from aieplace_amd.batch import BatchPlacer
+    print(f"case batch shared launches {counts}", flush=True)
+    nls = [A.generate("stdcell", seed=3 + k, n_movable=n) for k, n in enumerate(counts)]
+    out = []
+    for fork in (1, 1 << 30):
+        p = A.placer_params(A.CONFIGS["stdcell_200k"], max_iters=6, fork_min_cells=fork)
+        bp = BatchPlacer(nls, [64] * len(counts), p)
+        bp.run()
+        out.append([a for i in range(len(counts)) for a in bp.positions(i)])
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
