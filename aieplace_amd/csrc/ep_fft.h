@@ -8,6 +8,16 @@
 
 namespace ep {
 
+// Stages of an FFT whose length is no power of two (Stockham, radix r after a product
+// ns of radices), with the reciprocals for the index divisions.
+struct FftPlan {
+    int stages;
+    struct Stage {
+        int r, ns;
+        float inv_ns, inv_span;  // 1 / ns, 1 / (r ns)
+    } st[8];
+};
+
 // One solve; every pointer is device memory.
 struct FftArgs {
     const float *map;      // [Mx][My] density map
@@ -19,24 +29,32 @@ struct FftArgs {
     float2 *exy;           // [Mx][My] field
     int Mx, My;
     float scale, wxs, wys;  // spectral scaling, as GemmArgs
+    FftPlan px, py;         // fft_plan(Mx), fft_plan(My)
 };
 
-// Grid sides that the FFT path takes: powers of two from 16 (the smallest grid)
-// to 8192 (the columns of two FFTs of 16384 points do not fit the LDS).
-inline bool fft_side(int n) { return n >= 16 && n <= 8192 && (n & (n - 1)) == 0; }
+// Grid sides are multiples of 16.  The FFT path takes powers of two up to 8192 (the
+// columns of two FFTs of 16384 points do not fit the LDS) and any other side up to
+// 4080 (40 bytes of LDS per point in the columns kernel).
+constexpr int kFftPow2Max = 8192, kFftMixedMax = 4080;
+inline bool fft_pow2(int n) { return (n & (n - 1)) == 0; }
+inline bool fft_side(int n) { return n >= 16 && n % 16 == 0 && n <= (fft_pow2(n) ? kFftPow2Max : kFftMixedMax); }
 
-// Constants of length-n transforms (n a power of two), made in FP64.
+// Constants of length-n transforms, made in FP64.
 void fft_table(int n, std::vector<float2> &tab);
+// Stages of a length that is no power of two (none for one that is).
+FftPlan fft_plan(int n);
 void launch_field_fft(const FftArgs &a, hipStream_t s);
 
 // Batched solves: one launch per stage (rows, columns, field) and class covers
 // the tiles (instance, block of the instance's stage) of every instance.  The
-// classes are block sizes: 128 threads for sides up to 1024, 1024 above.
-constexpr int kFftClasses = 2;
+// classes: powers of two up to 1024 and above (128 and 1024 threads), other sides.
+constexpr int kFftClasses = 3;
 struct FftBatchTiles {
     int2 *d[3];
     int n[3];
+    int longest;  // side among the tiles' instances
 };
+int fft_class(int M);
 // Appends instance i's tiles (side M) to the lists of its class.
 void fft_batch_tiles(int i, int M, std::vector<int2> (&tiles)[kFftClasses][3]);
 void launch_field_fft_batch(const FftArgs *args, const FftBatchTiles (&t)[kFftClasses], hipStream_t s);

@@ -1,4 +1,4 @@
-// k_fft.hip -- Poisson field solve on power-of-two grids as FP32 FFTs in LDS.
+// k_fft.hip -- Poisson field solve as FP32 FFTs in LDS.
 //
 // The same field as the transform products of k_field.hip (RePlAce scaling,
 // python/AIEmath/fft_replace/fft.cpp:118-212), in three kernels instead of four:
@@ -36,6 +36,7 @@
 #include <cmath>
 #include <vector>
 
+#include "ep_device.h"
 #include "ep_fft.h"
 
 // Multiply-adds only where they are written: the single and the batched kernels
@@ -516,6 +517,311 @@ __global__ __launch_bounds__(field_ffts_of<L>() * Plan<L>::T) void k_fft_field(F
     field_pass<L, field_ffts_of<L>()>(a, blockIdx.x, fft_lds);
 }
 
+// ------------------------------------------------------------------ other lengths
+// Lengths that are no power of two: the same three passes over a plan of stages, the odd
+// factors first, then radices 8 and 4.  A long odd radix is a plain sum (61 is a plan like
+// 3 is), and a block's threads share every stage's points, so that a length of 240 keeps
+// eight waves busy.  One solve alone in us, products (FP32 / split BF16 / split FP16) -> FFTs:
+// 48^2 17.8 / 16.0 / 23.0 -> 14.8, 96 x 80 23.3 / 19.6 / 26.0 -> 15.9, 400 x 240 37.3 /
+// 29.1 / 34.6 -> 18.8, 544^2 (17) 54 / 46 / 52 -> 24, 976^2 (61) 105 / 82 / 92 -> 43, 1008^2
+// 104 / 75 / 89 -> 44, 2000^2 588 / 497 / 560 -> 144; max-norm error at most 9e-7 (products:
+// 7e-6 / 1.4e-5 / 1.8e-6).  Small sides are bound by latency (a barrier and an LDS round
+// trip per stage), large ones by LDS bandwidth.  512 threads: 256 and 1024 take 20.2 and
+// 18.7 at 400 x 240 (512: 19.3), 55 and 56 at 976^2 (49).
+
+// o / d for 0 <= o < 2^12 and inv = 1 / d rounded: (o + 1/2) / d is further from a whole
+// number than its error.
+__device__ inline int quotient(int o, float inv) { return (int)(((float)o + 0.5f) * inv); }
+
+// First stage, r odd, ns = 1, so no twiddles: outputs q and r - q of a butterfly share the
+// sums of cosines and sines over the pairs (i, r - i).  Lanes run over the butterflies:
+// they read consecutive points and the same root (one output per item and lanes over the
+// outputs, which reads the roots with bank conflicts, took 203 us for 61 at 976^2).
+template <bool INV, int R>
+__device__ __forceinline__ void mixed_first(const float2 *__restrict__ in, float2 *__restrict__ out, const float2 *root, int N,
+                                   int C, int r_any)
+{
+    const int r = R ? R : r_any, half = (r - 1) / 2, jump = N / r, items = jump * (half + 1);
+    const float inv = 1.0f / (float)jump;
+    for (int e = threadIdx.x; e < C * items; e += blockDim.x) {
+        const int c = e >= items ? 1 : 0, w = e - c * items;
+        const int q = quotient(w, inv), g = w - q * jump;
+        const float2 *x = in + c * N + g;
+        float2 cs = x[0], sn = make_float2(0.0f, 0.0f);
+        int k = 0;
+        auto pair = [&](int i) {
+            k += q;
+            k -= k >= r ? r : 0;
+            const float2 a = x[i * jump], b = x[(r - i) * jump], t = root[k * jump];  // (cos, -sin)
+            cs = make_float2(fmaf(t.x, a.x + b.x, cs.x), fmaf(t.x, a.y + b.y, cs.y));
+            sn = make_float2(fmaf(t.y, a.x - b.x, sn.x), fmaf(t.y, a.y - b.y, sn.y));
+        };
+        if (R) {
+#pragma unroll
+            for (int i = 1; i <= (R - 1) / 2; ++i) pair(i);
+        } else {
+#pragma unroll 4
+            for (int i = 1; i <= half; ++i) pair(i);
+        }
+        const float2 d = INV ? make_float2(sn.y, -sn.x) : make_float2(-sn.y, sn.x);
+        float2 *y = out + c * N + g * r;
+        y[q] = cadd(cs, d);
+        if (q) y[r - q] = csub(cs, d);
+    }
+}
+
+// A later stage with an odd radix: point o = (j / ns) r ns + j % ns + q ns is the sum over
+// i < r of in[j + i N/r] e^{-2 pi i (o mod r ns) i / (r ns)}, one point per item.
+template <bool INV, int R>
+__device__ __forceinline__ void mixed_stage(const float2 *__restrict__ in, float2 *__restrict__ out,
+                                            const float2 *root, int N, int C, int r_any, const FftPlan::Stage &st)
+{
+    const int r = R ? R : r_any, span = r * st.ns, step = N / span, jump = N / r;
+    for (int e = threadIdx.x; e < C * N; e += blockDim.x) {
+        const int c = e >= N ? 1 : 0, o = e - c * N;
+        const int g = quotient(o, st.inv_span), m = o - g * span;
+        const int k = m - quotient(m, st.inv_ns) * st.ns;
+        const float2 *x = in + c * N + g * st.ns + k;
+        const int turn = m * step;  // < N
+        float2 acc = x[0];
+        int w = 0;
+        auto term = [&](int i) {
+            w += turn;
+            w -= w >= N ? N : 0;
+            const float2 z = x[i * jump], t = root[w];
+            const float s = INV ? -t.y : t.y;
+            acc = make_float2(fmaf(-z.y, s, fmaf(z.x, t.x, acc.x)), fmaf(z.y, t.x, fmaf(z.x, s, acc.y)));
+        };
+        if (R) {
+#pragma unroll
+            for (int i = 1; i < R; ++i) term(i);
+        } else {
+#pragma unroll 4
+            for (int i = 1; i < r; ++i) term(i);
+        }
+        out[e] = acc;
+    }
+}
+
+// A later stage of radix 4 or 8: one butterfly per item (one output per item: 47.5 us at
+// 976^2, 20.5 at 480 x 352; 43.0 and 19.0 so).
+template <bool INV, int R>
+__device__ __forceinline__ void mixed_butterflies(const float2 *__restrict__ in, float2 *__restrict__ out,
+                                                  const float2 *root, int N, int C, const FftPlan::Stage &st)
+{
+    const int jump = N / R, step = jump / st.ns;
+    for (int e = threadIdx.x; e < C * jump; e += blockDim.x) {
+        const int c = e >= jump ? 1 : 0, j = e - c * jump, k = j - quotient(j, st.inv_ns) * st.ns;
+        float2 v[R];
+#pragma unroll
+        for (int i = 0; i < R; ++i) v[i] = in[c * N + j + i * jump];
+#pragma unroll
+        for (int i = 1; i < R; ++i) v[i] = cmul<INV>(v[i], root[i * k * step]);  // i k < R ns
+        if constexpr (R == 8) bfly8<INV>(v);
+        else bfly4<INV>(v[0], v[1], v[2], v[3]);
+        float2 *y = out + c * N + (j - k) * R + k;
+#pragma unroll
+        for (int i = 0; i < R; ++i) y[i * st.ns] = v[i];
+    }
+}
+
+// C FFTs of N points in a ([c][N]) with b as the other buffer; returns the one that
+// holds the result, visible to the block.
+template <bool INV>
+__device__ __forceinline__ float2 *mixed_fft(float2 *a, float2 *b, const float2 *root, int N, int C, const FftPlan &p)
+{
+    __syncthreads();
+    switch (p.st[0].r) {
+    case 3: mixed_first<INV, 3>(a, b, root, N, C, 3); break;
+    case 5: mixed_first<INV, 5>(a, b, root, N, C, 5); break;
+    case 7: mixed_first<INV, 7>(a, b, root, N, C, 7); break;
+    default: mixed_first<INV, 0>(a, b, root, N, C, p.st[0].r); break;
+    }
+    for (int s = 1; s < p.stages; ++s) {
+        float2 *t = a;
+        a = b;
+        b = t;
+        __syncthreads();
+        const FftPlan::Stage &st = p.st[s];
+        switch (st.r) {
+        case 3: mixed_stage<INV, 3>(a, b, root, N, C, 3, st); break;
+        case 4: mixed_butterflies<INV, 4>(a, b, root, N, C, st); break;
+        case 5: mixed_stage<INV, 5>(a, b, root, N, C, 5, st); break;
+        case 7: mixed_stage<INV, 7>(a, b, root, N, C, 7, st); break;
+        case 8: mixed_butterflies<INV, 8>(a, b, root, N, C, st); break;
+        default: mixed_stage<INV, 0>(a, b, root, N, C, st.r, st); break;
+        }
+    }
+    __syncthreads();
+    return b;
+}
+
+// Table of such a length: the N/2 half-sample shifts, then the N roots.
+__device__ __forceinline__ void load_roots(const float2 *__restrict__ tab, float2 *root, int N)
+{
+    for (int i = threadIdx.x; i < N; i += blockDim.x) root[i] = tab[N / 2 + i];
+}
+
+// A thread's first half-sample shift, loaded ahead of the FFT, and that of any k.
+__device__ inline float2 first_half(const float2 *__restrict__ tab, int N) { return tab[min((int)threadIdx.x, N / 2 - 1)]; }
+__device__ inline float2 half_at(const float2 *__restrict__ tab, float2 first, int k)
+{
+    return k == (int)threadIdx.x ? first : tab[k];
+}
+
+// Rows 2 blk and 2 blk + 1.  3 N points of LDS.
+__device__ __forceinline__ void mixed_rows(const FftArgs &a, const FftPlan &p, int blk, float2 *lds)
+{
+    const int N = a.My, rows = a.Mx;
+    if (*a.skip) return;
+    float2 *root = lds, *b0 = lds + N, *b1 = b0 + N;
+    const float2 *__restrict__ x0 = reinterpret_cast<const float2 *>(a.map + (size_t)2 * blk * N);
+    const float2 *__restrict__ x1 = x0 + N / 2;
+    const float mean = *a.mean;
+    const float2 half = first_half(a.tab_y, N);
+    load_roots(a.tab_y, root, N);
+    for (int n = threadIdx.x; n < N / 2; n += blockDim.x) {
+        const float2 xa = x0[n], xb = x1[n];
+        b0[n] = make_float2(xa.x - mean, xb.x - mean);
+        b0[N - 1 - n] = make_float2(xa.y - mean, xb.y - mean);
+    }
+    float2 *z = mixed_fft<false>(b0, b1, root, N, 1, p);
+    for (int k = threadIdx.x; k < N / 2; k += blockDim.x) {
+        if (k == 0) {  // and N/2
+            const float2 h = z[N / 2];
+            z[N / 2] = make_float2(h.x * kSqrtHalf, h.y * kSqrtHalf);
+        } else {
+            const DctPair d = dct_pair(z[k], z[N - k], half_at(a.tab_y, half, k));
+            z[k] = make_float2(d.a_k, d.b_k);
+            z[N - k] = make_float2(d.a_n, d.b_n);
+        }
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < N / 2; e += blockDim.x) {
+        const int r = e & 1, g = e >> 1;
+        float o[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const float2 v = z[4 * g + c];
+            o[c] = r ? v.y : v.x;
+        }
+        *reinterpret_cast<float4 *>(a.t1 + ((size_t)g * rows + 2 * blk + r) * 4) = make_float4(o[0], o[1], o[2], o[3]);
+    }
+}
+
+// Columns 2 blk and 2 blk + 1.  5 N points of LDS.
+__device__ __forceinline__ void mixed_columns(const FftArgs &a, const FftPlan &p, int blk, float2 *lds)
+{
+    const int N = a.Mx, ca = 2 * blk;
+    if (*a.skip) return;
+    float2 *root = lds, *b0 = lds + N, *b1 = b0 + 2 * N;
+    const size_t at = (size_t)(ca >> 2) * N * 4 + (ca & 3);
+    const float2 half = first_half(a.tab_x, N);
+    load_roots(a.tab_x, root, N);
+    for (int i = threadIdx.x; i < N; i += blockDim.x)
+        b0[(i & 1) ? N - 1 - (i >> 1) : i >> 1] = *reinterpret_cast<const float2 *>(a.t1 + at + (size_t)i * 4);
+    const float2 *z = mixed_fft<false>(b0, b1, root, N, 1, p);
+    float2 *in = z == b0 ? b1 : b0, *other = z == b0 ? b0 : b1;  // the spectrum is read before `other` is written
+    for (int k = threadIdx.x; k < N / 2; k += blockDim.x) {  // both columns' points k and N - k
+        const float2 zk = z[k], zn = z[k == 0 ? N / 2 : N - k];
+        if (k == 0) {  // and N/2
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const float2 e = spectral(a, 0, ca + c, c ? zk.y : zk.x);
+                const float2 q = spectral(a, N / 2, ca + c, (c ? zn.y : zn.x) * kSqrtHalf);
+                in[c * N] = make_float2(0.0f, e.y);
+                in[c * N + N / 2] = make_float2(q.x * kSqrtHalf, q.y * kSqrtHalf);
+            }
+        } else {
+            const float2 w = half_at(a.tab_x, half, k);
+            const DctPair d = dct_pair(zk, zn, w);
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const float2 ek = spectral(a, k, ca + c, c ? d.b_k : d.a_k);
+                const float2 en = spectral(a, N - k, ca + c, c ? d.b_n : d.a_n);
+                idct_pair(en.x, ek.x, ek.y, en.y, w, in[c * N + k], in[c * N + N - k]);  // sine sum: reversed spectrum
+            }
+        }
+    }
+    z = mixed_fft<true>(in, other, root, N, 2, p);
+    for (int i = threadIdx.x; i < N; i += blockDim.x) {
+        const int n = (i & 1) ? N - 1 - (i >> 1) : i >> 1;
+        const float2 z0 = z[n], z1 = z[N + n];
+        const float sg = (i & 1) ? -1.0f : 1.0f;
+        *reinterpret_cast<float4 *>(a.pq + at + (size_t)i * 4) = make_float4(sg * z0.x, z0.y, sg * z1.x, z1.y);
+    }
+}
+
+// Row blk of the field.  3 N points of LDS.
+__device__ __forceinline__ void mixed_field(const FftArgs &a, const FftPlan &p, int row, float2 *lds)
+{
+    const int N = a.My, rows = a.Mx;
+    if (*a.skip) return;
+    float2 *root = lds, *b0 = lds + N, *b1 = b0 + N;
+    const float2 half = first_half(a.tab_y, N);
+    load_roots(a.tab_y, root, N);
+    for (int e = threadIdx.x; e < N / 2; e += blockDim.x) {
+        const float4 x = *reinterpret_cast<const float4 *>(a.pq + ((size_t)(e >> 1) * rows + row) * 4 + 2 * (e & 1));
+        b1[2 * e] = make_float2(x.x, x.y);
+        b1[2 * e + 1] = make_float2(x.z, x.w);
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k < N / 2; k += blockDim.x) {
+        const float2 ek = b1[k], en = b1[k == 0 ? N / 2 : N - k];
+        if (k == 0) {  // and N/2
+            b0[0] = make_float2(ek.x, 0.0f);
+            b0[N / 2] = make_float2(en.x * kSqrtHalf, en.y * kSqrtHalf);
+        } else {
+            float2 zk, zn;
+            idct_pair(ek.x, en.x, en.y, ek.y, half_at(a.tab_y, half, k), zk, zn);
+            b0[k] = zk;
+            b0[N - k] = zn;
+        }
+    }
+    const float2 *z = mixed_fft<true>(b0, b1, root, N, 1, p);
+    for (int n = threadIdx.x; n < N / 2; n += blockDim.x) {
+        const float2 z0 = z[n], z1 = z[N - 1 - n];
+        *reinterpret_cast<float4 *>(a.exy + (size_t)row * N + 2 * n) = make_float4(z0.x, z0.y, z1.x, -z1.y);
+    }
+}
+
+constexpr int kMixedThreads = 512;
+
+// Pass S (rows, columns, field).  Neighbouring rows and columns, which share the
+// layout groups' cache lines, go to one XCD.
+template <int S>
+__global__ __launch_bounds__(kMixedThreads) void k_fft_mixed(FftArgs a)
+{
+    const int blk = dev::xcd_block(blockIdx.x, gridDim.x);
+    if (S == 0) mixed_rows(a, a.py, blk, fft_lds);
+    else if (S == 1) mixed_columns(a, a.px, blk, fft_lds);
+    else mixed_field(a, a.py, blk, fft_lds);
+}
+
+template <int S>
+__global__ __launch_bounds__(kMixedThreads) void k_fft_mixed_b(const FftArgs *__restrict__ args, const int2 *__restrict__ tiles)
+{
+    const int2 t = tiles[dev::xcd_block(blockIdx.x, gridDim.x)];
+    const FftArgs a = args[t.x];  // a batch's grids are square
+    __shared__ FftPlan p;         // indexed by stage: not in registers
+    for (int i = threadIdx.x; i < (int)(sizeof(FftPlan) / 4); i += kMixedThreads)
+        reinterpret_cast<int *>(&p)[i] = reinterpret_cast<const int *>(&args[t.x].px)[i];
+    __syncthreads();
+    if (S == 0) mixed_rows(a, p, t.y, fft_lds);
+    else if (S == 1) mixed_columns(a, p, t.y, fft_lds);
+    else mixed_field(a, p, t.y, fft_lds);
+}
+
+template <int S>
+void launch_mixed(const FftArgs &a, hipStream_t s)
+{
+    const int n = S == 1 ? a.Mx : a.My, blocks = S == 0 ? a.Mx / 2 : S == 1 ? a.My / 2 : a.Mx;
+    const size_t lds = (S == 1 ? 5 : 3) * sizeof(float2) * (size_t)n;
+    hipLaunchKernelGGL(k_fft_mixed<S>, dim3(blocks), dim3(kMixedThreads), lds, s, a);
+}
+
+// ------------------------------------------------------------------ batches
+
 // Batched: block b runs tile tiles[b] = (instance, block) of stage S with
 // blocks of NT threads; the instance's side picks the length.
 template <int NT, int S, int L>
@@ -579,14 +885,51 @@ void with_length(int l, Go go)
 
 }  // namespace
 
+// Odd primes share a stage up to this product.  One solve in us, 1 / 9 / 25 / 63: 400 x 240
+// 20.0 / 19.8 / 19.6 / 19.5, 1008^2 47.0 / 51.9 / 47.6 / 49.3, 2000^2 174 / 174 / 159 / 160.
+constexpr int kMixedOdd = 25;
+
+FftPlan fft_plan(int n)
+{
+    FftPlan p{};
+    if (fft_pow2(n)) return p;
+    int odd = n, twos = 0;
+    for (; odd % 2 == 0; odd /= 2) ++twos;
+    std::vector<int> primes, r;
+    for (int f = 3; odd > 1; f += 2)
+        for (; odd % f == 0; odd /= f) primes.insert(primes.begin(), f);  // the largest first
+    while (!primes.empty()) {  // one stage of up to kMixedOdd saves a barrier and an exchange
+        int f = 1;
+        for (size_t i = 0; i < primes.size();)
+            if (f == 1 || f * primes[i] <= kMixedOdd) {
+                f *= primes[i];
+                primes.erase(primes.begin() + i);
+            } else {
+                ++i;
+            }
+        r.push_back(f);
+    }
+    for (int s = 0; twos > 0; twos -= r.back() == 8 ? 3 : 2, ++s) r.push_back(radix_of(twos, 0));
+    int ns = 1;
+    for (int f : r) {
+        p.st[p.stages++] = {f, ns, 1.0f / (float)ns, 1.0f / (float)(f * ns)};
+        ns *= f;
+    }
+    return p;
+}
+
 void fft_table(int n, std::vector<float2> &tab)
 {
-    const int l = log2_of(n);
     tab.clear();
     auto unit = [&](double turns) {  // e^{-2 pi i turns}
         tab.push_back(make_float2((float)std::cos(2.0 * M_PI * turns), (float)-std::sin(2.0 * M_PI * turns)));
     };
     for (int k = 0; k < n / 2; ++k) unit(k / (4.0 * n));
+    if (!fft_pow2(n)) {
+        for (int k = 0; k < n; ++k) unit((double)k / n);
+        return;
+    }
+    const int l = log2_of(n);
     for (int s = 1, ns = radix_of(l, 0); ns < n; ns *= radix_of(l, s++)) {
         const int R = radix_of(l, s);
         for (int r = 1; r < R; ++r)
@@ -597,26 +940,32 @@ void fft_table(int n, std::vector<float2> &tab)
 void launch_field_fft(const FftArgs &a, hipStream_t s)
 {
     const int lx = log2_of(a.Mx), ly = log2_of(a.My);
-    with_length(ly, [&](auto c) {
+    if (!fft_pow2(a.My)) launch_mixed<0>(a, s);
+    else with_length(ly, [&](auto c) {
         constexpr int L = decltype(c)::value, F = ffts_of<L>();
         hipLaunchKernelGGL(k_fft_rows<L>, dim3((a.Mx + 2 * F - 1) / (2 * F)), dim3(F * Plan<L>::T),
                            F * Plan<L>::buf * sizeof(float2), s, a);
     });
-    with_length(lx, [&](auto c) {
+    if (!fft_pow2(a.Mx)) launch_mixed<1>(a, s);
+    else with_length(lx, [&](auto c) {
         constexpr int L = decltype(c)::value, F = col_ffts_of<L>();
         hipLaunchKernelGGL(k_fft_columns<L>, dim3((a.My + 2 * F - 1) / (2 * F)),
                            dim3(col_halves_of<L>() * F * Plan<L>::T), 2 * F * Plan<L>::buf * sizeof(float2), s, a);
     });
-    with_length(ly, [&](auto c) {
+    if (!fft_pow2(a.My)) launch_mixed<2>(a, s);
+    else with_length(ly, [&](auto c) {
         constexpr int L = decltype(c)::value, F = field_ffts_of<L>();
         hipLaunchKernelGGL(k_fft_field<L>, dim3((a.Mx + F - 1) / F), dim3(F * Plan<L>::T),
                            F * Plan<L>::buf * sizeof(float2), s, a);
     });
 }
 
+int fft_class(int M) { return !fft_pow2(M) ? 2 : M <= 1024 ? 0 : 1; }
+
 void fft_batch_tiles(int i, int M, std::vector<int2> (&tiles)[kFftClasses][3])
 {
-    const int cls = M <= 1024 ? 0 : 1, nt = cls ? 1024 : 128, F = nt / (M / 8);
+    const int cls = fft_class(M);
+    const int F = cls < 2 ? (cls ? 1024 : 128) / (M / 8) : 1;
     for (int stage = 0; stage < 3; ++stage) {
         const int per = stage == 2 ? F : 2 * F;  // rows or columns per block
         for (int b = 0; b < (M + per - 1) / per; ++b) tiles[cls][stage].push_back(make_int2(i, b));
@@ -625,18 +974,21 @@ void fft_batch_tiles(int i, int M, std::vector<int2> (&tiles)[kFftClasses][3])
 
 void launch_field_fft_batch(const FftArgs *args, const FftBatchTiles (&t)[kFftClasses], hipStream_t s)
 {
-    // 8 NT points per block; the columns hold both inverse FFTs of each
-    const size_t pt = 9 * sizeof(float2);
+    // Powers of two: 8 NT points per block (9 with their padding).  Others: the longest
+    // of the class.  The columns hold both inverse FFTs of each.
     auto stage = [&](int k, int i, auto kern, int nt) {
-        if (t[k].n[i])
-            hipLaunchKernelGGL(kern, dim3(t[k].n[i]), dim3(nt), nt * pt * (i == 1 ? 2 : 1), s, args, t[k].d[i]);
+        const size_t lds = sizeof(float2) * (k < 2 ? 9 * nt * (i == 1 ? 2 : 1) : (i == 1 ? 5 : 3) * t[k].longest);
+        if (t[k].n[i]) hipLaunchKernelGGL(kern, dim3(t[k].n[i]), dim3(nt), lds, s, args, t[k].d[i]);
     };
     stage(0, 0, k_fft_b<128, 0>, 128);
     stage(1, 0, k_fft_b<1024, 0>, 1024);
+    stage(2, 0, k_fft_mixed_b<0>, kMixedThreads);
     stage(0, 1, k_fft_b<128, 1>, 128);
     stage(1, 1, k_fft_b<1024, 1>, 1024);
+    stage(2, 1, k_fft_mixed_b<1>, kMixedThreads);
     stage(0, 2, k_fft_b<128, 2>, 128);
     stage(1, 2, k_fft_b<1024, 2>, 1024);
+    stage(2, 2, k_fft_mixed_b<2>, kMixedThreads);
 }
 
 }  // namespace ep

@@ -1,6 +1,6 @@
 // k_field.hip -- Poisson field solve as dense transform-matrix products on MFMA,
-// for grids with a side that is not a power of two (the others: k_fft.hip), and
-// the standalone transforms.
+// for grids with a side that the FFT path does not take (ep_fft.h: above 4080 and no
+// power of two, or above 8192), and the standalone transforms.
 //
 // Reference: the separable DCT field of vck5000/host/src/AIEplace.cpp:752-934
 // (compute_a_uv_DCT / compute_eField_DCT with DCT_naive/IDCT_naive/IDXST_naive,
@@ -865,7 +865,7 @@ void launch_field(Ctx &c, int precision, hipStream_t s)
     a.skip = &c.d_scal->halt;  // a finished device-controlled run skips the solve
     if (fm->fft_x) {
         FftArgs f{c.map_field, c.map_mean, a.skip, fm->fft_x, fm->fft_y, c.tA, reinterpret_cast<float2 *>(c.tB),
-                  c.exy, c.Mx, c.My, a.scale, a.wxs, a.wys};
+                  c.exy, c.Mx, c.My, a.scale, a.wxs, a.wys, fft_plan(c.Mx), fft_plan(c.My)};
         launch_field_fft(f, s);
         return;
     }
@@ -1064,7 +1064,10 @@ ep_status batch_field_init(BatchField *&out, const std::vector<BatchFieldInst> &
             a.skip = d.skip;
             if (pi == 0 && bf->fft_tabs[si]) {
                 fargs[i] = FftArgs{d.map_field, d.map_mean, d.skip, bf->fft_tabs[si], bf->fft_tabs[si], d.tA,
-                                   reinterpret_cast<float2 *>(d.tB), d.exy, d.M, d.M, a.scale, a.wxs, a.wys};
+                                   reinterpret_cast<float2 *>(d.tB), d.exy, d.M, d.M, a.scale, a.wxs, a.wys,
+                                   fft_plan(d.M), fft_plan(d.M)};
+                int &longest = bf->fft[fft_class(d.M)].longest;
+                longest = std::max(longest, d.M);
                 fft_batch_tiles(i, d.M, ftiles);
             }
             auto setA = [&](GemmArgs &g, int z, int m) { set_operand(g, z, ms.half[m], m, prec); };
