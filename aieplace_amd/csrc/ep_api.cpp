@@ -97,8 +97,7 @@ void enqueue_eval(Ctx &c, const float2 *pos, const float2 *vref, const float2 *g
     if (!counted) launch_sort_count(c, pos, s);
     launch_sort_wa(c, pos, s);
     launch_density_pins(c, s);
-    launch_overflow(c, s);
-    launch_field(c, c.prm.precision, s);
+    launch_overflow_field(c, c.prm.precision, s);
     launch_cell_grad(c, pos, counted ? nullptr : vref, gref, gout, gw_out, f_out, s);
     launch_finalize(c, s, counted);
     (void)hipMemcpyAsync(c.h_res, c.d_res, sizeof(DevResult), hipMemcpyDeviceToHost, s);
@@ -635,6 +634,7 @@ extern "C" ep_status ep_create(const ep_netlist *nl, const ep_params *p, ep_ctx 
     }
     const size_t nb = (size_t)c->Mx * c->My;
     c->ovf_blocks = (int)std::min<size_t>(1024, (nb + kBlock * 4 - 1) / (kBlock * 4));
+    if (fft_side(c->Mx) && fft_side(c->My)) c->ovf_blocks = std::max(c->ovf_blocks, fft_row_blocks(c->Mx, c->My));
     c->cell_blocks = (int)std::min<int64_t>(kCellGridCap, ((int64_t)c->n_place + 2 * kBlock - 1) / (2 * kBlock));
     c->part_wa_off = 0;
     c->part_ovf_off = 2 * c->wa_part_blocks;
@@ -1287,8 +1287,7 @@ static ep_status build_ctl_graph(ep_ctx *c, const CtlParams &p)
             EP_CAP(hipStreamWaitEvent(x.side, x.fork, 0), s);
             launch_sort(x, vt, x.side);
             launch_density(x, x.side);
-            launch_overflow(x, x.side);
-            launch_field(x, x.prm.precision, x.side);
+            launch_overflow_field(x, x.prm.precision, x.side);
             EP_CAP(hipEventRecord(x.join, x.side), s);
             launch_wa(x, vt, s);
             launch_pin_sum(x, s);
@@ -1297,8 +1296,7 @@ static ep_status build_ctl_graph(ep_ctx *c, const CtlParams &p)
         } else {
             launch_sort_wa(x, vt, s);
             launch_density_pins(x, s);
-            launch_overflow(x, s);
-            launch_field(x, x.prm.precision, s);
+            launch_overflow_field(x, x.prm.precision, s);
             launch_cell_grad(x, vt, none, gc, gn, nullptr, nullptr, s);
         }
         launch_finalize_decide(x, p, s);

@@ -32,6 +32,19 @@ struct FftArgs {
     FftPlan px, py;         // fft_plan(Mx), fft_plan(My)
 };
 
+// What the overflow pass (k_overflow) does, done by the rows kernel as it reads the map:
+// scatter accumulators -> maps, overflow numerator, accumulators and tile counts cleared.
+struct FftMaps {
+    unsigned long long *acc_field, *acc_mov;
+    const float *map_fix;
+    float *map_field, *map_mov;
+    double unit;
+    float rho_t, cap;
+    double *part;        // overflow partials, [part_blocks] of four (the first is used)
+    int part_blocks;     // at least fft_row_blocks; the rest is zeroed
+    int32_t *count;      // sort counts and cursors
+};
+
 // Grid sides are multiples of 16.  The FFT path takes powers of two up to 8192 (the
 // columns of two FFTs of 16384 points do not fit the LDS) and any other side up to
 // 4080 (40 bytes of LDS per point in the columns kernel).
@@ -43,7 +56,10 @@ inline bool fft_side(int n) { return n >= 16 && n % 16 == 0 && n <= (fft_pow2(n)
 void fft_table(int n, std::vector<float2> &tab);
 // Stages of a length that is no power of two (none for one that is).
 FftPlan fft_plan(int n);
-void launch_field_fft(const FftArgs &a, hipStream_t s);
+// Blocks of the rows kernel.
+int fft_row_blocks(int Mx, int My);
+// `maps`: the overflow pass goes with the rows (null: the map is there).
+void launch_field_fft(const FftArgs &a, const FftMaps *maps, hipStream_t s);
 
 // Batched solves: one launch per stage (rows, columns, field) and class covers
 // the tiles (instance, block of the instance's stage) of every instance.  The

@@ -261,10 +261,47 @@ constexpr int field_ffts_of()
     return Plan<L>::T >= 1024 ? 1 : Plan<L>::T >= 512 ? 2 : Plan<L>::T >= 16 ? 4 : 64 / Plan<L>::T;
 }
 
+// Bins o and o + 1 of the map (o even) from their accumulators, which are cleared; adds
+// their overflow.  Bins of a row that is another block's (`mine` unset) are only read.
+struct MapBins {
+    ulonglong2 field, mov;
+    float2 fix;
+};
+__device__ inline MapBins load_bins(const FftMaps &mp, size_t o)
+{
+    return {*reinterpret_cast<const ulonglong2 *>(mp.acc_field + o), *reinterpret_cast<const ulonglong2 *>(mp.acc_mov + o),
+            *reinterpret_cast<const float2 *>(mp.map_fix + o)};
+}
+__device__ inline float2 store_bins(const FftMaps &mp, size_t o, const MapBins &b, bool mine, double &ovf)
+{
+    const float2 fd = make_float2(dev::field_bin(b.fix.x, b.field.x, mp.unit, mp.rho_t),
+                                  dev::field_bin(b.fix.y, b.field.y, mp.unit, mp.rho_t));
+    const float2 mv = make_float2(dev::mov_bin(b.mov.x, mp.unit), dev::mov_bin(b.mov.y, mp.unit));
+    if (mine) {
+        const ulonglong2 zero = {0ull, 0ull};
+        *reinterpret_cast<ulonglong2 *>(mp.acc_field + o) = zero;
+        *reinterpret_cast<ulonglong2 *>(mp.acc_mov + o) = zero;
+        *reinterpret_cast<float2 *>(mp.map_mov + o) = mv;
+        *reinterpret_cast<float2 *>(mp.map_field + o) = fd;
+        ovf += fmax((double)dev::ovf_bin(mv.x, b.fix.x, mp.rho_t, mp.cap), 0.0);
+        ovf += fmax((double)dev::ovf_bin(mv.y, b.fix.y, mp.rho_t, mp.cap), 0.0);
+    }
+    return fd;
+}
+// The tile counts, and the overflow partials of the launch (NT threads per block).
+template <int NT>
+__device__ inline void finish_maps(const FftMaps &mp, int blk, int blocks, double ovf)
+{
+    for (int t = blk * NT + (int)threadIdx.x; t < 2 * kSortTiles; t += blocks * NT) mp.count[t] = 0;
+    for (int p = blocks + blk * NT + (int)threadIdx.x; p < mp.part_blocks; p += blocks * NT) mp.part[4 * p] = 0.0;
+    double v[1] = {ovf};
+    dev::block_reduce<1, 0, NT>(v, mp.part + 4 * blk);
+}
+
 // Rows 2 F blk ... of the map (row length N, `rows` rows, an even number).
-// F * T threads, F * buf points of LDS.
-template <int L, int F>
-__device__ inline void rows_pass(const FftArgs &a, int blk, float2 *lds)
+// F * T threads, F * buf points of LDS.  With MAPS the map is made on the way.
+template <int L, int F, bool MAPS>
+__device__ inline void rows_pass(const FftArgs &a, const FftMaps &mp, int blk, float2 *lds)
 {
     using P = Plan<L>;
     constexpr int N = P::N, T = P::T;
@@ -276,14 +313,34 @@ __device__ inline void rows_pass(const FftArgs &a, int blk, float2 *lds)
     const int halt = *a.skip;
     const float mean = *a.mean;
     float2 xa[4], xb[4];
+    [[maybe_unused]] MapBins ma[4], mb[4];
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
-        xa[m] = x0[t + m * T];
-        xb[m] = x1[t + m * T];
+        if constexpr (MAPS) {
+            const size_t o = (size_t)r0 * N + 2 * (t + m * T);
+            ma[m] = load_bins(mp, o);
+            mb[m] = load_bins(mp, o + N);
+        } else {
+            xa[m] = x0[t + m * T];
+            xb[m] = x1[t + m * T];
+        }
     }
     Twiddles<L> w;
-    load_twiddles<L>(a.tab_y, t, w);
+    if constexpr (!MAPS) load_twiddles<L>(a.tab_y, t, w);
     if (halt) return;
+    [[maybe_unused]] double ovf = 0.0;
+    if constexpr (MAPS) {
+        const bool mine = (blk * F + f) * 2 < rows;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            const size_t o = (size_t)r0 * N + 2 * (t + m * T);
+            xa[m] = store_bins(mp, o, ma[m], mine, ovf);
+            xb[m] = store_bins(mp, o + N, mb[m], mine, ovf);
+        }
+        // not before: with the bins' registers they would not fit (256 and spills)
+        __builtin_amdgcn_sched_barrier(0);
+        load_twiddles<L>(a.tab_y, t, w);
+    }
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
         const int n = t + m * T;
@@ -326,6 +383,7 @@ __device__ inline void rows_pass(const FftArgs &a, int blk, float2 *lds)
         if (row < rows)
             *reinterpret_cast<float4 *>(a.t1 + ((size_t)g * rows + row) * 4) = make_float4(o[0], o[1], o[2], o[3]);
     }
+    if constexpr (MAPS) finish_maps<F * T>(mp, blk, gridDim.x, ovf);
 }
 
 // One value of the spectral scaling: A -> (A wx / k^2, A wy / k^2), the halved
@@ -501,10 +559,10 @@ __device__ inline void field_pass(const FftArgs &a, int blk, float2 *lds)
 
 extern __shared__ __attribute__((aligned(16))) float2 fft_lds[];
 
-template <int L>
-__global__ __launch_bounds__(ffts_of<L>() * Plan<L>::T) void k_fft_rows(FftArgs a)
+template <int L, bool MAPS>
+__global__ __launch_bounds__(ffts_of<L>() * Plan<L>::T) void k_fft_rows(FftArgs a, FftMaps mp)
 {
-    rows_pass<L, ffts_of<L>()>(a, blockIdx.x, fft_lds);
+    rows_pass<L, ffts_of<L>(), MAPS>(a, mp, blockIdx.x, fft_lds);
 }
 template <int L>
 __global__ __launch_bounds__(col_halves_of<L>() * col_ffts_of<L>() * Plan<L>::T) void k_fft_columns(FftArgs a)
@@ -532,6 +590,8 @@ __global__ __launch_bounds__(field_ffts_of<L>() * Plan<L>::T) void k_fft_field(F
 // o / d for 0 <= o < 2^12 and inv = 1 / d rounded: (o + 1/2) / d is further from a whole
 // number than its error.
 __device__ inline int quotient(int o, float inv) { return (int)(((float)o + 0.5f) * inv); }
+
+constexpr int kMixedThreads = 512;
 
 // First stage, r odd, ns = 1, so no twiddles: outputs q and r - q of a butterfly share the
 // sums of cosines and sines over the pairs (i, r - i).  Lanes run over the butterflies:
@@ -670,7 +730,8 @@ __device__ inline float2 half_at(const float2 *__restrict__ tab, float2 first, i
 }
 
 // Rows 2 blk and 2 blk + 1.  3 N points of LDS.
-__device__ __forceinline__ void mixed_rows(const FftArgs &a, const FftPlan &p, int blk, float2 *lds)
+template <bool MAPS>
+__device__ __forceinline__ void mixed_rows(const FftArgs &a, const FftMaps &mp, const FftPlan &p, int blk, float2 *lds)
 {
     const int N = a.My, rows = a.Mx;
     if (*a.skip) return;
@@ -680,8 +741,18 @@ __device__ __forceinline__ void mixed_rows(const FftArgs &a, const FftPlan &p, i
     const float mean = *a.mean;
     const float2 half = first_half(a.tab_y, N);
     load_roots(a.tab_y, root, N);
+    [[maybe_unused]] double ovf = 0.0;
     for (int n = threadIdx.x; n < N / 2; n += blockDim.x) {
-        const float2 xa = x0[n], xb = x1[n];
+        float2 xa, xb;
+        if constexpr (MAPS) {
+            const size_t o = (size_t)2 * blk * N + 2 * n;
+            const MapBins ma = load_bins(mp, o), mb = load_bins(mp, o + N);
+            xa = store_bins(mp, o, ma, true, ovf);
+            xb = store_bins(mp, o + N, mb, true, ovf);
+        } else {
+            xa = x0[n];
+            xb = x1[n];
+        }
         b0[n] = make_float2(xa.x - mean, xb.x - mean);
         b0[N - 1 - n] = make_float2(xa.y - mean, xb.y - mean);
     }
@@ -707,6 +778,7 @@ __device__ __forceinline__ void mixed_rows(const FftArgs &a, const FftPlan &p, i
         }
         *reinterpret_cast<float4 *>(a.t1 + ((size_t)g * rows + 2 * blk + r) * 4) = make_float4(o[0], o[1], o[2], o[3]);
     }
+    if constexpr (MAPS) finish_maps<kMixedThreads>(mp, blk, rows / 2, ovf);
 }
 
 // Columns 2 blk and 2 blk + 1.  5 N points of LDS.
@@ -785,15 +857,13 @@ __device__ __forceinline__ void mixed_field(const FftArgs &a, const FftPlan &p, 
     }
 }
 
-constexpr int kMixedThreads = 512;
-
 // Pass S (rows, columns, field).  Neighbouring rows and columns, which share the
 // layout groups' cache lines, go to one XCD.
-template <int S>
-__global__ __launch_bounds__(kMixedThreads) void k_fft_mixed(FftArgs a)
+template <int S, bool MAPS>
+__global__ __launch_bounds__(kMixedThreads) void k_fft_mixed(FftArgs a, FftMaps mp)
 {
     const int blk = dev::xcd_block(blockIdx.x, gridDim.x);
-    if (S == 0) mixed_rows(a, a.py, blk, fft_lds);
+    if (S == 0) mixed_rows<MAPS>(a, mp, a.py, blk, fft_lds);
     else if (S == 1) mixed_columns(a, a.px, blk, fft_lds);
     else mixed_field(a, a.py, blk, fft_lds);
 }
@@ -807,17 +877,21 @@ __global__ __launch_bounds__(kMixedThreads) void k_fft_mixed_b(const FftArgs *__
     for (int i = threadIdx.x; i < (int)(sizeof(FftPlan) / 4); i += kMixedThreads)
         reinterpret_cast<int *>(&p)[i] = reinterpret_cast<const int *>(&args[t.x].px)[i];
     __syncthreads();
-    if (S == 0) mixed_rows(a, p, t.y, fft_lds);
+    if (S == 0) mixed_rows<false>(a, FftMaps{}, p, t.y, fft_lds);
     else if (S == 1) mixed_columns(a, p, t.y, fft_lds);
     else mixed_field(a, p, t.y, fft_lds);
 }
 
 template <int S>
-void launch_mixed(const FftArgs &a, hipStream_t s)
+void launch_mixed(const FftArgs &a, const FftMaps *maps, hipStream_t s)
 {
     const int n = S == 1 ? a.Mx : a.My, blocks = S == 0 ? a.Mx / 2 : S == 1 ? a.My / 2 : a.Mx;
     const size_t lds = (S == 1 ? 5 : 3) * sizeof(float2) * (size_t)n;
-    hipLaunchKernelGGL(k_fft_mixed<S>, dim3(blocks), dim3(kMixedThreads), lds, s, a);
+    auto go = [&](auto kern, const FftMaps &mp) {
+        hipLaunchKernelGGL(kern, dim3(blocks), dim3(kMixedThreads), lds, s, a, mp);
+    };
+    if (S == 0 && maps) go(k_fft_mixed<S, S == 0>, *maps);
+    else go(k_fft_mixed<S, false>, FftMaps{});
 }
 
 // ------------------------------------------------------------------ batches
@@ -828,7 +902,7 @@ template <int NT, int S, int L>
 __device__ inline void batch_tile(const FftArgs &a, int blk)
 {
     constexpr int F = NT / Plan<L>::T;
-    if (S == 0) rows_pass<L, F>(a, blk, fft_lds);
+    if (S == 0) rows_pass<L, F, false>(a, FftMaps{}, blk, fft_lds);
     else if (S == 1) columns_pass<L, F, 1>(a, blk, fft_lds);
     else field_pass<L, F>(a, blk, fft_lds);
 }
@@ -937,22 +1011,37 @@ void fft_table(int n, std::vector<float2> &tab)
     }
 }
 
-void launch_field_fft(const FftArgs &a, hipStream_t s)
+int fft_row_blocks(int Mx, int My)
+{
+    if (!fft_pow2(My)) return Mx / 2;
+    int blocks = 0;
+    with_length(log2_of(My), [&](auto c) {
+        constexpr int F = ffts_of<decltype(c)::value>();
+        blocks = (Mx + 2 * F - 1) / (2 * F);
+    });
+    return blocks;
+}
+
+void launch_field_fft(const FftArgs &a, const FftMaps *maps, hipStream_t s)
 {
     const int lx = log2_of(a.Mx), ly = log2_of(a.My);
-    if (!fft_pow2(a.My)) launch_mixed<0>(a, s);
+    if (!fft_pow2(a.My)) launch_mixed<0>(a, maps, s);
     else with_length(ly, [&](auto c) {
         constexpr int L = decltype(c)::value, F = ffts_of<L>();
-        hipLaunchKernelGGL(k_fft_rows<L>, dim3((a.Mx + 2 * F - 1) / (2 * F)), dim3(F * Plan<L>::T),
-                           F * Plan<L>::buf * sizeof(float2), s, a);
+        auto go = [&](auto kern, const FftMaps &mp) {
+            hipLaunchKernelGGL(kern, dim3(fft_row_blocks(a.Mx, a.My)), dim3(F * Plan<L>::T),
+                               F * Plan<L>::buf * sizeof(float2), s, a, mp);
+        };
+        if (maps) go(k_fft_rows<L, true>, *maps);
+        else go(k_fft_rows<L, false>, FftMaps{});
     });
-    if (!fft_pow2(a.Mx)) launch_mixed<1>(a, s);
+    if (!fft_pow2(a.Mx)) launch_mixed<1>(a, nullptr, s);
     else with_length(lx, [&](auto c) {
         constexpr int L = decltype(c)::value, F = col_ffts_of<L>();
         hipLaunchKernelGGL(k_fft_columns<L>, dim3((a.My + 2 * F - 1) / (2 * F)),
                            dim3(col_halves_of<L>() * F * Plan<L>::T), 2 * F * Plan<L>::buf * sizeof(float2), s, a);
     });
-    if (!fft_pow2(a.My)) launch_mixed<2>(a, s);
+    if (!fft_pow2(a.My)) launch_mixed<2>(a, nullptr, s);
     else with_length(ly, [&](auto c) {
         constexpr int L = decltype(c)::value, F = field_ffts_of<L>();
         hipLaunchKernelGGL(k_fft_field<L>, dim3((a.Mx + F - 1) / F), dim3(F * Plan<L>::T),

@@ -853,7 +853,7 @@ void field_free(Ctx &c)
     c.map_mean = nullptr;
 }
 
-void launch_field(Ctx &c, int precision, hipStream_t s)
+static void launch_solve(Ctx &c, int precision, bool maps, hipStream_t s)
 {
     FieldMats *fm = static_cast<FieldMats *>(c.split_mats);
     const size_t nb = (size_t)c.Mx * c.My;
@@ -866,9 +866,12 @@ void launch_field(Ctx &c, int precision, hipStream_t s)
     if (fm->fft_x) {
         FftArgs f{c.map_field, c.map_mean, a.skip, fm->fft_x, fm->fft_y, c.tA, reinterpret_cast<float2 *>(c.tB),
                   c.exy, c.Mx, c.My, a.scale, a.wxs, a.wys, fft_plan(c.Mx), fft_plan(c.My)};
-        launch_field_fft(f, s);
+        const FftMaps m{c.acc_field, c.acc_mov, c.map_fix, c.map_field, c.map_mov, c.dens_unit(),
+                        c.prm.target_density, c.bin_cap(), c.part + c.part_ovf_off, c.ovf_blocks, c.sort_count};
+        launch_field_fft(f, maps ? &m : nullptr, s);
         return;
     }
+    if (maps) launch_overflow(c, s);
     auto setA = [&](int z, int m) { set_operand(a, z, fm->half[m], m, precision); };
     if (f16) {
         launch_map_range(c, s);
@@ -901,6 +904,14 @@ void launch_field(Ctx &c, int precision, hipStream_t s)
     a.c_pair = 1;
     a.bmax = fm->fmax + 3; a.cmax = nullptr;
     gemm(a, 2, true, 0, precision, s);
+}
+
+void launch_field(Ctx &c, int precision, hipStream_t s) { launch_solve(c, precision, false, s); }
+void launch_overflow_field(Ctx &c, int precision, hipStream_t s)
+{
+    const bool joint = c.n_place < kForkMinCells;
+    if (!joint) launch_overflow(c, s);
+    launch_solve(c, precision, joint, s);
 }
 
 // FP64 field of the current map into the reference scratch, then the max-norm

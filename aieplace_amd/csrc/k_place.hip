@@ -1126,10 +1126,8 @@ void launch_density_pins(Ctx &c, hipStream_t s)
 void launch_overflow(Ctx &c, hipStream_t s)
 {
     const int nb = c.Mx * c.My;
-    const float cap = c.prm.target_density * c.bw * c.bh;
-    const double unit = (double)c.bw * (double)c.bh / kDensFixUnits;
     hipLaunchKernelGGL(k_overflow, dim3(c.ovf_blocks), dim3(kBlock), 0, s, c.acc_field, c.acc_mov,
-                       c.map_fix, unit, c.prm.target_density, cap, nb, c.map_field, c.map_mov,
+                       c.map_fix, c.dens_unit(), c.prm.target_density, c.bin_cap(), nb, c.map_field, c.map_mov,
                        c.part + c.part_ovf_off, c.sort_count, c.d_scal);
 }
 

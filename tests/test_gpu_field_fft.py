@@ -99,3 +99,26 @@ def test_batch_of_mixed_sides():
             sx, sy = pl.get_positions()
         print(f"  bins {b}", flush=True)
         assert np.array_equal(x, sx) and np.array_equal(y, sy), b
+
+
+# powers of two with one and several rows per block, blocks past the last row, a long
+# grid in each direction, sides that are none
+@pytest.mark.parametrize("mx,my", [(16, 16), (48, 64), (16, 1024), (1024, 32), (256, 256), (400, 240), (64, 976),
+                                   (16, 8192)])
+def test_rows_make_the_maps(mx, my):
+    """The map pass inside the field solve (gradient) against the one by itself
+    (computeOverlaps): equal maps, an equal overflow up to the order of its FP64 sum,
+    and cleared accumulators (a second pass gives the same)."""
+    print(f"case rows maps {mx} x {my}", flush=True)
+    nl = A.generate("stdcell", seed=1, n_movable=3_000)
+    p = A.placer_params(A.CONFIGS["stdcell_200k"], bins_x=mx, bins_y=my)
+    with A.Placer(nl, p) as pl:
+        field, mov, _, tau = pl.computeOverlaps()
+        for _ in range(2):
+            g = pl.gradient(1.0, 1.0)
+            made = [np.zeros(pl.bins, np.float32) for _ in range(2)]
+            api.check(api.lib.ep_get_density(pl._ctx, api.fptr(made[0]), api.fptr(made[1]), None))
+            assert np.array_equal(made[0], field) and np.array_equal(made[1], mov)
+            assert g["tau"] == pytest.approx(tau, rel=mx * my * 2.0 ** -52)
+        again = pl.computeOverlaps()
+    assert np.array_equal(again[0], field) and np.array_equal(again[1], mov) and again[3] == tau
