@@ -658,7 +658,7 @@ extern "C" ep_status ep_create(const ep_netlist *nl, const ep_params *p, ep_ctx 
     EP_TRY(dalloc(&c->pin_off, L.n_pins));
     EP_TRY(dalloc(&c->pin_grad, L.n_pins));
     EP_TRY(dalloc(&c->cell_pin_start, c->n_mov + 1));
-    EP_TRY(dalloc(&c->gw_cell, std::max(1, c->n_mov)));
+    EP_TRY(dalloc(&c->gw_cell, std::max(1, c->n_place)));
     EP_TRY(dalloc(&c->cell_pins, L.cpins.size()));
     for (int i = 0; i < 2; ++i) {
         EP_TRY(dalloc(&c->V[i], c->n_all));
@@ -707,6 +707,7 @@ extern "C" ep_status ep_create(const ep_netlist *nl, const ep_params *p, ep_ctx 
         }
     }
     if (hipMemset(c->pin_grad, 0, sizeof(float2) * std::max(1, L.n_pins)) != hipSuccess ||
+        hipMemset(c->gw_cell, 0, sizeof(float2) * std::max(1, c->n_place)) != hipSuccess ||
         hipMemset(c->exy, 0, sizeof(float2) * nb) != hipSuccess ||
         hipMemset(c->part, 0, sizeof(double) * c->part_total) != hipSuccess ||
         hipMemset(c->fin_ticket, 0, sizeof(unsigned)) != hipSuccess ||
@@ -926,14 +927,11 @@ extern "C" ep_status ep_get_wa_grad(ep_ctx *c, float *gx, float *gy)
     if (!c) return fail(EP_EINVAL, "ep_get_wa_grad: null context");
     c->h_scal->lambda = 0.0f;
     push_scalars(*c, c->stream);
-    // the other parity's buffers hold a past trial
-    float2 *scratch = c->G[c->cur ^ 1], *gw = c->U[c->cur ^ 1];
     launch_pin_sum(*c, c->stream);
-    launch_cell_grad(*c, c->V[c->cur], nullptr, nullptr, scratch, gw, nullptr, c->stream);
     ep_status st = check_launch();
     if (st != EP_OK) return st;
     StageOut out(c->stage);
-    st = cell_pairs(out, c, gw, gx, gy);
+    st = cell_pairs(out, c, c->gw_cell, gx, gy);
     const ep_status fin = out.finish();
     if (st != EP_OK || fin != EP_OK) return st != EP_OK ? st : fin;
     return sync(*c);

@@ -337,7 +337,7 @@ struct Ctx {
     float2 *wh = nullptr;
     int32_t *net_start = nullptr, *pin_cell = nullptr;
     float2 *pin_off = nullptr, *pin_grad = nullptr;
-    float2 *gw_cell = nullptr;  // per movable cell: sum of its pin partials
+    float2 *gw_cell = nullptr;  // [n_place] per movable cell the sum of its pin partials, 0 for fillers
     int32_t *cell_pin_start = nullptr, *cell_pins = nullptr;
     BucketTable buckets{};
     int32_t wa_blocks = 0;

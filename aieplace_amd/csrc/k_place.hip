@@ -500,7 +500,7 @@ __global__ __launch_bounds__(kBlock) void k_cell_grad(
         // n_mov + 1 entries, so a fixed cell or filler reads k0 == k1 (no pins).
         const bool mov = c < n_mov;
         const int k0 = cell_pin_start[min(c, n_mov)], k1 = cell_pin_start[min(c + 1, n_mov)];
-        const float2 gwc = gw_cell[max(0, min(c, n_mov - 1))];  // holds max(1, n_mov) entries
+        const float2 gwc = gw_cell[max(0, min(c, n_mov - 1))];  // a filler's would be 0
         const int np = k1 - k0;
         const float2 f = cell_force(p, s, exy, g, Mx, My);
         const float2 gw = mov ? gwc : make_float2(0.f, 0.f);

@@ -27,6 +27,16 @@ __global__ __launch_bounds__(kStageBlock) void k_unpack(const float2 *__restrict
     }
 }
 
+// n floats, whole float4s while they last (both ends 16-byte aligned).
+__global__ __launch_bounds__(kStageBlock) void k_download(const float *__restrict__ src, int64_t n,
+                                                          float *__restrict__ out)
+{
+    const int64_t t = (int64_t)blockIdx.x * kStageBlock + threadIdx.x, step = (int64_t)gridDim.x * kStageBlock;
+    for (int64_t i = t; i < n / 4; i += step)
+        reinterpret_cast<float4 *>(out)[i] = reinterpret_cast<const float4 *>(src)[i];
+    for (int64_t i = n / 4 * 4 + t; i < n; i += step) out[i] = src[i];
+}
+
 __global__ __launch_bounds__(kStageBlock) void k_place_cells(const float *__restrict__ x, const float *__restrict__ y,
                                                              const int32_t *__restrict__ order, int64_t n_order,
                                                              const float2 *__restrict__ wh, int64_t n, float4 die,
@@ -58,6 +68,8 @@ ep_status stage_init(Stage &st, hipStream_t stream, size_t most)
     char *p = nullptr;
     if (hipHostMalloc((void **)&p, 2 * st.bytes + 256, hipHostMallocDefault) != hipSuccess)
         return fail(EP_ENOMEM, "pinned host allocation failed");
+    // the host's first touch of a megabyte's pages takes 110 us: here, not in the first transfer
+    std::memset(p, 0, 2 * st.bytes + 256);
     st.pin[0] = p;
     st.pin[1] = p + st.bytes;
     st.flag = reinterpret_cast<int32_t *>(p + 2 * st.bytes);
@@ -132,10 +144,18 @@ ep_status StageOut::flat(const float *src, int64_t n, float *out)
         ep_status s = take();
         if (s != EP_OK) return s;
         const int64_t m = std::min(per, n - o);
-        s = hip_ok(hipMemcpyAsync(st_.pin[next_], src + o, (size_t)m * sizeof(float), hipMemcpyDeviceToHost,
-                                  st_.stream),
-                   "download");
-        if (s != EP_OK) return s;
+        float *pin = reinterpret_cast<float *>(st_.pin[next_]);
+        if (n <= per) {
+            // a kernel starts sooner than the copy engine (three maps of 128^2, 224^2, 480^2:
+            // 92 / 104 / 186 us a call, 103 / 120 / 199 with copies), but chunks that follow
+            // each other are slower with it (three of 1024^2: 826, 764 with copies)
+            const unsigned blocks = (unsigned)((m / 4 + kStageBlock) / kStageBlock);
+            hipLaunchKernelGGL(k_download, dim3(blocks), dim3(kStageBlock), 0, st_.stream, src, m, pin);
+        } else {
+            s = hip_ok(hipMemcpyAsync(pin, src + o, (size_t)m * sizeof(float), hipMemcpyDeviceToHost, st_.stream),
+                       "download");
+            if (s != EP_OK) return s;
+        }
         piece_[next_].dst[0] = out + o;
         piece_[next_].dst[1] = nullptr;
         piece_[next_].n = (size_t)m;
