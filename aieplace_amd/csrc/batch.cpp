@@ -729,7 +729,16 @@ extern "C" ep_status ep_batch_run(ep_batch *b, int32_t max_launches, ep_batch_ru
     // replay runs.  Decisions therefore see the state one replay late: a
     // replay queued after every instance has stopped returns at once (stopped
     // instances skip their work), and the block tables are rebuilt only after
-    // the stream has drained.
+    // the stream has drained.  No replay is queued behind one that likely
+    // brings every instance to the iteration limit (as in run_device).
+    auto near_end = [&]() {
+        for (int i = 0; i < b->n; ++i) {
+            const BState &S = b->h_st[i];
+            const double per = S.iteration > 0 ? (double)S.evals / S.iteration : 1.0;
+            if (!S.done && (b->prm.max_iters - S.iteration) * per > kTrialsPerLaunch) return false;
+        }
+        return true;
+    };
     int slot = 0, last = -1;
     bool pending = false;  // h_rb[slot ^ 1] holds a queued read-back not yet checked
     for (;;) {
@@ -760,7 +769,12 @@ extern "C" ep_status ep_batch_run(ep_batch *b, int32_t max_launches, ep_batch_ru
             }
         }
         if (!launch) break;
-        pending = true;
+        pending = !near_end();
+        if (!pending) {
+            EPB_HIP(hipEventSynchronize(b->rb_done[slot]));
+            std::memcpy(b->h_st, b->h_rb[slot], st_bytes);
+            if ((st = check_errors(b)) != EP_OK) return st;
+        }
         slot ^= 1;
     }
     EPB_HIP(hipStreamSynchronize(b->stream));

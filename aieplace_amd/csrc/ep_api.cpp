@@ -1216,9 +1216,10 @@ extern "C" ep_status ep_step(ep_ctx *c, ep_step_info *info)
 // The kernels take the current and trial buffers from Pair arguments indexed
 // by the device's `cur`, so the same graph serves every trial; the host
 // replays it kCtlReplays times per batch and reads the control state back
-// after each batch.  Two batches are in flight: the host waits for the state
-// of one while the next one runs, so the GPU does not idle for the host's
-// round trip.  After the stop the remaining trials return at once (halt flag).
+// after each batch.  Two batches are in flight, except near the iteration limit:
+// the host waits for the state of one while the next one runs, so the GPU does
+// not idle for the host's round trip.  After the stop the remaining trials
+// return at once (halt flag).
 
 constexpr int kCtlTrialsPerGraph = 8;  // one replay per read-back (a graph boundary costs ~3.5 us)
 constexpr int kCtlReplays = 1;
@@ -1357,19 +1358,37 @@ static ep_status run_device(ep_ctx *c, ep_step_info *log, int32_t log_cap, int *
     if ((st = check_launch()) != EP_OK) return st;
     // batch b reads the state back into slot b % 2; the state upload above has
     // left slot 0 before batch 0's read-back is queued behind it on the stream
-    int slot = 0;
-    for (int64_t b = 0;; ++b, slot ^= 1) {
+    const int it0 = c->iteration;
+    const int64_t ev0 = c->evals;
+    int iteration = it0;          // in the latest state read
+    double per_iteration = 1.0;   // trials, so far
+    bool stopped = false;
+    auto wait = [&](int k) -> ep_status {
+        const hipError_t e = hipEventSynchronize(c->ctl_read[k]);
+        if (e != hipSuccess) return fail(EP_EDEVICE, "ep_run: %s", hipGetErrorString(e));
+        const DevCtl &S = c->h_ctl[k];
+        stopped = S.done || S.error;
+        iteration = S.iteration;
+        if (iteration > it0) per_iteration = (double)(S.evals - ev0) / (iteration - it0);
+        return EP_OK;
+    };
+    int slot = 1;
+    for (bool older = false;;) {  // older: the batch before `slot`'s is not read yet
+        slot ^= 1;
         for (int r = 0; r < kCtlReplays; ++r) EP_HIP(hipGraphLaunch(c->ctl_exec, c->stream));
         EP_HIP(hipMemcpyAsync(c->h_ctl + slot, c->d_ctl, sizeof(DevCtl), hipMemcpyDeviceToHost, c->stream));
         EP_HIP(hipEventRecord(c->ctl_read[slot], c->stream));
-        if (b == 0) continue;
-        const hipError_t e = hipEventSynchronize(c->ctl_read[slot ^ 1]);
-        if (e != hipSuccess) return fail(EP_EDEVICE, "ep_run: %s", hipGetErrorString(e));
-        const DevCtl &P = c->h_ctl[slot ^ 1];
-        if (P.done || P.error) break;
+        if (older && (st = wait(slot ^ 1)) != EP_OK) return st;
+        if (stopped) break;
+        // The batch in flight is likely the last one: no batch behind it.  One that
+        // finds the run stopped takes 130 us for its 8 x 8 launches, a wait for the
+        // state between two batches 15 us.
+        older = (p.max_iters - iteration) * per_iteration > kCtlReplays * kCtlTrialsPerGraph;
+        if (!older && (st = wait(slot)) != EP_OK) return st;
+        if (stopped) break;
     }
-    // the batch queued after the stop returned at once: the last read-back
-    // (slot) holds the final state
+    // a batch queued after the stop returned at once: the last read-back (slot)
+    // holds the final state
     if ((st = sync(*c)) != EP_OK) return st;
     DevCtl &H = c->h_ctl[slot];
     const int n = std::min(H.n_log, c->ctl_cap);

@@ -62,3 +62,30 @@ def test_batch_shared_launches_equal_forked(counts):
         out.append([a for i in range(len(counts)) for a in bp.positions(i)])
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+# limits on both sides of one and two batches of trials (8 in a single run, 4 in a
+# batch), where the host stops queueing ahead
+@pytest.mark.parametrize("limit", [1, 3, 4, 5, 7, 8, 9, 16, 17])
+def test_iteration_limit(limit):
+    """Device-controlled and batched runs stop at the limit where the host loop does, and
+    a second run does nothing."""
+    from aieplace_amd.batch import BatchPlacer
+    print(f"case iteration limit {limit}", flush=True)
+    nl = A.generate("stdcell", seed=4, n_movable=2_000)
+    out = []
+    for graph in (0, 1):
+        p = A.placer_params(A.CONFIGS["stdcell_200k"], bins_x=64, bins_y=64, use_graph=graph, max_iters=limit)
+        with A.Placer(nl, p) as pl:
+            r = pl.run()
+            assert r["iterations"] == limit
+            assert pl.run()["evals"] == 0
+            out.append((r["evals"], *pl.get_positions()))
+    bp = BatchPlacer([nl], [64], p)
+    bp.run()
+    r = bp.results()
+    assert r["iterations"][0] == limit
+    out.append((r["evals"][0], *bp.positions(0)))
+    for other in out[1:]:
+        for a, b in zip(out[0], other):
+            assert np.array_equal(a, b)
