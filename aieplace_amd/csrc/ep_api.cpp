@@ -1019,11 +1019,17 @@ extern "C" ep_status ep_init_optimizer(ep_ctx *c)
     ep_status st = run_density(c);
     if (st != EP_OK) return st;
     c->gamma = gamma_of(*c, c->h_res->tau);
-    // gradient pieces at v_0 with lambda = 0 give |gW|_1 and |F|_1
+    // gradient pieces at v_0 with lambda = 0 give |gW|_1 and |F|_1; the density maps
+    // and the overflow's partial sums are there
     c->h_scal->gamma_inv = (float)(1.0 / c->gamma);
     c->h_scal->lambda = 0.0f;
     push_scalars(*c, c->stream);
-    enqueue_eval(*c, c->V[a], nullptr, nullptr, c->G[a], nullptr, nullptr, c->stream);
+    launch_wa(*c, c->V[a], c->stream);
+    launch_pin_sum(*c, c->stream);
+    launch_field(*c, c->prm.precision, c->stream);
+    launch_cell_grad(*c, c->V[a], nullptr, nullptr, c->G[a], nullptr, nullptr, c->stream);
+    launch_finalize(*c, c->stream);
+    (void)hipMemcpyAsync(c->h_res, c->d_res, sizeof(DevResult), hipMemcpyDeviceToHost, c->stream);
     if ((st = check_launch()) != EP_OK || (st = sync(*c)) != EP_OK) return st;
     c->evals++;
     const double sw = c->h_res->sum_gw, sf = c->h_res->sum_f;
