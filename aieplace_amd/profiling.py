@@ -290,11 +290,6 @@ def batch_stats(args) -> str:
 
 # ---------------------------------------------------------------- traffic
 
-# kernel dispatches per call of each ep_profile item (field: 4 products, plus
-# the maxima reset of the split-FP16 form)
-DISPATCHES = {"cell_sort": 3, "overflow": 2, "field_transforms": 4}
-
-
 def _dispatches(rows, counter):
     """[(dispatch id, kernel, KiB)] of one counter, in dispatch order."""
     out = [(int(r["Dispatch_Id"]), _short(r["Kernel_Name"]), float(r["Counter_Value"]))
@@ -371,7 +366,7 @@ def traffic(args) -> str:
                      f"{fetch.get(k, 0.0) * 1024 * f_fetch / 1e6:.3f} |")
     summary = {}
     for fam, q in prof.items():
-        n_disp = DISPATCHES.get(fam, 1) + (1 if fam == "field_transforms" and args.precision == 2 else 0)
+        n_disp = int(q["launches"])
         fb = _per_call(disp["FETCH_SIZE"], fam, n_disp, args.reps) * 1024 * f_fetch
         wb = _per_call(disp["WRITE_SIZE"], fam, n_disp, args.reps) * 1024 * f_write
         if fb + wb > 0:

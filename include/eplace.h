@@ -37,9 +37,9 @@ enum {
     EP_EIO = 7       /* file missing, unreadable or malformed (LEF/DEF)   */
 };
 
-/* Arithmetic of the field-solve transform products.  Grids whose sides are powers
- * of two (up to 8192) need no products: FP32 FFTs solve them in every form, closer
- * to the exact field than any of the products. */
+/* Arithmetic of the field-solve transform products.  Grids with both sides up to 4080,
+ * or powers of two up to 8192, need no products: FP32 FFTs solve them in every form,
+ * closer to the exact field than any of the products. */
 enum {
     EP_PREC_FP32 = 0,   /* FP32 operands, FP32 MFMA (v_mfma_f32_32x32x2_f32)        */
     EP_PREC_BF16X3 = 1, /* operands split hi+lo BF16, 3 MFMA products, FP32 accum */
