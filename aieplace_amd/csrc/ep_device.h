@@ -425,7 +425,7 @@ __device__ inline void sort_tables(const int *start, int32_t *__restrict__ off, 
     if (t == kBlock - 1) dtab[ns] = run;
 }
 
-// Super tile s of density block b (dtab as written by sort_scan_block).
+// Super tile s of density block b (dtab as written by sort_tables).
 __device__ inline int dens_super_tile(const int32_t *__restrict__ dtab, int ns, int b)
 {
     int lo = 0, hi = ns;
