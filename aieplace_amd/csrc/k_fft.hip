@@ -19,8 +19,8 @@
 //
 // Why FFTs: the products execute 6.4 GFLOP per 1024^2 solve, the FFTs 0.16 GFLOP
 // over 36 MB of L2/MALL traffic.  One solve alone, FP32 products -> FFTs: 32^2
-// 14.8 -> 9.2 us, 128^2 23.6 -> 14.9, 256^2 31.5 -> 15.4, 512^2 48 -> 18.4, 1024^2
-// 108 -> 33 (split-BF16 products 72), 2048^2 585 -> 82; max-norm error at most
+// 14.8 -> 9.2 us, 128^2 23.6 -> 14.9, 256^2 31.5 -> 15.3, 512^2 48 -> 17.5, 1024^2
+// 108 -> 32 (split-BF16 products 72), 2048^2 585 -> 70; max-norm error at most
 // 5e-7 (products: FP32 3e-6, split-BF16 1.1e-5).  What bounds them is latency:
 // one wave per SIMD at 1024^2, where a kernel without its butterflies takes 5-10
 // us, without its stores 1.5-3 us less, and with free twiddles or LDS exchanges
@@ -29,8 +29,8 @@
 // groups against channel conflicts changed nothing either.
 //
 // Layout of T1 (float) and PQ (float2): [v/4][i][v%4].  The column kernel reads
-// and writes whole runs; a block of the row kernels touches 4 consecutive rows,
-// runs of 64 and 128 bytes.
+// and writes whole runs; a block of the row kernels touches two consecutive
+// rows, runs of 32 and 64 bytes of lines that the XCD's next blocks complete.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -236,29 +236,31 @@ __device__ inline void idct_pair(float a_k, float a_n, float b_k, float b_n, flo
     zn = make_float2(0.5f * (p + u), 0.5f * (r - q));
 }
 
-// FFTs per block: two (so that the four rows or columns of a layout group stay
-// together), more where one FFT is less than half a wave's threads.
+// FFTs per block: one where that is a wave or more, so that a 512^2 map occupies every
+// CU; neighbouring blocks, which share the layout groups' cache lines, then go to one
+// XCD.  One solve with two FFTs per block and four rows per field block / as now: 512^2
+// 18.7 / 17.5 us, 1024^2 32.9 / 32.0, 2048^2 81 / 70.
 template <int L>
 constexpr int ffts_of()
 {
-    return Plan<L>::T >= 1024 ? 1 : Plan<L>::T >= 32 ? 2 : 64 / Plan<L>::T;
+    return Plan<L>::T >= 64 ? 1 : Plan<L>::T >= 32 ? 2 : 64 / Plan<L>::T;
 }
-// The column kernel's FFTs and its threads per FFT point set (see columns_pass).
+template <int L>
+__device__ inline int fft_block()
+{
+    return Plan<L>::T >= 64 ? dev::xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
+}
+// The column kernel's threads per FFT point set (see columns_pass).
 template <int L>
 constexpr int col_halves_of()
 {
     return Plan<L>::T >= 1024 ? 1 : 2;
 }
-template <int L>
-constexpr int col_ffts_of()
-{
-    return Plan<L>::T >= 512 ? 1 : ffts_of<L>();
-}
-// The last kernel's: one row each, so four where the block stays below 1024 threads.
+// The last kernel's: one row each, so two (four of 128).
 template <int L>
 constexpr int field_ffts_of()
 {
-    return Plan<L>::T >= 1024 ? 1 : Plan<L>::T >= 512 ? 2 : Plan<L>::T >= 16 ? 4 : 64 / Plan<L>::T;
+    return Plan<L>::T >= 1024 ? 1 : Plan<L>::T >= 32 ? 2 : Plan<L>::T >= 16 ? 4 : 64 / Plan<L>::T;
 }
 
 // Bins o and o + 1 of the map (o even) from their accumulators, which are cleared; adds
@@ -562,17 +564,17 @@ extern __shared__ __attribute__((aligned(16))) float2 fft_lds[];
 template <int L, bool MAPS>
 __global__ __launch_bounds__(ffts_of<L>() * Plan<L>::T) void k_fft_rows(FftArgs a, FftMaps mp)
 {
-    rows_pass<L, ffts_of<L>(), MAPS>(a, mp, blockIdx.x, fft_lds);
+    rows_pass<L, ffts_of<L>(), MAPS>(a, mp, fft_block<L>(), fft_lds);
 }
 template <int L>
-__global__ __launch_bounds__(col_halves_of<L>() * col_ffts_of<L>() * Plan<L>::T) void k_fft_columns(FftArgs a)
+__global__ __launch_bounds__(col_halves_of<L>() * ffts_of<L>() * Plan<L>::T) void k_fft_columns(FftArgs a)
 {
-    columns_pass<L, col_ffts_of<L>(), col_halves_of<L>()>(a, blockIdx.x, fft_lds);
+    columns_pass<L, ffts_of<L>(), col_halves_of<L>()>(a, fft_block<L>(), fft_lds);
 }
 template <int L>
 __global__ __launch_bounds__(field_ffts_of<L>() * Plan<L>::T) void k_fft_field(FftArgs a)
 {
-    field_pass<L, field_ffts_of<L>()>(a, blockIdx.x, fft_lds);
+    field_pass<L, field_ffts_of<L>()>(a, fft_block<L>(), fft_lds);
 }
 
 // ------------------------------------------------------------------ other lengths
@@ -1037,7 +1039,7 @@ void launch_field_fft(const FftArgs &a, const FftMaps *maps, hipStream_t s)
     });
     if (!fft_pow2(a.Mx)) launch_mixed<1>(a, nullptr, s);
     else with_length(lx, [&](auto c) {
-        constexpr int L = decltype(c)::value, F = col_ffts_of<L>();
+        constexpr int L = decltype(c)::value, F = ffts_of<L>();
         hipLaunchKernelGGL(k_fft_columns<L>, dim3((a.My + 2 * F - 1) / (2 * F)),
                            dim3(col_halves_of<L>() * F * Plan<L>::T), 2 * F * Plan<L>::buf * sizeof(float2), s, a);
     });
