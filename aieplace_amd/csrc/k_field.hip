@@ -709,8 +709,9 @@ static size_t place_halves(int M, void *mem, HalfMats &hm)
 //   forward (T[f][x]):  E[r][x] = T[2r][x],  O[r][x] = T[2r+1][x]     (x < M/2)
 //   inverse (T'[x][f]): E[x][r] = T'[x][2r], O[x][r] = T'[x][2r+1]    (x < M/2)
 // with T[f][x] = cos|sin(pi f (x + 1/2) / M) and T' its transpose.  The angle is
-// pi m / 2M with the integer m = f (2x + 1), reduced exactly mod 4M; FP64, then
-// rounded to FP32 and split.  Bound by FP64 arithmetic, 2-3 us up to 1024 x 1024.
+// pi m / 2M with the integer m = f (2x + 1), reduced exactly mod 4M (in 64 bits where
+// it passes 2^32: that division for every side takes a 1008-point transform from 515 to
+// 535 us); FP64, then rounded to FP32 and split.  Bound by FP64 arithmetic, 2-3 us up to 1024 x 1024.
 // Made on the host, the matrices were most of a standalone transform: 512 x 512 6.5
 // ms, 0.24 with them made here, one allocation per call and no staging of plain rows.
 __global__ __launch_bounds__(256) void k_halves(HalfMats hm, int M, int sine, int inverse)
@@ -720,7 +721,8 @@ __global__ __launch_bounds__(256) void k_halves(HalfMats hm, int M, int sine, in
     if (e >= (uint32_t)h * h) return;
     const uint32_t row = e / h, col = e - row * h;
     const uint32_t f = 2 * (inverse ? col : row) + odd, x = inverse ? row : col;
-    const double t = (double)(f * (2 * x + 1) % (4u * M)) / (2.0 * M);
+    const uint32_t m = M <= 65536 ? f * (2 * x + 1) % (4u * M) : (uint32_t)((uint64_t)f * (2 * x + 1) % (4ull * M));
+    const double t = (double)m / (2.0 * M);
     const float v = (float)(sine ? sinpi(t) : cospi(t));
     hm.f32[odd][e] = v;
     auto bf16 = [](float a, float &back) {  // rounded to nearest even
@@ -746,7 +748,9 @@ static void launch_halves(const HalfMats &hm, int M, int slot, hipStream_t s)
 static ep_status make_halves(int M, int slot, HalfMats &hm)
 {
     const size_t bytes = place_halves(M, nullptr, hm);
-    if (hipMalloc(&hm.mem, bytes) != hipSuccess)
+    // k_halves counts a half's elements in 32 bits; the three matrices of a side above
+    // 131070 would take 309 GB
+    if (M / 2 > 65535 || hipMalloc(&hm.mem, bytes) != hipSuccess)
         return fail(EP_ENOMEM, "field: hipMalloc of transform matrices failed");
     place_halves(M, hm.mem, hm);
     launch_halves(hm, M, slot, nullptr);

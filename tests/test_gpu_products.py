@@ -127,3 +127,27 @@ def test_batch_of_products_and_ffts(precision, fork):
             pl.run()
             sx, sy = pl.get_positions()
         assert np.array_equal(x, sx) and np.array_equal(y, sy), b
+
+
+@pytest.mark.gpu
+def test_side_above_65536():
+    """A side whose matrix angles f (2 x + 1) pass 2^32.  Cells of one bin on every other
+    bin around the middle: the map's spectrum sits at the highest frequencies.  The
+    matrices take 83 GB of device memory."""
+    mx, my = 68_000, 16
+    print(f"case field products {mx} x {my}", flush=True)
+    i, j = np.meshgrid(np.arange(32_000, 36_000, 2), np.arange(my), indexing="ij")
+    on = np.random.default_rng(1).random(i.shape) < 0.5
+    i, j = i[on], j[on]
+    none = np.zeros(0, np.float32)
+    nl = A.Netlist(die=(0, 0, mx, my), n_mov=len(i), w=np.ones(len(i)), h=np.ones(len(i)), x=i, y=j, net_start=np.zeros(1),
+                   pin_cell=none, pin_dx=none, pin_dy=none)
+    p = A.placer_params(A.CONFIGS["stdcell_200k"], bins_x=mx, bins_y=my, use_fillers=0)
+    with A.Placer(nl, p) as pl:
+        fmap = pl.computeOverlaps()[0]
+        fields = [pl.computeElectricFields(k) for k in PRECISIONS]
+    want = fft_field(fmap.astype(np.float64), 1.0)
+    for k, got in zip(PRECISIONS, fields):
+        err = [np.abs(g - e).max() / np.abs(e).max() for g, e in zip(got, want)]
+        print(f"  precision {k}: {err[0]:.2e} {err[1]:.2e} (tolerance {tolerance(mx, my, k):.2e})", flush=True)
+        assert max(err) <= tolerance(mx, my, k)
