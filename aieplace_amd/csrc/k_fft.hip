@@ -632,6 +632,47 @@ __device__ __forceinline__ void mixed_first(const float2 *__restrict__ in, float
     }
 }
 
+// The same with a long radix, outputs 2 p and 2 p + 1 per item: they share the sums and
+// differences of a pair, so that LDS, which bounds the stage, is read four times for two
+// terms and not six.  Same operations per output.  One and two outputs per item, us per
+// solve: 4016 x 16 (251) 114 / 92 (split-BF16 products 107), 4016^2 1690 / 1317, 2032^2
+// (127) 191 / 162, 1808^2 (113) 169 / 164.
+template <bool INV>
+__device__ __forceinline__ void mixed_first_two(const float2 *__restrict__ in, float2 *__restrict__ out,
+                                                const float2 *root, int N, int C, int r)
+{
+    const int half = (r - 1) / 2, jump = N / r, items = jump * (half / 2 + 1);
+    const float inv = 1.0f / (float)jump;
+    for (int e = threadIdx.x; e < C * items; e += blockDim.x) {
+        const int c = e >= items ? 1 : 0, w = e - c * items;
+        const int p = quotient(w, inv), g = w - p * jump;
+        const float2 *x = in + c * N + g;
+        float2 cs[2] = {x[0], x[0]}, sn[2] = {};
+        int k[2] = {0, 0};
+#pragma unroll 4
+        for (int i = 1; i <= half; ++i) {
+            const float2 a = x[i * jump], b = x[(r - i) * jump];
+#pragma unroll
+            for (int o = 0; o < 2; ++o) {
+                k[o] += 2 * p + o;
+                k[o] -= k[o] >= r ? r : 0;
+                const float2 t = root[k[o] * jump];  // (cos, -sin)
+                cs[o] = make_float2(fmaf(t.x, a.x + b.x, cs[o].x), fmaf(t.x, a.y + b.y, cs[o].y));
+                sn[o] = make_float2(fmaf(t.y, a.x - b.x, sn[o].x), fmaf(t.y, a.y - b.y, sn[o].y));
+            }
+        }
+        float2 *y = out + c * N + g * r;
+#pragma unroll
+        for (int o = 0; o < 2; ++o) {
+            const int q = 2 * p + o;
+            if (q > half) break;
+            const float2 d = INV ? make_float2(sn[o].y, -sn[o].x) : make_float2(-sn[o].y, sn[o].x);
+            y[q] = cadd(cs[o], d);
+            if (q) y[r - q] = csub(cs[o], d);
+        }
+    }
+}
+
 // A later stage with an odd radix: point o = (j / ns) r ns + j % ns + q ns is the sum over
 // i < r of in[j + i N/r] e^{-2 pi i (o mod r ns) i / (r ns)}, one point per item.
 template <bool INV, int R>
@@ -697,7 +738,13 @@ __device__ __forceinline__ float2 *mixed_fft(float2 *a, float2 *b, const float2 
     case 3: mixed_first<INV, 3>(a, b, root, N, C, 3); break;
     case 5: mixed_first<INV, 5>(a, b, root, N, C, 5); break;
     case 7: mixed_first<INV, 7>(a, b, root, N, C, 7); break;
-    default: mixed_first<INV, 0>(a, b, root, N, C, p.st[0].r); break;
+    default: {
+        const int r = p.st[0].r, jump = N / r;
+        // two outputs per item where that leaves every thread one
+        if (C * jump * ((r + 3) / 4) >= (int)blockDim.x) mixed_first_two<INV>(a, b, root, N, C, r);
+        else mixed_first<INV, 0>(a, b, root, N, C, r);
+        break;
+    }
     }
     for (int s = 1; s < p.stages; ++s) {
         float2 *t = a;

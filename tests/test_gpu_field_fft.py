@@ -122,3 +122,10 @@ def test_rows_make_the_maps(mx, my):
             assert g["tau"] == pytest.approx(tau, rel=mx * my * 2.0 ** -52)
         again = pl.computeOverlaps()
     assert np.array_equal(again[0], field) and np.array_equal(again[1], mov) and again[3] == tau
+
+
+# long odd radices, two outputs per item: just enough items for a block's threads, not
+# enough in a single FFT but in two, an odd and an even number of outputs
+@pytest.mark.parametrize("mx,my", [(2032, 32), (1808, 48), (16, 3856), (4016, 16)])
+def test_long_odd_radix_matches_oracle(oracle, mx, my):
+    test_mixed_field_matches_oracle(oracle, mx, my)
