@@ -27,14 +27,16 @@ __global__ __launch_bounds__(kStageBlock) void k_unpack(const float2 *__restrict
     }
 }
 
-// n floats, whole float4s while they last (both ends 16-byte aligned).
-__global__ __launch_bounds__(kStageBlock) void k_download(const float *__restrict__ src, int64_t n,
-                                                          float *__restrict__ out)
+// n floats, whole float4s while they last where both ends are 16-byte aligned; one end is
+// a slot.
+__global__ __launch_bounds__(kStageBlock) void k_move(const float *__restrict__ src, int64_t n,
+                                                      float *__restrict__ out)
 {
     const int64_t t = (int64_t)blockIdx.x * kStageBlock + threadIdx.x, step = (int64_t)gridDim.x * kStageBlock;
-    for (int64_t i = t; i < n / 4; i += step)
+    const int64_t v = (reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(out)) % 16 ? 0 : n / 4;
+    for (int64_t i = t; i < v; i += step)
         reinterpret_cast<float4 *>(out)[i] = reinterpret_cast<const float4 *>(src)[i];
-    for (int64_t i = n / 4 * 4 + t; i < n; i += step) out[i] = src[i];
+    for (int64_t i = v * 4 + t; i < n; i += step) out[i] = src[i];
 }
 
 __global__ __launch_bounds__(kStageBlock) void k_place_cells(const float *__restrict__ x, const float *__restrict__ y,
@@ -52,6 +54,12 @@ __global__ __launch_bounds__(kStageBlock) void k_place_cells(const float *__rest
     const float2 p = make_float2(fminf(fmaxf(px, die.x), die.z - s.x), fminf(fmaxf(py, die.y), die.w - s.y));
     pos[k] = p;
     u[k] = p;
+}
+
+void launch_move(const float *src, int64_t n, float *out, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_move, dim3((unsigned)((n / 4 + kStageBlock) / kStageBlock)), dim3(kStageBlock), 0, s, src, n,
+                       out);
 }
 
 ep_status hip_ok(hipError_t e, const char *what)
@@ -108,6 +116,8 @@ ep_status StageOut::take() { return drain(next_); }
 ep_status StageOut::queued()
 {
     ep_status s = hip_ok(hipGetLastError(), "download");
+    // the end of a launch itself (hipExtLaunchKernel) as the event saves 2.5 us of a call,
+    // but then the next work on another stream takes 100 us more
     if (s == EP_OK) s = hip_ok(hipEventRecord(st_.done[next_], st_.stream), "download");
     if (s != EP_OK) return s;
     piece_[next_].busy = true;
@@ -136,8 +146,10 @@ ep_status StageOut::pairs(const float2 *src, const int32_t *stored, int64_t n_st
     return EP_OK;
 }
 
-ep_status StageOut::flat(const float *src, int64_t n, float *out)
+ep_status StageOut::flat(const void *from, int64_t n, void *to)
 {
+    const float *src = static_cast<const float *>(from);
+    float *out = static_cast<float *>(to);
     if (!out) return EP_OK;
     const int64_t per = (int64_t)(st_.bytes / sizeof(float));
     for (int64_t o = 0; o < n; o += per) {
@@ -149,8 +161,7 @@ ep_status StageOut::flat(const float *src, int64_t n, float *out)
             // a kernel starts sooner than the copy engine (three maps of 128^2, 224^2, 480^2:
             // 92 / 104 / 186 us a call, 103 / 120 / 199 with copies), but chunks that follow
             // each other are slower with it (three of 1024^2: 826, 764 with copies)
-            const unsigned blocks = (unsigned)((m / 4 + kStageBlock) / kStageBlock);
-            hipLaunchKernelGGL(k_download, dim3(blocks), dim3(kStageBlock), 0, st_.stream, src, m, pin);
+            launch_move(src, m, pin, st_.stream);
         } else {
             s = hip_ok(hipMemcpyAsync(pin, src + o, (size_t)m * sizeof(float), hipMemcpyDeviceToHost, st_.stream),
                        "download");
@@ -174,15 +185,20 @@ ep_status StageOut::finish()
 ep_status stage_in(Stage &st, float *dst, const float *src, int64_t n)
 {
     const int64_t per = (int64_t)(st.bytes / sizeof(float));
-    int k = 0;
-    for (int64_t o = 0; o < n; o += per, k ^= 1) {
+    for (int64_t o = 0; o < n; o += per, st.up ^= 1) {
         const int64_t m = std::min(per, n - o);
+        const int k = st.up;
         // the slot's last use, in this call or an earlier one
         ep_status s = hip_ok(hipEventSynchronize(st.done[k]), "upload");
         if (s != EP_OK) return s;
         std::memcpy(st.pin[k], src + o, (size_t)m * sizeof(float));
-        s = hip_ok(hipMemcpyAsync(dst + o, st.pin[k], (size_t)m * sizeof(float), hipMemcpyHostToDevice, st.stream),
-                   "upload");
+        if (n <= per) {
+            launch_move(reinterpret_cast<const float *>(st.pin[k]), m, dst, st.stream);
+            s = hip_ok(hipGetLastError(), "upload");
+        } else {
+            s = hip_ok(hipMemcpyAsync(dst + o, st.pin[k], (size_t)m * sizeof(float), hipMemcpyHostToDevice, st.stream),
+                       "upload");
+        }
         if (s == EP_OK) s = hip_ok(hipEventRecord(st.done[k], st.stream), "upload");
         if (s != EP_OK) return s;
     }
