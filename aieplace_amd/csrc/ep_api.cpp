@@ -717,8 +717,8 @@ extern "C" ep_status ep_create(const ep_netlist *nl, const ep_params *p, ep_ctx 
         destroy_ctx(c);
         return fail(EP_EDEVICE, "ep_create: hipMemset failed");
     }
-    // a slot holds the cells' coordinates or the field, whichever is larger, or a chunk of it
-    EP_TRY(stage_init(c->stage, c->stream, sizeof(float2) * std::max<size_t>(nb, c->n_place)));
+    // a slot holds the cells' bin ranges or the field, whichever is larger, or a chunk of it
+    EP_TRY(stage_init(c->stage, c->stream, std::max(sizeof(float2) * nb, sizeof(int4) * (size_t)c->n_place)));
     if (!L.cell_order.empty()) {
         std::vector<int32_t> stored(L.cell_order.size());
         for (size_t k = 0; k < stored.size(); ++k) stored[L.cell_order[k]] = (int32_t)k;
@@ -967,21 +967,15 @@ extern "C" ep_status ep_gradient(ep_ctx *c, float gamma, float lambda, float *gx
 extern "C" ep_status ep_cell_bins(ep_ctx *c, int32_t stretched, int32_t *out)
 {
     if (!c || !out) return fail(EP_EINVAL, "ep_cell_bins: null argument");
-    int32_t *d = nullptr;
-    ep_status st = dalloc(&d, 4 * (size_t)std::max(1, c->n_place));
-    if (st != EP_OK) return st;
+    // the packed cells' buffer is free between evaluations
+    int4 *d = reinterpret_cast<int4 *>(c->sorted);
     launch_cell_bins(*c, c->V[c->cur], stretched ? 1 : 0, d, c->stream);
-    st = check_launch();
-    if (st == EP_OK) st = sync(*c);
-    if (st == EP_OK) {
-        std::vector<int32_t> h(4 * (size_t)std::max(1, c->n_place));
-        hipError_t e = hipMemcpy(h.data(), d, sizeof(int32_t) * 4 * (size_t)c->n_place, hipMemcpyDeviceToHost);
-        if (e != hipSuccess) st = fail(EP_EDEVICE, "ep_cell_bins: copy failed");
-        for (int k = 0; st == EP_OK && k < c->n_place; ++k)
-            std::memcpy(out + 4 * (size_t)caller_cell(c->cell_order, k), &h[4 * (size_t)k], 4 * sizeof(int32_t));
-    }
-    (void)hipFree(d);
-    return st;
+    ep_status st = check_launch();
+    if (st != EP_OK) return st;
+    StageOut copy(c->stage);
+    st = copy.flat(d, 4 * (int64_t)c->n_place, out);
+    const ep_status fin = copy.finish();
+    return st != EP_OK ? st : fin;
 }
 
 extern "C" ep_status ep_hpwl(ep_ctx *c, double *hpwl)

@@ -307,7 +307,7 @@ void launch_wa_packet_fast64(const float *data, int net_size, int n_nets, int gr
 // Device address of the current GPU's fixed packet staging (2 x
 // EP_WA_PACKET_NOALLOC_MAX floats: data, then partials), looked up once per device.
 ep_status wa_packet_stage(float **stage);
-void launch_cell_bins(Ctx &c, const float2 *pos, int stretched, int32_t *out, hipStream_t s);
+void launch_cell_bins(Ctx &c, const float2 *pos, int stretched, int4 *out, hipStream_t s);
 ep_status field_init(Ctx &c);   // builds transform matrices
 // FP64 device solve of the current map; max-norm relative error of ex/ey against it.
 ep_status field_error(Ctx &c, double *err_ex, double *err_ey);

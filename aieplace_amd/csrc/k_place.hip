@@ -789,20 +789,20 @@ __global__ __launch_bounds__(kBlock) void k_probe(const float2 *__restrict__ v,
     }
 }
 
+// Bin ranges (i0, i1, j0, j1) in the caller's order: cell o is stored[o] for o < n_mov,
+// else o (stored may be null).
 __global__ void k_cell_bins(const float2 *__restrict__ pos, const float2 *__restrict__ wh,
-                            int n_place, GeomArgs g, int Mx, int My, int stretched,
-                            int32_t *__restrict__ out)
+                            const int32_t *__restrict__ stored, int n_mov, int n_place, GeomArgs g, int Mx, int My,
+                            int stretched, int4 *__restrict__ out)
 {
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n_place; c += gridDim.x * blockDim.x) {
+    for (int o = blockIdx.x * blockDim.x + threadIdx.x; o < n_place; o += gridDim.x * blockDim.x) {
+        const int c = stored && o < n_mov ? stored[o] : o;
         Rect r;
         if (stretched)
             stretched_rect(pos[c], wh[c], g, Mx, My, r);
         else
             exact_rect(pos[c], wh[c], g, Mx, My, r);
-        out[4 * c + 0] = r.i0;
-        out[4 * c + 1] = r.i1;
-        out[4 * c + 2] = r.j0;
-        out[4 * c + 3] = r.j1;
+        out[o] = make_int4(r.i0, r.i1, r.j0, r.j1);
     }
 }
 
@@ -1250,10 +1250,10 @@ ep_status wa_packet_stage(float **stage)
     return EP_OK;
 }
 
-void launch_cell_bins(Ctx &c, const float2 *pos, int stretched, int32_t *out, hipStream_t s)
+void launch_cell_bins(Ctx &c, const float2 *pos, int stretched, int4 *out, hipStream_t s)
 {
     hipLaunchKernelGGL(k_cell_bins, dim3(grid_for(c.n_place, kBlock, 8192)), dim3(kBlock), 0, s,
-                       pos, c.wh, c.n_place, geom_args(c), c.Mx, c.My, stretched, out);
+                       pos, c.wh, c.d_stored, c.n_mov, c.n_place, geom_args(c), c.Mx, c.My, stretched, out);
 }
 
 }  // namespace ep

@@ -79,3 +79,24 @@ def test_batch_positions_after_reset(order):
         for k in range(2):
             assert np.array_equal(s[k], want[k]) and np.array_equal(a[k], want[k])
             assert not np.array_equal(m[k], want[k])
+
+
+# one chunk and two, a length that is no multiple of four cells
+@pytest.mark.parametrize("n", [1_001, 65_537])
+@pytest.mark.parametrize("stretched", [0, 1])
+def test_cell_bins_keep_the_callers_order(n, stretched):
+    print(f"case cell bins n={n} stretched={stretched}", flush=True)
+    nl = A.generate("stdcell", seed=3, n_movable=n, shuffle_storage=1)
+    rng = np.random.default_rng(n)
+    xl, yl, xh, yh = nl.die
+    x, y = xl + rng.random(n) * (xh - xl), yl + rng.random(n) * (yh - yl)
+    out = []
+    for order in (0, 1):
+        p = A.placer_params(A.CONFIGS["stdcell_200k"], bins_x=64, bins_y=64, use_fillers=0, cell_order=order)
+        with A.Placer(nl, p) as pl:
+            pl.set_positions(x, y)
+            out.append(pl.cell_bins(stretched))
+    assert np.array_equal(out[0], out[1])
+    bw = (xh - xl) / 64  # a cell's first bin holds its corner, or lies left of it by the stretch
+    first = np.floor((np.minimum(x, xh - nl.w[:n]) - xl) / bw)
+    assert np.abs(out[0][:, 0] - first).max() <= 1
