@@ -925,8 +925,6 @@ extern "C" ep_status ep_wa_grad(ep_ctx *c, float gamma, double *wa, double *hpwl
 extern "C" ep_status ep_get_wa_grad(ep_ctx *c, float *gx, float *gy)
 {
     if (!c) return fail(EP_EINVAL, "ep_get_wa_grad: null context");
-    c->h_scal->lambda = 0.0f;
-    push_scalars(*c, c->stream);
     launch_pin_sum(*c, c->stream);
     ep_status st = check_launch();
     if (st != EP_OK) return st;
