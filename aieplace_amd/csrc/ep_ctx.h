@@ -260,12 +260,13 @@ void launch_overflow(Ctx &c, hipStream_t s);
 // field_max[0] (the operand scale of the first product).
 void launch_map_range(Ctx &c, hipStream_t s);
 void launch_field(Ctx &c, int precision, hipStream_t s);
-// launch_overflow, then launch_field.  Below kForkMinCells placeable cells the FFTs' rows
-// kernel does the overflow pass as it reads the map: us per evaluation 20k cells 48.5 ->
-// 47.4, 75k 57.4 -> 56.0, 100k on a 400^2 grid 69.7 -> 66.4, 200k 76.1 -> 74.8, 500k 132.7
-// -> 131.1.  Beside the gathers of a large instance's other branch its few waves lose: 2M
-// 269.6 -> 276.  The line is that of the default fork, not this context's: the order of
-// the overflow sum then does not depend on fork_min_cells.
+// launch_overflow, then launch_field.  Below kForkMinCells placeable cells, and with rows
+// of up to kFftMapsMax bins, the FFTs' rows kernel does the overflow pass as it reads the
+// map: us per evaluation 20k cells 48.5 -> 47.4, 75k 57.4 -> 56.0, 100k on a 400^2 grid
+// 69.7 -> 66.4, 200k 76.1 -> 74.8, 500k 132.7 -> 131.1.  Beside the gathers of a large
+// instance's other branch its few waves lose: 2M 269.6 -> 276.  The line is that of the
+// default fork, not this context's: the order of the overflow sum then does not depend
+// on fork_min_cells.
 void launch_overflow_field(Ctx &c, int precision, hipStream_t s);
 // Reads the cells' pin-partial sums (gw_cell).
 void launch_cell_grad(Ctx &c, Pair<const float2> pos, Pair<const float2> vref,

@@ -52,13 +52,21 @@ constexpr int kFftPow2Max = 8192, kFftMixedMax = 4080;
 inline bool fft_pow2(int n) { return (n & (n - 1)) == 0; }
 inline bool fft_side(int n) { return n >= 16 && n % 16 == 0 && n <= (fft_pow2(n) ? kFftPow2Max : kFftMixedMax); }
 
+// Rows of 8192 points leave the overflow pass to its own kernel: their blocks of 1024
+// threads hold 128 registers a thread and spill 31 beside the bins.  us per evaluation, in
+// the rows / by itself: 16 x 8192 134 / 124 (100k cells), 64 x 8192 157 / 147, 1024 x 8192 4480 /
+// 4400; 16 x 4096 105.7 / 104.7, 64 x 4096 106 / 106, 256 x 4096 141 / 143 (400k), 16 x 2048
+// 89.5 / 89.6, 16 x 1008 78.5 / 81.8.
+constexpr int kFftMapsMax = 4096;
+
 // Constants of length-n transforms, made in FP64.
 void fft_table(int n, std::vector<float2> &tab);
 // Stages of a length that is no power of two (none for one that is).
 FftPlan fft_plan(int n);
 // Blocks of the rows kernel.
 int fft_row_blocks(int Mx, int My);
-// `maps`: the overflow pass goes with the rows (null: the map is there).
+// `maps`: the overflow pass goes with the rows (null: the map is there), which are no
+// longer than kFftMapsMax.
 void launch_field_fft(const FftArgs &a, const FftMaps *maps, hipStream_t s);
 
 // Batched solves: one launch per stage (rows, columns, field) and class covers

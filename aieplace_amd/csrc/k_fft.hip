@@ -1081,7 +1081,8 @@ void launch_field_fft(const FftArgs &a, const FftMaps *maps, hipStream_t s)
             hipLaunchKernelGGL(kern, dim3(fft_row_blocks(a.Mx, a.My)), dim3(F * Plan<L>::T),
                                F * Plan<L>::buf * sizeof(float2), s, a, mp);
         };
-        if (maps) go(k_fft_rows<L, true>, *maps);
+        constexpr bool can = Plan<L>::N <= kFftMapsMax;
+        if (can && maps) go(k_fft_rows<L, can>, *maps);
         else go(k_fft_rows<L, false>, FftMaps{});
     });
     if (!fft_pow2(a.Mx)) launch_mixed<1>(a, nullptr, s);

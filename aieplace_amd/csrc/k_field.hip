@@ -913,7 +913,7 @@ static void launch_solve(Ctx &c, int precision, bool maps, hipStream_t s)
 void launch_field(Ctx &c, int precision, hipStream_t s) { launch_solve(c, precision, false, s); }
 void launch_overflow_field(Ctx &c, int precision, hipStream_t s)
 {
-    const bool joint = c.n_place < kForkMinCells;
+    const bool joint = c.n_place < kForkMinCells && c.My <= kFftMapsMax;
     if (!joint) launch_overflow(c, s);
     launch_solve(c, precision, joint, s);
 }

@@ -129,3 +129,9 @@ def test_rows_make_the_maps(mx, my):
 @pytest.mark.parametrize("mx,my", [(2032, 32), (1808, 48), (16, 3856), (4016, 16)])
 def test_long_odd_radix_matches_oracle(oracle, mx, my):
     test_mixed_field_matches_oracle(oracle, mx, my)
+
+
+# the longest row that makes the maps, and the ones past it on a short and a long grid
+@pytest.mark.parametrize("mx,my", [(16, 4096), (16, 8192), (64, 8192)])
+def test_maps_of_long_rows(mx, my):
+    test_rows_make_the_maps(mx, my)
