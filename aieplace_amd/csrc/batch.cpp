@@ -17,6 +17,7 @@
 
 #include "../../include/eplace_batch.h"
 #include "ep_batch.h"
+#include "ep_fft.h"
 #include "ep_layout.h"
 #include "ep_stage.h"
 
@@ -65,7 +66,8 @@ struct ep_batch {
     hipStream_t side = nullptr;              // second captured branch (WA beside the maps and field)
     hipEvent_t fork = nullptr, join = nullptr;
     ep_params prm{};
-    bool f16() const { return prm.precision == EP_PREC_FP16X3; }  // products scale by the map range
+    bool products = false;  // an instance's grid is none that the FFTs take
+    bool map_range() const { return products && prm.precision == EP_PREC_FP16X3; }  // split-FP16 products scale by it
     int n = 0;
     std::vector<BInst> inst;
     std::vector<int32_t> n_fix;
@@ -180,7 +182,7 @@ struct ep_batch {
         bl_sort_count(d, kAtCur, sort_blocks, stream);
         bl_sort(d, kAtCur, sort_blocks, kDensCpt[v], stream);
         bl_density(d, dens_blocks[v], kDensCpt[v], stream);
-        bl_overflow(d, bin_blocks, f16(), stream);
+        bl_overflow(d, bin_blocks, map_range(), stream);
     }
 
     // One gradient evaluation as a captured fork: the tile sort, the density
@@ -194,7 +196,7 @@ struct ep_batch {
         if (e != hipSuccess) return e;
         bl_sort(d, at, sort_blocks, kDensCpt[v], side);
         bl_density(d, dens_blocks[v], kDensCpt[v], side);
-        bl_overflow(d, bin_blocks, f16(), side);
+        bl_overflow(d, bin_blocks, map_range(), side);
         launch_field_batch(bf, prm.precision, side);
         if ((e = hipEventRecord(join, side)) != hipSuccess) return e;
         bl_wa(d, at, wa_blocks, s);
@@ -213,7 +215,7 @@ struct ep_batch {
         if (!counted) bl_sort_count(d, at, sort_blocks, s);
         bl_sort_wa(d, at, sort_blocks, kDensCpt[v], wa_blocks, s);
         bl_density_pins(d, dens_blocks[v], kDensCpt[v], cell_blocks, s);
-        bl_overflow(d, bin_blocks, f16(), s);
+        bl_overflow(d, bin_blocks, map_range(), s);
         launch_field_batch(bf, prm.precision, s);
         bl_cell_grad(d, at, true, cell_blocks, s);
         bl_reduce_control(d, ctl_mode, s);
@@ -617,6 +619,7 @@ extern "C" ep_status ep_batch_create(const ep_netlist *const *nls, const int32_t
         fi[i].map_mean = b->map_mean + i;
         fi[i].skip = &b->d_st[i].done;
     }
+    for (const BatchFieldInst &f : fi) b->products = b->products || !fft_side(f.M);
     EPB_TRY(batch_field_init(b->bf, fi));
     EPB_TRY(reset_state(b));
     EPB_TRY(autotune(b));
