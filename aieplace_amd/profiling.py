@@ -7,10 +7,11 @@
       FETCH_SIZE and WRITE_SIZE per dispatch (two --pmc passes) for the
       placement kernels, scaled by the same counters read on a device copy of
       known size -> profiles/traffic_<workload>_<prec>.md
-  python -m aieplace_amd.profiling mfma    [--workload stdcell_2m] [--precision 0]
+  python -m aieplace_amd.profiling mfma    [--workload stdcell_2m] [--precision 0] [--bins 4112]
       matrix-core utilisation of the transform products (one --pmc pass of SQ
       counters): SQ_VALU_MFMA_BUSY_CYCLES / (4 SIMDs x SQ_BUSY_CU_CYCLES) per
-      kernel, with the products' achieved TFLOP/s -> profiles/mfma_<workload>_<prec>.md
+      kernel, with the products' achieved TFLOP/s, on a grid that the products
+      solve (the FFTs take sides up to 4080) -> profiles/mfma_<workload>_<bins>_<prec>.md
   python -m aieplace_amd.profiling timeline [--workload stdcell_2m] [--precision 0]
       kernel trace of one placement split at each Nesterov trial: trial wall
       time, kernels' busy time (so the idle gaps between them) and each
@@ -21,8 +22,9 @@
   python -m aieplace_amd.profiling drive ...
       the profiled program itself (run under rocprofv3 by the two commands
       above): a full placement, then `reps` ep_profile repetitions of each
-      kernel at the final placement; with --copy-mib N it instead copies an
-      N MiB device buffer `reps` times (the calibration kernel).
+      kernel at the final placement; --bins N takes an N x N grid for the
+      workload's own, --iters N stops after N iterations; with --copy-mib N it
+      instead copies an N MiB device buffer `reps` times (the calibration kernel).
 
 The parent process never touches the GPU; rocprofv3 runs the driver as a child.
 """
@@ -86,6 +88,10 @@ def drive(args) -> None:
     cfg = A.CONFIGS[args.workload]
     nl = A.generate(seed=1, **cfg["gen"])
     p = A.placer_params(cfg, precision=args.precision, use_graph=1)
+    if args.bins:
+        p.bins_x = p.bins_y = args.bins
+    if args.iters:
+        p.max_iters = args.iters
     with A.Placer(nl, p) as pl:
         r = pl.run()
         prof = pl.profile(args.reps) if args.reps > 0 else []
@@ -113,6 +119,9 @@ def drive_batch(args) -> None:
 def _drive_cmd(args, extra=()):
     cmd = [sys.executable, "-u", "-m", "aieplace_amd.profiling", "drive", "--workload", args.workload,
            "--precision", str(args.precision), "--reps", str(args.reps)]
+    for name in ("bins", "iters"):
+        if getattr(args, name):
+            cmd += [f"--{name}", str(getattr(args, name))]
     return cmd + list(extra)
 
 
@@ -304,6 +313,13 @@ def _per_kernel(disp, last_n):
     return {k: sum(v[-last_n:]) / len(v[-last_n:]) for k, v in by.items()}
 
 
+def _item_dispatches(q, precision):
+    """Dispatches of one call of ep_profile item q that _family counts to it: the
+    split-FP16 products also clear their operands' maxima."""
+    products = q["name"] == "field_transforms" and q["flops"] > 0
+    return int(q["launches"]) + (1 if products and precision == 2 else 0)
+
+
 def _per_call(disp, fam, n_disp, reps):
     """KiB of one call of item `fam`: the last reps * n_disp dispatches of its
     kernels (the ep_profile repetitions at the end of the driver) / reps."""
@@ -366,7 +382,7 @@ def traffic(args) -> str:
                      f"{fetch.get(k, 0.0) * 1024 * f_fetch / 1e6:.3f} |")
     summary = {}
     for fam, q in prof.items():
-        n_disp = int(q["launches"])
+        n_disp = _item_dispatches(q, args.precision)
         fb = _per_call(disp["FETCH_SIZE"], fam, n_disp, args.reps) * 1024 * f_fetch
         wb = _per_call(disp["WRITE_SIZE"], fam, n_disp, args.reps) * 1024 * f_write
         if fb + wb > 0:
@@ -394,12 +410,18 @@ def traffic(args) -> str:
 MFMA_COUNTERS = ["SQ_VALU_MFMA_BUSY_CYCLES", "SQ_BUSY_CU_CYCLES", "SQ_INSTS_MFMA", "SQ_INSTS_VALU",
                  "SQ_WAVES", "SQ_WAVE_CYCLES", "SQ_WAIT_INST_ANY", "SQ_ACTIVE_INST_VALU"]
 PEAK_TFLOPS = {0: 157.3, 1: 2500.0, 2: 2500.0}  # dense MFMA: FP32, BF16, FP16
+PRODUCT_BINS = 4112  # the smallest side that the FFTs do not take
 
 
 def mfma(args) -> str:
+    args.bins = args.bins or PRODUCT_BINS
+    args.iters = args.iters or 8
     prec = PREC_NAME[args.precision]
     od = os.path.join(args.scratch, f"pmc_mfma_{args.workload}_{args.precision}")
-    full, _ = _rocprof(["--pmc"] + MFMA_COUNTERS, _drive_cmd(args), od, args.timeout)
+    full, res = _rocprof(["--pmc"] + MFMA_COUNTERS, _drive_cmd(args), od, args.timeout)
+    if res and any(q["name"] == "field_transforms" and q["flops"] == 0 for q in res["profile"]):
+        raise SystemExit(f"mfma: FFTs solve the field on {args.bins} x {args.bins} bins, without matrix products; "
+                         f"take a grid that they refuse (--bins {PRODUCT_BINS})")
     rows = _csv(od, "counter_collection.csv")
     per = {c: _per_kernel(_dispatches(rows, c), args.reps) for c in MFMA_COUNTERS}
     # timings from the same driver run without the profiler (counter collection
@@ -412,15 +434,15 @@ def mfma(args) -> str:
     if plain.returncode != 0 or drv is None:
         raise RuntimeError(f"driver run failed ({plain.returncode}):\n{plain.stderr[-2000:]}")
     prof = {q["name"]: q for q in drv["profile"]}
-    lines = [f"# Matrix-core utilisation: {args.workload}, {prec} transforms", "",
-             "One rocprofv3 --pmc pass of SQ counters over the driver (a full placement, then "
+    lines = [f"# Matrix-core utilisation: {args.workload} on {args.bins} x {args.bins} bins, {prec} transforms", "",
+             f"One rocprofv3 --pmc pass of SQ counters over the driver ({args.iters} iterations, then "
              f"{args.reps} ep_profile repetitions of each item; per-dispatch values are the mean of each "
              "kernel's last dispatches).  MFMA busy = SQ_VALU_MFMA_BUSY_CYCLES / (4 SIMDs x "
              "SQ_BUSY_CU_CYCLES): the share of SIMD cycles, while the CUs are busy, in which the matrix core "
              "works.  VALU active and waiting are per wave: SQ_ACTIVE_INST_VALU (quad-cycles, 4 cycles "
              "each) and SQ_WAIT_INST_ANY over SQ_WAVE_CYCLES.", "",
              f"Written by `python -m aieplace_amd.profiling mfma --workload {args.workload} --precision "
-             f"{args.precision}`, which runs (from the repository root):", "", "```",
+             f"{args.precision} --bins {args.bins}`, which runs (from the repository root):", "", "```",
              _cmd_text(full), "```", "",
              "| kernel | waves | MFMA instr / wave | MFMA busy | VALU instr / wave | VALU active | waiting |",
              "|---|---:|---:|---:|---:|---:|---:|"]
@@ -453,7 +475,7 @@ def mfma(args) -> str:
                       "half of these flops in FP32; the split forms execute three products each, 1.5x "
                       "of them at the 16-bit rate.", ""]
         lines.append(f"mfma field_transforms busy {busy_m / (4 * busy_c):.4f} tflops {tf:.2f}")
-    path = os.path.join(PROFILES, f"mfma_{args.workload}_{prec}.md")
+    path = os.path.join(PROFILES, f"mfma_{args.workload}_{args.bins}_{prec}.md")
     with open(path, "w") as f:
         f.write("\n".join(lines) + "\n")
     return path
@@ -477,6 +499,8 @@ def main(argv=None) -> int:
     ap.add_argument("--workload", default="stdcell_2m")
     ap.add_argument("--precision", type=int, default=0)
     ap.add_argument("--reps", type=int, default=5)
+    ap.add_argument("--bins", type=int, default=0, help="side of the grid (default: the workload's; mfma: 4112)")
+    ap.add_argument("--iters", type=int, default=0, help="iterations of the placement (default: all; mfma: 8)")
     ap.add_argument("--instances", type=int, default=64, help="batch: instances of the batched workload")
     ap.add_argument("--copy-mib", type=int, default=0, help="drive: copy calibration instead of placement")
     ap.add_argument("--calib-mib", type=int, default=256, help="traffic: size of the calibration copy")
