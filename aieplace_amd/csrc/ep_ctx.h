@@ -91,7 +91,10 @@ constexpr int kModelBackoffMax = 32;
 // branch of single kernels): 383k placeable cells 90.7 / 84.6 (93.4), 643k 134.3 / 133.5
 // (145), 1.28M 173 / 179 (193), 2.56M 271 / 295 (302).  A batch's running instances
 // count together; 100 iterations in ms: 16 instances (358k movable cells) 12.0 / 11.5
-// (12.3), 24 (513k) 13.9 / 13.9 (15.0), 32 (1.6M) 28.7 / 31.9 (32.7).
+// (12.3), 24 (513k) 13.9 / 13.9 (15.0), 32 (1.6M) 28.7 / 31.9 (32.7).  The pin sums'
+// blocks hold the scatter's window of LDS, too: 22 KB there, but 102 KB with a movable
+// cell of 60 bins, one block per CU; single kernels / shared launches then, at 20k, 100k,
+// 200k and 400k cells on 512^2 bins, 112 / 109, 127 / 126, 140 / 142 and 167 / 169 us.
 constexpr int64_t kForkMinCells = 800000;
 inline int64_t fork_min_cells(const ep_params &p)
 {

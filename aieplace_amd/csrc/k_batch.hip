@@ -58,8 +58,8 @@ __device__ inline const float2 *eval_pos(const BDev &d, int cur, int at)
 // ------------------------------------------------------------------ moves
 
 // kMoveTrial: u' = clamp(v - alpha g), v' = clamp(u' + coef (u' - u)) into the
-// other parity, counting v' into the instance's sort tiles (the evaluation's
-// sort then skips its counting pass); kMoveProbe: v_-1 = clamp(v - eps g);
+// other parity, counting v' into the instance's sort tiles, as kb_sort_count
+// does; kMoveProbe: v_-1 = clamp(v - eps g);
 // kMoveInitU: u = v.  Blocks take kBlock * CPT cells (pre_sort).
 template <int CPT>
 __global__ __launch_bounds__(kBlock) void kb_move(BDev d, int mode)

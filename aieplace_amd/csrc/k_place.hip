@@ -721,8 +721,7 @@ __global__ __launch_bounds__(finalize_threads(kBlocks)) void k_finalize(Finalize
 
 // u' = clamp(v - alpha g); v' = clamp(u' + coef (u' - u))   (ePlace Nesterov step)
 // With `count`, the new positions are also counted into the sort's coarse
-// tiles (the first pass of launch_sort, which then skips it).  Blocks take
-// kBlock * CPT cells, as k_sort_count.
+// tiles, as k_sort_count does.  Blocks take kBlock * CPT cells, as there.
 template <int CPT>
 __global__ __launch_bounds__(kBlock) void k_trial(Pair<const float2> v_pair,
                                                   Pair<const float2> u_pair,
@@ -751,8 +750,9 @@ __global__ __launch_bounds__(kBlock) void k_trial(Pair<const float2> v_pair,
     const int base = blockIdx.x * kBlock * CPT;
     double dv2[1] = {0.0};  // |v' - v|^2, for the step-length estimate
     // One cell per pass: every wave of the grid walks the same slice k at
-    // about the same time.  Loading all of a thread's 16 cells first measured
-    // slower at 2M cells (22.4 -> 25.7 us; groups of four cells: 23.5 us).
+    // about the same time.  With 16 cells per thread (the most is kSortMost now),
+    // loading all of them first measured slower at 2M cells (22.4 -> 25.7 us; groups
+    // of four cells: 23.5 us).
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
         const int c = base + k * kBlock + threadIdx.x;

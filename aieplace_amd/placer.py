@@ -2,9 +2,9 @@
 
 Mirrors class Placer of vck5000/host/src/include/AIEplace.h:21-99 (method names
 kept): computeAllPartials -> WA gradient kernel, computeOverlaps -> density
-scatter, computeElectricFields -> MFMA transform field solve, nudgeAllNodes ->
-one Nesterov step with backtracking, performIteration/run/printIterationResults
-as in AIEplace.cpp:9-76, 1048-1070.  Errors raise EplaceError (the reference
+scatter, computeElectricFields -> field solve by FFTs (sides that these do not
+take: MFMA products), nudgeAllNodes -> one Nesterov step with backtracking,
+performIteration/run/printIterationResults as in AIEplace.cpp:9-76, 1048-1070.  Errors raise EplaceError (the reference
 logs and exits, AIEplace.cpp:95-98).
 """
 from __future__ import annotations
