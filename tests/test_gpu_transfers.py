@@ -100,3 +100,31 @@ def test_cell_bins_keep_the_callers_order(n, stretched):
     bw = (xh - xl) / 64  # a cell's first bin holds its corner, or lies left of it by the stretch
     first = np.floor((np.minimum(x, xh - nl.w[:n]) - xl) / bw)
     assert np.abs(out[0][:, 0] - first).max() <= 1
+
+
+@pytest.mark.parametrize("n", [1_001, 65_537])
+def test_reads_between_steps_change_nothing(n):
+    """Reads, single stages and refused positions between two steps use the buffers of the
+    other parity and of the sort; the steps after them are the same."""
+    print(f"case reads between steps n={n}", flush=True)
+    nl = A.generate("stdcell", seed=3, n_movable=n)
+    p = A.placer_params(A.CONFIGS["stdcell_200k"], bins_x=64, bins_y=64)
+    out = []
+    for read in (False, True):
+        with A.Placer(nl, p) as pl:
+            pl.initializePlacement()
+            log = []
+            for _ in range(4):
+                log.append(sorted(pl.nudgeAllNodes().items()))
+                if read:
+                    x, y = pl.get_positions()
+                    pl.cell_bins()
+                    pl.computeOverlaps()
+                    pl.computeAllPartials(3.0)
+                    pl.computeElectricFields()
+                    x[n // 3] = np.nan
+                    with pytest.raises(api.EplaceError):
+                        pl.set_positions(x, y)
+            out.append((log, *pl.get_positions()))
+    assert out[0][0] == out[1][0]
+    assert np.array_equal(out[0][1], out[1][1]) and np.array_equal(out[0][2], out[1][2])
